@@ -17,6 +17,7 @@
 #include "dsx_gemm_kernels.hpp"
 #include "dsx_misc_kernels.hpp"
 #include "dsx_q8_0_kernels.hpp"
+#include "dsx_stream_kernels.hpp"
 
 using namespace dsx;
 
@@ -75,6 +76,31 @@ int need_init(const char *who) {
     return DSX_OK;
 }
 
+// f(kernel, row tiles per stage) for the instance of k_mxfp4_stream that serves rows of n_sb super-blocks.
+template <bool PAIR, int NCG, typename F>
+int with_stream_kernel(uint32_t n_sb, F &&f) {
+    if constexpr (PAIR) {
+        if (n_sb <= 8u) return f(k_mxfp4_stream<PAIR, 2, NCG, 2>, 2u);
+    } else {
+        if (n_sb <= 4u) return f(k_mxfp4_stream<PAIR, 1, NCG, 4>, 4u);
+        if (n_sb <= 8u) return f(k_mxfp4_stream<PAIR, 2, NCG, 2>, 2u);
+    }
+    if (n_sb <= 16u) return f(k_mxfp4_stream<PAIR, 4, NCG, 1>, 1u);
+    return f(k_mxfp4_stream<PAIR, 7, NCG, 1>, 1u);
+}
+
+template <bool PAIR>
+void stream_raise_lds_limits() {
+    auto raise = [](auto kernel, uint32_t) {
+        (void)hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kStLds);
+        return 0;
+    };
+    for (uint32_t n_sb : {4u, 8u, 16u, kStMaxSb}) {
+        with_stream_kernel<PAIR, 1>(n_sb, raise);
+        with_stream_kernel<PAIR, 2>(n_sb, raise);
+    }
+}
+
 void raise_lds_limits() {
     {
         allow_lds(k_mxfp4_gate_up<1, false, false, false>);
@@ -118,6 +144,8 @@ void raise_lds_limits() {
         allow_lds(k_mxfp4_down_be4<4>);
         allow_lds(k_mxfp4_down_be4<8>);
         allow_lds(k_mxfp4_down_be4<16>);
+        stream_raise_lds_limits<true>();
+        stream_raise_lds_limits<false>();
         q8_0_raise_lds_limits();
         q8_0_gemm_raise_lds_limits();
     }
@@ -199,6 +227,21 @@ int launch_gemm(hipStream_t st, const GemmParams &p, uint32_t max_wi, bool plana
     hipLaunchKernelGGL((k_mxfp4_gemm<PAIR, MT>), dim3((uint32_t)grid), dim3(kGemmWaves * 64),
                        gemm_lds_bytes(MT, false), st, p);
     return launched(PAIR ? "gate_up gemm" : "down gemm");
+}
+
+// Streaming launch for groups of few members (items of up to 16 ncg members), one workgroup per CU.
+template <bool PAIR>
+int launch_stream(hipStream_t st, StreamParams p, uint32_t ncg) {
+    auto go = [&](auto kernel, uint32_t rt) -> int {
+        const uint64_t act_rows = (uint64_t)p.n_tokens * (p.n_used + 1u);
+        if (p.n_rows % (16u * rt) || p.n_sb > kStMaxSb || !stream_layout(p, PAIR, rt, ncg))
+            return fail(DSX_ERR_SHAPE, "stream: %u rows of %u super-blocks", p.n_rows, p.n_sb);
+        if (act_rows * p.act_row_bytes > 0xFFFFFFFFull)
+            return fail(DSX_ERR_INVALID_ARG, "stream: the activation rows exceed 4 GiB");
+        hipLaunchKernelGGL(kernel, dim3((uint32_t)g_num_cu), dim3(kStThreads), stream_lds_bytes(p, PAIR, rt, ncg), st, p);
+        return launched(PAIR ? "gate_up stream" : "down stream");
+    };
+    return ncg == 1u ? with_stream_kernel<PAIR, 1>(p.n_sb, go) : with_stream_kernel<PAIR, 2>(p.n_sb, go);
 }
 
 }  // namespace

@@ -502,7 +502,9 @@ __global__ __launch_bounds__(256) void k_sanitize_picks(int32_t *__restrict__ ou
     out[i] = (e < 0 || (uint32_t)e >= n_expert) ? -1 : e;
 }
 
-// Rows of f32 -> staged rows (the mid activations of the by-expert path).
+// Rows of f32 -> staged rows, FP6 planes or FP8 planes (the mid activations of the kernels for few
+// members per expert).
+template <bool FP6>
 __global__ __launch_bounds__(256) void k_quantize_staged(uint8_t *__restrict__ out,
                                                          const float *__restrict__ x,
                                                          uint32_t n_rows, uint32_t n_sb,
@@ -513,7 +515,8 @@ __global__ __launch_bounds__(256) void k_quantize_staged(uint8_t *__restrict__ o
     const uint32_t t = blk / n_sb, b = blk - t * n_sb;
     const float4 v = *(const float4 *)(x + (uint64_t)blk * 256u + lane * 4u);
     uint8_t *row = out + (uint64_t)t * row_bytes;
-    quantize_block_to_staged(v, lane, row + (size_t)b * 512u, (float *)(row + (size_t)n_sb * 512u) + b);
+    if (FP6) quantize_block_to_staged6(v, lane, row + (size_t)b * kStaged6Bytes, (float *)(row + (size_t)n_sb * kStaged6Bytes) + b);
+    else quantize_block_to_staged(v, lane, row + (size_t)b * 512u, (float *)(row + (size_t)n_sb * 512u) + b);
 }
 
 // ---------------------------------------------------------------------------------------

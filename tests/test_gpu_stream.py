@@ -1,0 +1,45 @@
+"""The streaming kernels for groups of few members (whole row tiles through LDS, columns in registers)
+against the CPU oracle: rows of an odd and an even number of super-blocks, each instance by row length
+(up to 4, 8, 16 and 28), groups around the 16- and 32-column items, empty slots, an expert that every
+token names (several items), no shared expert."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+from deepstrix_amd.executor import MoeLayer
+from oracle import ref
+from tests import helpers as H
+
+pytestmark = pytest.mark.gpu
+
+ROUTER = dict(router_mode=1, route_scale=2.5, bias_sigma=0.01, clamp=10.0)
+# (hidden, inter): gate/up rows of hidden / 256 super-blocks, down rows of inter / 256
+SHAPES = [(512, 256), (1280, 768), (2048, 1280), (3328, 2304), (4096, 2048), (4352, 1024), (7168, 512)]
+
+
+@pytest.mark.parametrize("hidden,inter", SHAPES)
+@pytest.mark.parametrize("T", [9, 33, 100])
+def test_stream_matches_the_oracle(monkeypatch, hidden, inter, T):
+    monkeypatch.setattr(MoeLayer, "v3_thresholds_below_experts", None)   # the library's own thresholds
+    s = H.Shape(hidden, inter, 8, 2, shared=hidden != 1280, seed=500 + T, **ROUTER)
+    x, _, _ = H.host_inputs(s, T)
+    rng = np.random.default_rng(T)
+    sel = np.stack([rng.permutation(8)[:2] for _ in range(T)]).astype(np.int32)
+    sel[:, 0] = np.where(sel[:, 1] == 3, sel[:, 0], 3)     # nearly every token names expert 3
+    sel[T // 2, 1] = -1                                    # an empty slot
+    w = rng.uniform(0.05, 0.6, sel.shape).astype(np.float32)
+    layer = MoeLayer(H.device_weights(s), T)
+    dx, ds, dwt = torch.from_numpy(x).cuda(), torch.from_numpy(sel).cuda(), torch.from_numpy(w).cuda()
+    out = layer.run(dx, None, selected_in=ds, weights_in=dwt).clone()
+    again = layer.run(dx, None, selected_in=ds, weights_in=dwt)
+    layer.set_tuning(gemm_min_tokens=1, gemm_narrow_members=1)   # the wide GEMM tile on the same inputs
+    gemm = layer.run(dx, None, selected_in=ds, weights_in=dwt).cpu().numpy()
+    torch.cuda.synchronize()
+    assert torch.equal(out, again)
+    out = out.cpu().numpy()
+    if inter % 512 == 0 and hidden % 512 == 0:
+        # other orders of the same f32 sums; a mid value may round to the neighbouring int8 step
+        # (1/127 of its block's largest value)
+        assert H.max_rel(out, gemm) < 1e-3
+    H.assert_close(out, ref.moe_forward(H.host_weights(s), x, sel, w), 2e-3, f"{hidden} x {inter} T={T}")
