@@ -198,10 +198,12 @@ static int fit_nt(uint32_t chunk, uint32_t n_blocks, int cap) {
 // optional extra group `n_expert` that holds every token (slot n_used).
 int group_build_big(hipStream_t st, int32_t *group_count, int32_t *group_offset, int32_t *members,
                     int32_t *work_items, int32_t *n_work_items, const int32_t *selected, uint32_t b,
-                    uint32_t n_used, uint32_t n_expert, uint32_t chunk, bool extra) {
-    hipLaunchKernelGGL(k_group_tables, dim3(n_expert + (extra ? 1u : 0u) + 1u), dim3(kGbThreads), 0, st,
+                    uint32_t n_used, uint32_t n_expert, uint32_t chunk, bool extra, int32_t *items2 = nullptr,
+                    int32_t *n_items2 = nullptr, uint32_t chunk2 = 0) {
+    // items2: a second list of work items, of chunk2 members
+    hipLaunchKernelGGL(k_group_tables, dim3(n_expert + (extra ? 1u : 0u) + (items2 ? 2u : 1u)), dim3(kGbThreads), 0, st,
                        group_count, group_offset, members, work_items, n_work_items, selected, b, n_used,
-                       n_expert, chunk, extra ? 1u : 0u);
+                       n_expert, chunk, extra ? 1u : 0u, items2, n_items2, chunk2);
     return launched("group_tables");
 }
 

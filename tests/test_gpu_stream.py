@@ -7,6 +7,7 @@ import pytest
 
 torch = pytest.importorskip("torch")
 
+from deepstrix_amd.capi import FMT_Q8_0
 from deepstrix_amd.executor import MoeLayer
 from oracle import ref
 from tests import helpers as H
@@ -43,3 +44,28 @@ def test_stream_matches_the_oracle(monkeypatch, hidden, inter, T):
         # (1/127 of its block's largest value)
         assert H.max_rel(out, gemm) < 1e-3
     H.assert_close(out, ref.moe_forward(H.host_weights(s), x, sel, w), 2e-3, f"{hidden} x {inter} T={T}")
+
+
+@pytest.mark.parametrize("hidden,inter", [(512, 256), (1280, 768), (2048, 1280), (4352, 1024), (7168, 512)])
+@pytest.mark.parametrize("T", [2, 15, 16, 64])
+@pytest.mark.parametrize("shared", ["none", "same", "q8_0"])
+def test_stream_gate_up_beside_a_q8_0_down_matches_the_oracle(monkeypatch, hidden, inter, T, shared):
+    """Gate/up from the streaming kernel, down from the by-expert kernel and the int8 GEMM (16 tokens: two
+    picks per expert); the shared expert as the extra group or beside it; one expert named by nearly every
+    token."""
+    monkeypatch.setattr(MoeLayer, "v3_thresholds_below_experts", None)
+    fmts = dict(sh_gate_fmt=FMT_Q8_0, sh_down_fmt=FMT_Q8_0) if shared == "q8_0" else {}
+    s = H.Shape(hidden, inter, 16, 2, down_fmt=FMT_Q8_0, shared=shared != "none", seed=700 + T, **fmts, **ROUTER)
+    x, _, _ = H.host_inputs(s, T)
+    rng = np.random.default_rng(T)
+    sel = np.stack([rng.permutation(16)[:2] for _ in range(T)]).astype(np.int32)
+    sel[: T // 2, 0] = np.where(sel[: T // 2, 1] == 3, sel[: T // 2, 0], 3)
+    sel[T // 2, 1] = -1
+    w = rng.uniform(0.05, 0.6, sel.shape).astype(np.float32)
+    layer = MoeLayer(H.device_weights(s), T)
+    dx, ds, dwt = torch.from_numpy(x).cuda(), torch.from_numpy(sel).cuda(), torch.from_numpy(w).cuda()
+    out = layer.run(dx, None, selected_in=ds, weights_in=dwt).clone()
+    again = layer.run(dx, None, selected_in=ds, weights_in=dwt)
+    torch.cuda.synchronize()
+    assert torch.equal(out, again)
+    H.assert_close(out.cpu().numpy(), ref.moe_forward(H.host_weights(s), x, sel, w), 2e-3, f"{hidden} x {inter} T={T} {shared}")
