@@ -197,6 +197,32 @@ def test_default_thresholds_follow_the_picks_per_expert():
     assert 49 <= mixed["gemm_q8"] <= 64
 
 
+def _workspace_bytes(T, hidden, inter, n_expert, n_used, gate_fmt, down_fmt):
+    l = capi.lib()
+    d = _desc(hidden=hidden, inter=inter, n_expert=n_expert, n_used=n_used, gate_fmt=gate_fmt, up_fmt=gate_fmt,
+              down_fmt=down_fmt, sh_inter=inter, sh_gate_fmt=gate_fmt, sh_up_fmt=gate_fmt, sh_down_fmt=down_fmt,
+              sh_gate=0x1000, sh_up=0x1000, sh_down=0x1000)
+    rc, h = _create(d)
+    assert rc == 0, l.dsx_last_error()
+    n = l.dsx_moe_layer_workspace_bytes(h, T)
+    l.dsx_moe_layer_destroy(h)
+    return n
+
+
+def test_workspaces_do_not_grow():
+    """A caller may hold a buffer of a size that dsx_moe_layer_workspace_bytes has returned, and
+    dsx_moe_layer_forward_noalloc serves what fits DSX_NOALLOC_SCRATCH_BYTES: a new table of a path
+    goes into a region that is idle at that time, not behind the others."""
+    M, Q = capi.FMT_MXFP4, capi.FMT_Q8_0
+    v3 = (7168, 2048, 256, 8)
+    assert [_workspace_bytes(T, *v3, M, M) for T in (1, 15, 16, 64)] == [533504, 7899136, 8424704, 31908864]
+    assert _workspace_bytes(64, *v3, M, Q) == 31908864
+    assert _workspace_bytes(512, 2048, 1408, 64, 6, Q, Q) == 80995584
+    noalloc = int(re.search(r"#define\s+DSX_NOALLOC_SCRATCH_BYTES\s+\((\d+)u << 20\)", open(HEADER).read()).group(1)) << 20
+    for T, *shape in [(114, 1024, 256, 128, 8), (79, 1024, 768, 128, 8), (15, *v3)]:   # the largest that fit
+        assert _workspace_bytes(T, *shape, M, M) <= noalloc < _workspace_bytes(T + 1, *shape, M, M), shape
+
+
 def test_missing_library_is_an_import_error_not_a_fallback(monkeypatch):
     monkeypatch.setattr(capi, "_lib", None)
     monkeypatch.setattr(capi, "LIB_PATH", os.path.join(ROOT, "deepstrix_amd", "lib", "absent.so"))
