@@ -357,4 +357,28 @@ __device__ __forceinline__ void hc_post_store4(const HcPost &h, uint64_t t, uint
     }
 }
 
+// Where one product is launched both as a streaming kernel (items of 16 or 32 members) and as the grouped GEMM
+// (items of 128), which of the two computes it -- the other returns at once: the picks are known on the device
+// only.  Both launches, and a quantizer that belongs to one of them, read the same two counts.
+//
+// gain, in twelfths: streaming takes 2.9 us per item at 7168 x 2048, the GEMM 3.9 where it fills the chip, so
+// streaming pays up to 16/12 of the GEMM's items (256 experts, top-8, MXFP4 gate/up beside a Q8_0 down matrix,
+// uniform picks, layer us streaming / GEMM: 512 tokens, ratio 1.05: 1893 / 2094, 800 tokens, 1.14: 2183 / 2312,
+// 1000 tokens, 1.49: 2573 / 2453; all-MXFP4, Zipf-skewed, 512 tokens, about 1.25: 1591 / 1613).  Matrices of
+// up to 4 M elements: 18/12 (all-MXFP4, Zipf-skewed, about 1.35: 4096 x 1024, 128 experts, 440 tokens 311 / 346;
+// 2048 x 1536, 64 experts, 290 tokens 147 / 166).
+// fill: a GEMM of fewer items than workgroups that the chip holds (CUs / row tiles of gate/up) takes no less
+// time, so up to so many items -- and four more, which the idle launches make up for -- streaming pays whatever
+// the GEMM's count (every token on the same picks, streaming / GEMM with its idle launches: 4096 x 1024, fill
+// 68: 36 items 96 / 121, 72: 140 / 131; 4096 x 2048, fill 36: 36 items 108 / 124; 2048 x 1536, fill 46: 49
+// items 96 / 96; 7168 x 2048, fill 36: 63 items 247 / 186, 72: 334 / 238, 144: 585 / 412).
+struct StreamChoice {
+    const int32_t *n_stream_items, *n_gemm_items;   // null: nothing to choose
+    uint32_t gain, fill;
+    __device__ __forceinline__ bool offered() const { return n_stream_items != nullptr; }
+    __device__ __forceinline__ bool streams() const {
+        return 12u * (uint32_t)*n_stream_items <= max(gain * (uint32_t)*n_gemm_items, 12u * fill);
+    }
+};
+
 }  // namespace dsx

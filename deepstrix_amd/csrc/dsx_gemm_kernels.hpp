@@ -80,7 +80,7 @@ struct GemmParams {
     uint64_t bpe0, bpe1;
     const uint8_t *act;            // staged activation rows, act_row_bytes apart
     const int32_t *group_count, *group_offset, *members, *work_items, *n_work_items;
-    const int32_t *n_stream_items;   // items of a streaming launch that offers the same product, or null
+    StreamChoice choice;           // a streaming launch offers the same product
     const float *ew;               // [n_tokens, n_used]               (gate/up)
     uint8_t *midq;                 // staged rows out, out_row_bytes, or null (gate/up)
     float *mid;                    // f32 [dest rows, n_rows] or null  (gate/up)
@@ -92,15 +92,6 @@ struct GemmParams {
     uint32_t n_row_tiles;          // n_rows / 256 (gate/up) or n_rows / 512 (down)
     float clamp, sh_clamp;
 };
-
-// Where a gate/up product is launched both as a streaming kernel (items of 16 or 32 members) and as the GEMM
-// (items of 128), which one computes it: the picks are known on the device only.  Streaming takes 2.9 us per
-// item at 7168 x 2048, the GEMM 3.9 where it fills the chip, so streaming pays up to 4/3 of the GEMM's items
-// (256 experts, top-8, uniform picks, layer us streaming / GEMM: 512 tokens, ratio 1.05: 1893 / 2094, 800
-// tokens, 1.14: 2183 / 2312, 1000 tokens, 1.49: 2573 / 2453; every token on the same picks, 256 tokens, 4: 446 / 372).
-__device__ __forceinline__ bool stream_pays(uint32_t n_stream_items, uint32_t n_gemm_items) {
-    return 3u * n_stream_items <= 4u * n_gemm_items;
-}
 
 // Row of a per-(token, slot) table for member m = (token << 16) | slot; slot n_used is the
 // extra expert, whose rows follow the n_tokens * n_used routed ones.
@@ -142,7 +133,7 @@ __global__ __launch_bounds__(kGemmWaves * 64, MT == kGemmMT ? 2 : 4) void k_mxfp
     // weight stream.)
     const uint32_t xcd = blockIdx.x & 7u, seq = blockIdx.x >> 3;
     const uint32_t n_items = (uint32_t)*p.n_work_items;   // the grid is only an upper bound
-    if (PAIR && p.n_stream_items && stream_pays((uint32_t)*p.n_stream_items, n_items)) return;  // uniform
+    if (MT == kGemmMT && !PLANAR && p.choice.offered() && p.choice.streams()) return;  // uniform
     const uint32_t local = seq / p.n_row_tiles;
     // Many column tiles per expert (skewed routing, many tokens): the items are dealt to the XCDs
     // like cards, which spreads the wide groups -- contiguous ranges of the list (it is by expert)

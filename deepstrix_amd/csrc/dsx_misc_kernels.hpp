@@ -503,15 +503,15 @@ __global__ __launch_bounds__(256) void k_sanitize_picks(int32_t *__restrict__ ou
 }
 
 // Rows of f32 -> staged rows, FP6 planes or FP8 planes (the mid activations of the kernels for few
-// members per expert).
+// members per expert).  Launched beside a GEMM that stores its staged rows itself: choice.
 template <bool FP6>
 __global__ __launch_bounds__(256) void k_quantize_staged(uint8_t *__restrict__ out,
                                                          const float *__restrict__ x,
                                                          uint32_t n_rows, uint32_t n_sb,
-                                                         uint32_t row_bytes) {
+                                                         uint32_t row_bytes, StreamChoice choice) {
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t blk = blockIdx.x * 4u + (threadIdx.x >> 6);
-    if (blk >= n_rows * n_sb) return;
+    if (blk >= n_rows * n_sb || (FP6 && choice.offered() && !choice.streams())) return;
     const uint32_t t = blk / n_sb, b = blk - t * n_sb;
     const float4 v = *(const float4 *)(x + (uint64_t)blk * 256u + lane * 4u);
     uint8_t *row = out + (uint64_t)t * row_bytes;

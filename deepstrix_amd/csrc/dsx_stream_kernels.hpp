@@ -43,7 +43,7 @@ struct StreamParams {
     uint64_t bpe0, bpe1;
     const uint8_t *act;            // staged FP6 rows, act_row_bytes apart: by token (PAIR) or by dest row
     const int32_t *group_count, *group_offset, *members, *work_items, *n_work_items;
-    const int32_t *n_gemm_items;   // items of a GEMM launch that offers the same product, or null
+    StreamChoice choice;           // a GEMM launch offers the same product
     const float *ew;               // [n_tokens, n_used]   (PAIR)
     float *out;                    // PAIR: mid, else partial rows: f32 [dest rows, n_rows]
     uint32_t n_tokens, n_used, n_expert, n_rows, n_sb, act_row_bytes;
@@ -111,7 +111,7 @@ __global__ __launch_bounds__(kStThreads, 2) void k_mxfp4_stream(const StreamPara
     const uint32_t G = gridDim.x;
     const uint32_t r = G % 8u == 0u ? (blockIdx.x & 7u) * (G >> 3) + (blockIdx.x >> 3) : blockIdx.x;
     const uint32_t n_items = __builtin_amdgcn_readfirstlane((uint32_t)*p.n_work_items);
-    if (PAIR && p.n_gemm_items && !stream_pays(n_items, (uint32_t)*p.n_gemm_items)) return;   // uniform
+    if (p.choice.offered() && !p.choice.streams()) return;   // uniform
     const uint32_t n_ut = p.n_rows / (16u * kTiles);
     const uint64_t total = (uint64_t)n_items * n_ut;
     const uint64_t lo = total * r / G, hi = total * (r + 1u) / G;

@@ -69,3 +69,59 @@ def test_stream_gate_up_beside_a_q8_0_down_matches_the_oracle(monkeypatch, hidde
     torch.cuda.synchronize()
     assert torch.equal(out, again)
     H.assert_close(out.cpu().numpy(), ref.moe_forward(H.host_weights(s), x, sel, w), 2e-3, f"{hidden} x {inter} T={T} {shared}")
+
+
+def _picks(s, T, kind, seed):
+    rng = np.random.default_rng(seed)
+    sel = np.stack([rng.choice(s.n_expert, s.n_used, replace=False) for _ in range(T)]).astype(np.int32)
+    if kind == "same":
+        sel[:] = sel[0]
+    return sel, rng.uniform(0.05, 0.6, sel.shape).astype(np.float32)
+
+
+@pytest.mark.parametrize("shared", ["same", "q8_0", "none"])
+def test_picks_on_a_few_experts_take_the_gemm(shared):
+    """An all-MXFP4 layer, from gemm_min_tokens on: the device sends picks that all fall on a few experts to
+    the GEMM, whose bits a layer that only has the GEMM reproduces, and spread ones to the streaming kernels
+    (another order of the sums: other bits, the same values).  300 tokens: 80 or 90 items of 32 members against
+    24 or 27 of 128; 100 tokens: 32 or 36, of which the GEMM would leave most of the chip idle."""
+    fmts = dict(sh_gate_fmt=FMT_Q8_0, sh_down_fmt=FMT_Q8_0) if shared == "q8_0" else {}
+    s = H.Shape(4096, 1024, 128, 8, shared=shared != "none", seed=901, **fmts, **ROUTER)
+    dw = H.device_weights(s)
+    layer, gemm = MoeLayer(dw, 300), MoeLayer(dw, 300)
+    gemm.set_tuning(gemm_min_tokens=1)
+    for T in (100, 300):
+        x = torch.from_numpy(H.host_inputs(s, T)[0]).cuda()
+        for kind in ("same", "spread", "same"):   # one workspace: the counts of one call say nothing to the next
+            sel, w = (torch.from_numpy(a).cuda() for a in _picks(s, T, kind, T))
+            out = layer.run(x, None, selected_in=sel, weights_in=w)
+            want = gemm.run(x, None, selected_in=sel, weights_in=w)
+            torch.cuda.synchronize()
+            assert torch.equal(out, want) == (T == 300 and kind == "same"), (T, kind)
+            assert H.max_rel(out.cpu().numpy(), want.cpu().numpy()) < 1e-3, (T, kind)
+
+
+def test_a_captured_pass_chooses_at_every_replay():
+    s, T = H.Shape(4096, 1024, 128, 8, seed=902, **ROUTER), 300
+    layer = MoeLayer(H.device_weights(s), T)
+    x = torch.from_numpy(H.host_inputs(s, T)[0]).cuda()
+    sets = [tuple(torch.from_numpy(a).cuda() for a in _picks(s, T, kind, 3)) for kind in ("same", "spread")]
+    eager = [layer.run(x, None, selected_in=sel, weights_in=w).clone() for sel, w in sets]
+    sel, w = (t.clone() for t in sets[0])
+    out = torch.empty_like(x)
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        layer.run(x, None, out=out, selected_in=sel, weights_in=w)
+        side.synchronize()
+        with torch.cuda.graph(graph, stream=side):
+            layer.run(x, None, out=out, selected_in=sel, weights_in=w)
+    torch.cuda.synchronize()
+    for rep in range(4):
+        sel.copy_(sets[rep % 2][0])
+        w.copy_(sets[rep % 2][1])
+        out.fill_(float(rep))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager[rep % 2]), rep
