@@ -164,6 +164,13 @@ class MoeLayer:
         return dict(zip(("by_expert_chunk", "gemm_min_tokens", "gemm_q8_min_tokens", "decode_max_tokens",
                          "gemm_narrow_members", "share_min_tokens"), (int(x) for x in v)))
 
+    def streaming(self) -> tuple:
+        """First and last token count that take the streaming kernels, (0, 0) for none
+        (include/dsx_moe.h: dsx_moe_layer_get_streaming)."""
+        v = (C.c_uint32 * 2)()
+        check(lib().dsx_moe_layer_get_streaming(self._h, C.byref(v)))
+        return int(v[0]), int(v[1])
+
     def set_decode(self, fused: int = 0, spin_limit: int = 0):
         """fused: 1 = one launch for gate/up + down, pairing tokens that name one expert from 4
         tokens on (default), 3 = never pairing, 4 = pairing from 2 tokens on, 2 = one launch per

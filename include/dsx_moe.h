@@ -334,6 +334,10 @@ int dsx_moe_layer_set_profile_events(dsx_moe_layer *layer, void *gate_up_begin, 
 /* Tuning knobs with no counterpart in the reference; 0 keeps the current value.  The defaults follow
  * from the layer's shape: which path a token count takes depends on the picks an expert receives,
  * T * n_used / n_expert (in brackets: the DeepSeek-V3 shape, 256 experts, top-8).
+ * On the engine's rows a layer with MXFP4 gate/up takes the streaming kernels over a range of token counts
+ * (dsx_moe_layer_get_streaming) in front of what the values below say -- until the caller sets one of them, to
+ * whatever value: by_expert_chunk, gemm_min_tokens and gemm_narrow_members end the streaming of the layer,
+ * decode_max_tokens that of an all-MXFP4 layer up to so many tokens.
  * by_expert_chunk (1..16): token columns per work item of the small-batch by-expert path.
  * gemm_min_tokens (default for an all-MXFP4 layer: 3.5 picks per expert [112 tokens], 7 where
  * n_expert * inter / 256 < 512; MXFP4 gate/up with a Q8_0 down matrix 2 [64], 4 for
@@ -357,8 +361,15 @@ int dsx_moe_layer_set_tuning(dsx_moe_layer *layer, uint32_t by_expert_chunk, uin
  * GEMMs are int8 (all-Q8_0), [3] decode_max_tokens, [4] gemm_narrow_members, [5] the token count
  * from which the one-launch decode path pairs tokens that name one expert (0: never). */
 int dsx_moe_layer_get_tuning(const dsx_moe_layer *layer, uint32_t out[6]);
-/* Decode path of an all-MXFP4 layer (up to decode_max_tokens tokens); no counterpart in the
- * reference.  fused: 1 = gate/up, mid quantization, down and the slot-order sum in ONE launch
+/* The token counts that take the streaming kernels: out[0] the first, out[1] the last, both 0 where there are
+ * none (planar weights, Q8_0 gate/up, weights that are not 8-byte aligned, rows of more than 7168 values, values
+ * set by the caller as above).  By default, all-MXFP4: from 9 tokens at the earliest to below 18 picks per
+ * expert, 28 where a matrix has up to 4 M elements [9 .. 575]; beside a Q8_0 down matrix gate/up alone, from 2
+ * tokens to below 28 picks per expert [2 .. 895]; matrices under 4 M elements start later.  Where the same
+ * token count would take a grouped GEMM otherwise, the device chooses between the two by the picks. */
+int dsx_moe_layer_get_streaming(const dsx_moe_layer *layer, uint32_t out[2]);
+/* Decode path of an all-MXFP4 layer (up to decode_max_tokens tokens, or to where streaming begins); no
+ * counterpart in the reference.  fused: 1 = gate/up, mid quantization, down and the slot-order sum in ONE launch
  * whose workgroups hand results to each other through device memory (the default); from an eighth
  * of a pick per expert on (DeepSeek-V3 shape: 4 tokens), the tokens of a step that name one expert are paired and the expert is streamed
  * once per pair (the reference's drafter groups few picks by distinct expert likewise,
@@ -366,7 +377,7 @@ int dsx_moe_layer_get_tuning(const dsx_moe_layer *layer, uint32_t out[6]);
  * with and without pairing.  3 = the same launch, never pairing; 4 = the same launch, pairing
  * from 2 tokens on (for steps whose tokens mostly name the same experts, such as the
  * verification of consecutive draft tokens); 2 = one launch per stage; 0 keeps the current
- * value.  spin_limit (0 keeps): bound, in polling rounds of about half a microsecond, of every
+ * value.  2, 3 and 4 hold up to decode_max_tokens tokens, where by default (1) streaming may begin earlier.  spin_limit (0 keeps): bound, in polling rounds of about half a microsecond, of every
  * wait one workgroup does for another; values above 2^20 are taken as 2^20, so that every wait
  * stays bounded. */
 int dsx_moe_layer_set_decode(dsx_moe_layer *layer, uint32_t fused, uint32_t spin_limit);

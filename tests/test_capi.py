@@ -223,6 +223,47 @@ def test_workspaces_do_not_grow():
         assert _workspace_bytes(T, *shape, M, M) <= noalloc < _workspace_bytes(T + 1, *shape, M, M), shape
 
 
+def _streaming(tuning=(0, 0, 0, 0), decode=0, **kw):
+    """First and last token count on the streaming kernels, after set_tuning and set_decode."""
+    l = capi.lib()
+    rc, h = _create(_desc(**kw))
+    assert rc == 0, l.dsx_last_error()
+    assert l.dsx_moe_layer_set_tuning(h, *tuning) == 0 and l.dsx_moe_layer_set_decode(h, decode, 0) == 0
+    v = (C.c_uint32 * 2)()
+    assert l.dsx_moe_layer_get_streaming(h, C.byref(v)) == 0
+    l.dsx_moe_layer_destroy(h)
+    return tuple(int(x) for x in v)
+
+
+_V3 = dict(hidden=7168, inter=2048, n_expert=256, n_used=8)
+
+
+def test_values_that_the_caller_sets_are_not_passed_over_by_streaming():
+    assert _streaming(**_V3) == (9, 575)
+    mixed = dict(_V3, down_fmt=capi.FMT_Q8_0)
+    assert _streaming(**mixed) == (2, 895)
+    for tuning in [(4, 0, 0, 0), (0, 112, 0, 0), (0, 0, 0, 1)]:   # (the values that are the defaults)
+        assert _streaming(tuning, **_V3) == _streaming(tuning, **mixed) == (0, 0)
+    assert _streaming((0, 0, 14, 0), **_V3) == (15, 575)
+    assert _streaming((0, 0, 5, 0), **_V3) == (9, 575)
+    for form in (2, 3, 4):
+        assert _streaming(decode=form, **_V3) == (15, 575)
+        assert _streaming(decode=form, **mixed) == (2, 895)   # (no decode path beside a Q8_0 down matrix)
+    assert _streaming(decode=1, **_V3) == (9, 575)
+
+
+@pytest.mark.parametrize("odd", [dict(gate=0x1004), dict(up=0x1004), dict(down=0x1004), dict(gate_bpe=12), dict(up_bpe=12),
+                                 dict(down_bpe=12), dict(sh_gate=0x1004), dict(sh_up=0x1004), dict(sh_down=0x1004),
+                                 dict(hidden=7424), dict(inter=7424, sh_inter=7424),
+                                 dict(gate_fmt=capi.FMT_Q8_0, up_fmt=capi.FMT_Q8_0, sh_inter=0)])
+def test_operands_that_the_streaming_kernels_do_not_take(odd):
+    """Weights that are not 8-byte aligned, rows of more than 28 super-blocks, other formats."""
+    sh = dict(sh_inter=2048, sh_gate_fmt=capi.FMT_MXFP4, sh_up_fmt=capi.FMT_MXFP4, sh_down_fmt=capi.FMT_MXFP4,
+              sh_gate=0x1000, sh_up=0x1000, sh_down=0x1000)
+    assert _streaming(**dict(_V3, **sh)) == (9, 575)
+    assert _streaming(**{**_V3, **sh, **odd}) == (0, 0)
+
+
 def test_missing_library_is_an_import_error_not_a_fallback(monkeypatch):
     monkeypatch.setattr(capi, "_lib", None)
     monkeypatch.setattr(capi, "LIB_PATH", os.path.join(ROOT, "deepstrix_amd", "lib", "absent.so"))

@@ -125,3 +125,28 @@ def test_a_captured_pass_chooses_at_every_replay():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, eager[rep % 2]), rep
+
+
+def test_the_paths_that_a_caller_asks_for_run(monkeypatch):
+    """A by-expert chunk and a decode form that the caller sets decide the path: the same bits as where
+    thresholds that leave no other path are set."""
+    monkeypatch.setattr(MoeLayer, "v3_thresholds_below_experts", None)
+    s = H.Shape(4096, 1280, 32, 2, seed=903, **ROUTER)
+    dw = H.device_weights(s)
+
+    def run(T, set_up):
+        layer = MoeLayer(dw, T)
+        set_up(layer)
+        sel, w = (torch.from_numpy(a).cuda() for a in _picks(s, T, "spread", T))
+        return layer.run(torch.from_numpy(H.host_inputs(s, T)[0]).cuda(), None, selected_in=sel, weights_in=w)
+
+    by_expert = run(40, lambda l: l.set_tuning(gemm_min_tokens=1 << 30, decode_max_tokens=1))
+    assert torch.equal(run(40, lambda l: l.set_tuning(by_expert_chunk=4)), by_expert)
+    assert not torch.equal(run(40, lambda l: None), by_expert)
+    s = H.Shape(4096, 1280, 64, 2, seed=903, **ROUTER)
+    dw = H.device_weights(s)
+    one_launch = run(14, lambda l: l.set_tuning(decode_max_tokens=14, gemm_min_tokens=1 << 30))
+    for form in (2, 3, 4):
+        forced = run(14, lambda l: (l.set_tuning(decode_max_tokens=14, gemm_min_tokens=1 << 30), l.set_decode(form)))
+        assert torch.equal(run(14, lambda l: l.set_decode(form)), forced), form
+    assert not torch.equal(run(14, lambda l: None), one_launch)
