@@ -365,7 +365,7 @@ int dsx_moe_layer_get_tuning(const dsx_moe_layer *layer, uint32_t out[6]);
  * none (planar weights, Q8_0 gate/up, weights that are not 8-byte aligned, rows of more than 7168 values, values
  * set by the caller as above).  By default, all-MXFP4: from 9 tokens at the earliest to below 18 picks per
  * expert, 28 where a matrix has up to 4 M elements [9 .. 575]; beside a Q8_0 down matrix gate/up alone, from 2
- * tokens to below 28 picks per expert [2 .. 895]; matrices under 4 M elements start later.  Where the same
+ * tokens to below 28 picks per expert [2 .. 895]; few picks in all and matrices under 4 M elements start later.  Where the same
  * token count would take a grouped GEMM otherwise, the device chooses between the two by the picks. */
 int dsx_moe_layer_get_streaming(const dsx_moe_layer *layer, uint32_t out[2]);
 /* Decode path of an all-MXFP4 layer (up to decode_max_tokens tokens, or to where streaming begins); no

@@ -238,6 +238,22 @@ def _streaming(tuning=(0, 0, 0, 0), decode=0, **kw):
 _V3 = dict(hidden=7168, inter=2048, n_expert=256, n_used=8)
 
 
+@pytest.mark.parametrize("shape,slower,faster", [
+    # (hidden, inter, experts, top), token counts at which the older path was measured faster, and streaming
+    ((7168, 2048, 256, 8), [8], [9, 10, 64]),
+    ((7168, 2048, 256, 4), [9, 10, 12, 14], [17, 20]),
+    ((4096, 1024, 256, 4), [9, 12, 14, 16], [17, 20]),
+    ((4096, 1024, 128, 8), [8], [9, 10, 37]),
+    ((5120, 1536, 160, 6), [8, 9], [11, 12]),
+    ((4096, 1536, 128, 4), [9, 10], [11, 12]),
+    ((2048, 1536, 64, 6), [14, 16, 20, 22], [24, 28]),
+    ((2048, 768, 128, 8), [18, 20, 28, 32], [36, 40]),
+    ((1536, 1536, 64, 6), [14, 20, 28, 36], [38, 64])])
+def test_streaming_begins_where_it_is_faster(shape, slower, faster):
+    first, last = _streaming(**dict(zip(("hidden", "inter", "n_expert", "n_used"), shape)))
+    assert max(slower) < first <= min(faster) and max(faster) <= last, (first, last)
+
+
 def test_values_that_the_caller_sets_are_not_passed_over_by_streaming():
     assert _streaming(**_V3) == (9, 575)
     mixed = dict(_V3, down_fmt=capi.FMT_Q8_0)
