@@ -367,17 +367,21 @@ __device__ __forceinline__ void hc_post_store4(const HcPost &h, uint64_t t, uint
 // 1000 tokens, 1.49: 2573 / 2453; all-MXFP4, Zipf-skewed, 512 tokens, about 1.25: 1591 / 1613).  Matrices of
 // up to 4 M elements: 18/12 (all-MXFP4, Zipf-skewed, about 1.35: 4096 x 1024, 128 experts, 440 tokens 311 / 346;
 // 2048 x 1536, 64 experts, 290 tokens 147 / 166).
-// fill: a GEMM of fewer items than workgroups that the chip holds (CUs / row tiles of gate/up) takes no less
-// time, so up to so many items -- and four more, which the idle launches make up for -- streaming pays whatever
-// the GEMM's count (every token on the same picks, streaming / GEMM with its idle launches: 4096 x 1024, fill
-// 68: 36 items 96 / 121, 72: 140 / 131; 4096 x 2048, fill 36: 36 items 108 / 124; 2048 x 1536, fill 46: 49
-// items 96 / 96; 7168 x 2048, fill 36: 63 items 247 / 186, 72: 334 / 238, 144: 585 / 412).
+// round, fill: the items that the GEMM's gate/up launch computes at a time -- every XCD takes whole items -- and
+// 7/8 of what its workgroups would be on all CUs.  A GEMM of few items takes as long as one of a full round, so up
+// to `fill` items streaming pays whatever the GEMM's count, and up to 1.25 fill more for each further round
+// (all-MXFP4, us GEMM / streaming; every token on the same picks: 4096 x 1024, round 64, 45 items 112 / 106, 63:
+// 112 / 127; 4096 x 2048, round 32, 36 items 112 / 129; 2048 x 1536, round 40, 42 items 89 / 87, 49: 89 / 95; picks
+// on 32 experts of 4096 x 2048, 33 GEMM items, about 60 items 217 / 160, 105: 241 / 281; on 64 of 4096 x 1024, 66
+// GEMM items, about 100 items 223 / 187; on 64 of 7168 x 2048, round 32, 66 GEMM items, about 100 items 524 / 545).
+// fill 0: gain alone.
 struct StreamChoice {
     const int32_t *n_stream_items, *n_gemm_items;   // null: nothing to choose
-    uint32_t gain, fill;
+    uint32_t gain, fill, round;
     __device__ __forceinline__ bool offered() const { return n_stream_items != nullptr; }
     __device__ __forceinline__ bool streams() const {
-        return 12u * (uint32_t)*n_stream_items <= max(gain * (uint32_t)*n_gemm_items, 12u * fill);
+        const uint32_t n = (uint32_t)*n_stream_items, gemm = (uint32_t)*n_gemm_items;
+        return 12u * n <= gain * gemm || 4u * n <= fill * (5u * ((gemm + round - 1u) / round) - 1u);
     }
 };
 

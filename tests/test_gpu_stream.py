@@ -101,6 +101,28 @@ def test_picks_on_a_few_experts_take_the_gemm(shared):
             assert H.max_rel(out.cpu().numpy(), want.cpu().numpy()) < 1e-3, (T, kind)
 
 
+@pytest.mark.parametrize("T,experts,streams", [(224, 48, False), (264, 64, True)])
+def test_the_device_chooses_by_the_rounds_of_the_gemm(T, experts, streams):
+    """Random picks on some of the experts: where the GEMM's items fit one round of the chip (64 at this width),
+    more than 56 streaming items go to it; where they make a second round, up to 126 stay."""
+    s = H.Shape(4096, 1024, 128, 8, seed=904, **ROUTER)
+    dw = H.device_weights(s)
+    layer, gemm = MoeLayer(dw, T), MoeLayer(dw, T)
+    gemm.set_tuning(gemm_min_tokens=1)
+    rng = np.random.default_rng(T)
+    sel = np.stack([rng.choice(experts, s.n_used, replace=False) for _ in range(T)]).astype(np.int32)
+    count = np.bincount(sel.reshape(-1), minlength=experts)
+    items = {c: int((-(-count // c)).sum()) + -(-T // c) for c in (32, 128)}
+    assert 1.5 * items[128] < items[32] and 56 < items[32] <= 126 and (items[128] > 64) == streams
+    x = torch.from_numpy(H.host_inputs(s, T)[0]).cuda()
+    sel, w = torch.from_numpy(sel).cuda(), torch.full((T, s.n_used), 0.3, device="cuda")
+    out = layer.run(x, None, selected_in=sel, weights_in=w)
+    want = gemm.run(x, None, selected_in=sel, weights_in=w)
+    torch.cuda.synchronize()
+    assert torch.equal(out, want) == (not streams)
+    assert H.max_rel(out.cpu().numpy(), want.cpu().numpy()) < 1e-3
+
+
 def test_a_captured_pass_chooses_at_every_replay():
     s, T = H.Shape(4096, 1024, 128, 8, seed=902, **ROUTER), 300
     layer = MoeLayer(H.device_weights(s), T)
