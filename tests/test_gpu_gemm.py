@@ -103,12 +103,16 @@ def test_gemm_path_skewed_routing():
     assert H.max_rel(got, base) < BASE_TOL
 
 
-def test_config2_v3_shape_T256_takes_the_gemm_path_by_default():
+@pytest.mark.parametrize("T", [256, 600])
+def test_config2_v3_shape_on_the_gemm_path(T):
+    """256 tokens with the streaming kernels off, 600 by default."""
     s = H.CFG2
-    T = 256
     x, logits, bias = H.host_inputs(s, T)
     dw = H.device_weights(s)
     layer = MoeLayer(dw, T)
+    if T == 256:
+        layer.set_tuning(gemm_min_tokens=layer.tuning()["gemm_min_tokens"])
+    assert layer.tuning()["gemm_min_tokens"] == 112 and layer.streaming()[1] < T
     out, sel, w = layer.run(torch.from_numpy(x).cuda(), torch.from_numpy(logits).cuda(),
                             want_routing=True)
     torch.cuda.synchronize()
@@ -117,8 +121,8 @@ def test_config2_v3_shape_T256_takes_the_gemm_path_by_default():
     _, scores = ref.router_scores(logits, bias, s.router_mode, s.n_group, s.topk_group)
     assert H.routing_mismatch_explained(sel_h, rsel, scores, s.n_used) == []
     # the oracle on a sample of tokens (each token is independent of the others)
-    pick = np.arange(0, T, 8)
-    hw = H.host_weights(s, experts=np.unique(sel_h[pick]))
+    pick = np.arange(0, T, T // 32)
+    hw = H.host_weights_from_device(s, dw, experts=np.unique(sel_h[pick]))
     want = ref.moe_forward(hw, x[pick], sel_h[pick], w_h[pick])
     assert H.max_rel(out.cpu().numpy()[pick], want) < OUT_TOL
 
@@ -127,7 +131,7 @@ def test_config3_v3_shape_T4096_zipf_routing():
     """BASELINE config 3 at its full size.  Checked three ways: the routing of all 4096 tokens
     against the oracle; a sample of tokens against the oracle's layer; and the size-independent
     property that a token's output does not depend on its batch -- 64 tokens taken out of the
-    4096 and run on their own (by-expert path, T=64) must give the rows they had in the batch."""
+    4096 and run on their own (by the streaming and by the by-expert kernels, T=64) must give the rows they had in the batch."""
     s = H.CFG2
     T = 4096
     shift = 0.416 * H.zipf_logit_shift(s.n_expert, 3)  # top 10 % of the experts get ~50 % of the picks
@@ -153,8 +157,12 @@ def test_config3_v3_shape_T4096_zipf_routing():
 
     sub = np.arange(17, T, 64)[:64]
     small = MoeLayer(dw, 64)
-    got = small.run(torch.from_numpy(x[sub]).cuda(), None,
-                    selected_in=torch.from_numpy(sel_h[sub]).cuda(),
-                    weights_in=torch.from_numpy(w_h[sub]).cuda())
-    torch.cuda.synchronize()
-    assert H.max_rel(out_h[sub], got.cpu().numpy()) < BASE_TOL
+    for streams in (True, False):
+        if not streams:
+            small.set_tuning(by_expert_chunk=4)
+        assert (small.streaming() != (0, 0)) == streams
+        got = small.run(torch.from_numpy(x[sub]).cuda(), None,
+                        selected_in=torch.from_numpy(sel_h[sub]).cuda(),
+                        weights_in=torch.from_numpy(w_h[sub]).cuda())
+        torch.cuda.synchronize()
+        assert H.max_rel(out_h[sub], got.cpu().numpy()) < BASE_TOL

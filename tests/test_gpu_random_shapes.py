@@ -1,6 +1,6 @@
 """Seeded random layers against the CPU oracle: shapes, formats, routers, shared-expert variants,
-token counts on every path (one-launch decode, by-expert kernels, grouped GEMMs) and both MXFP4
-layouts, drawn from a generator instead of being picked by hand.  Every case must be accepted by
+token counts on every path (one-launch decode, by-expert kernels, grouped GEMMs; with the library's own
+thresholds the streaming kernels too) and both MXFP4 layouts, drawn from a generator instead of being picked by hand.  Every case must be accepted by
 dsx_moe_layer_create (the generator only draws shapes the header documents as supported) and meet
 the same bar as the hand-picked layer tests."""
 import numpy as np
@@ -50,8 +50,10 @@ def draw_case(rng):
     return s, int(rng.choice(TOKEN_COUNTS)), bool(rng.random() < 0.3)
 
 
-@pytest.mark.parametrize("seed", [11, 12, 13, 14])
-def test_random_layers_match_the_oracle(seed):
+@pytest.mark.parametrize("seed,own_thresholds", [(11, False), (12, False), (13, False), (14, False), (15, True), (16, True)])
+def test_random_layers_match_the_oracle(monkeypatch, seed, own_thresholds):
+    if own_thresholds:
+        monkeypatch.setattr(MoeLayer, "v3_thresholds_below_experts", None)
     rng = np.random.default_rng(seed)
     for c in range(24):
         s, T, planar = draw_case(rng)

@@ -1,8 +1,8 @@
 """The reference's own layer mix -- MXFP4 routed experts beside a Q8_0 shared expert whose
 intermediate size differs from the routed one (docs/v41/ARCH_SPEC.md:239,
 crates/v4flash-kernels/src/het/dispatch.rs:196-214) -- against the CPU oracle at every token
-count that takes a different path: one launch / per-stage decode, by-expert, grouped GEMM with
-the shared expert on the int8 GEMM.  Up to three tokens the Q8_0 shared expert is computed by items
+count that takes a different path: one launch / per-stage decode, by-expert, streaming, grouped GEMM
+with the shared expert on the int8 GEMM.  Up to three tokens the Q8_0 shared expert is computed by items
 of the one-launch decode path, from four on by the dense kernels on a side stream."""
 import numpy as np
 import pytest
@@ -77,26 +77,30 @@ def test_small_layer_pre_norm_block_with_q8_0_shared_expert():
 
 
 @pytest.fixture(scope="module")
-def v3_layer():
+def v3_layers():
+    """The layer as it is, the same with the streaming kernels off, its bytes on the host."""
     dw = H.device_weights(V3)
-    return MoeLayer(dw, 512), H.host_weights_from_device(V3, dw)
+    layer, older = MoeLayer(dw, 512), MoeLayer(dw, 512)
+    older.set_tuning(by_expert_chunk=4)
+    assert layer.streaming() == (9, 575) and older.streaming() == (0, 0)
+    return layer, older, H.host_weights_from_device(V3, dw)
 
 
-@pytest.mark.parametrize("T", [1, 2, 4, 64, 512])
-def test_v3_shape_with_q8_0_shared_expert(T, v3_layer):
-    layer, hw = v3_layer
-    _check(V3, layer, hw, T, modes=(1, 2) if T <= 14 else (1,))
+@pytest.mark.parametrize("T,streams", [(1, True), (2, True), (4, True), (64, True), (512, True), (64, False), (512, False)])
+def test_v3_shape_with_q8_0_shared_expert(T, streams, v3_layers):
+    layer, older, hw = v3_layers
+    _check(V3, layer if streams else older, hw, T, modes=(1, 2) if T <= 14 else (1,))
 
 
-@pytest.mark.parametrize("T", [2, 4, 12, 24, 130])
-def test_side_stream_shared_expert_under_graph_capture(T, v3_layer):
-    """From seven tokens on (decode, by-expert and GEMM paths alike) the Q8_0 shared expert is
+@pytest.mark.parametrize("T,streams", [(2, True), (4, True), (12, True), (24, True), (130, True), (12, False), (24, False), (130, False)])
+def test_side_stream_shared_expert_under_graph_capture(T, streams, v3_layers):
+    """From seven tokens on (decode, by-expert, streaming and GEMM paths alike) the Q8_0 shared expert is
     computed on a stream of its own, forked from and joined to the caller's: a capture of the
     caller's stream must record both branches, and every replay must give what the eager call
     gives -- bitwise, with the program's own work and synchronizations between the replays.
     (Two and four tokens: the shared expert inside the decode launch, no second stream.)"""
     s = V3
-    layer, hw = v3_layer
+    layer = v3_layers[0 if streams else 1]
     layer.set_decode(fused=1)
     x, logits, _ = H.host_inputs(s, T)
     dx, dl = torch.from_numpy(x).cuda(), torch.from_numpy(logits).cuda()

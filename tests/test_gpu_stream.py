@@ -1,36 +1,44 @@
 """The streaming kernels for groups of few members (whole row tiles through LDS, columns in registers)
 against the CPU oracle: rows of an odd and an even number of super-blocks, each instance by row length
-(up to 4, 8, 16 and 28), groups around the 16- and 32-column items, empty slots, an expert that every
-token names (several items), no shared expert."""
+(gate/up: up to 8, 16 and 28 super-blocks, down: up to 4, 8, 16 and 28), groups around the 16- and
+32-column items, empty slots, an expert that nearly every token names (several items), no shared expert."""
 import numpy as np
 import pytest
 
 torch = pytest.importorskip("torch")
 
 from deepstrix_amd.capi import FMT_Q8_0
-from deepstrix_amd.executor import MoeLayer
+from deepstrix_amd.executor import MoeChain, MoeLayer
 from oracle import ref
 from tests import helpers as H
+from tests.test_gpu_chain import layer_shapes, verify_chain_stepwise
 
 pytestmark = pytest.mark.gpu
 
 ROUTER = dict(router_mode=1, route_scale=2.5, bias_sigma=0.01, clamp=10.0)
 # (hidden, inter): gate/up rows of hidden / 256 super-blocks, down rows of inter / 256
-SHAPES = [(512, 256), (1280, 768), (2048, 1280), (3328, 2304), (4096, 2048), (4352, 1024), (7168, 512)]
+SHAPES = [(512, 256), (1280, 768), (2048, 1280), (3328, 2304), (4096, 2048), (4352, 1024), (7168, 512), (512, 4352),
+          (512, 7168)]
 
 
 @pytest.mark.parametrize("hidden,inter", SHAPES)
-@pytest.mark.parametrize("T", [9, 33, 100])
-def test_stream_matches_the_oracle(monkeypatch, hidden, inter, T):
+@pytest.mark.parametrize("which", ["first", "23", "33", "last"])
+def test_stream_matches_the_oracle(monkeypatch, hidden, inter, which):
+    """The first and the last token count that stream, and 23 and 33: 23 (under 6 picks per expert) takes
+    16-column items, of which the expert that nearly every token names has two; from 24 on 32-column ones."""
     monkeypatch.setattr(MoeLayer, "v3_thresholds_below_experts", None)   # the library's own thresholds
-    s = H.Shape(hidden, inter, 8, 2, shared=hidden != 1280, seed=500 + T, **ROUTER)
+    s = H.Shape(hidden, inter, 8, 2, shared=hidden != 1280, seed=500, **ROUTER)
+    dw = H.device_weights(s)
+    first, last = MoeLayer(dw, 1).streaming()
+    T = {"first": first, "last": last}.get(which) or int(which)
+    assert 9 <= first <= 23 and 33 <= last and first <= T <= last
     x, _, _ = H.host_inputs(s, T)
     rng = np.random.default_rng(T)
     sel = np.stack([rng.permutation(8)[:2] for _ in range(T)]).astype(np.int32)
     sel[:, 0] = np.where(sel[:, 1] == 3, sel[:, 0], 3)     # nearly every token names expert 3
     sel[T // 2, 1] = -1                                    # an empty slot
     w = rng.uniform(0.05, 0.6, sel.shape).astype(np.float32)
-    layer = MoeLayer(H.device_weights(s), T)
+    layer = MoeLayer(dw, T)
     dx, ds, dwt = torch.from_numpy(x).cuda(), torch.from_numpy(sel).cuda(), torch.from_numpy(w).cuda()
     out = layer.run(dx, None, selected_in=ds, weights_in=dwt).clone()
     again = layer.run(dx, None, selected_in=ds, weights_in=dwt)
@@ -42,17 +50,17 @@ def test_stream_matches_the_oracle(monkeypatch, hidden, inter, T):
     if inter % 512 == 0 and hidden % 512 == 0:
         # other orders of the same f32 sums; a mid value may round to the neighbouring int8 step
         # (1/127 of its block's largest value)
-        assert H.max_rel(out, gemm) < 1e-3
+        assert H.max_rel(out, gemm) < 1e-3 and not np.array_equal(out, gemm)
     H.assert_close(out, ref.moe_forward(H.host_weights(s), x, sel, w), 2e-3, f"{hidden} x {inter} T={T}")
 
 
 @pytest.mark.parametrize("hidden,inter", [(512, 256), (1280, 768), (2048, 1280), (4352, 1024), (7168, 512)])
-@pytest.mark.parametrize("T", [2, 15, 16, 64])
+@pytest.mark.parametrize("T", [2, 10, 15, 16, 47, 64])
 @pytest.mark.parametrize("shared", ["none", "same", "q8_0"])
 def test_stream_gate_up_beside_a_q8_0_down_matches_the_oracle(monkeypatch, hidden, inter, T, shared):
     """Gate/up from the streaming kernel, down from the by-expert kernel and the int8 GEMM (16 tokens: two
-    picks per expert); the shared expert as the extra group or beside it; one expert named by nearly every
-    token."""
+    picks per expert); the shared expert as the extra group or beside it; one expert named by half of the
+    tokens and more (47: two 16-column items)."""
     monkeypatch.setattr(MoeLayer, "v3_thresholds_below_experts", None)
     fmts = dict(sh_gate_fmt=FMT_Q8_0, sh_down_fmt=FMT_Q8_0) if shared == "q8_0" else {}
     s = H.Shape(hidden, inter, 16, 2, down_fmt=FMT_Q8_0, shared=shared != "none", seed=700 + T, **fmts, **ROUTER)
@@ -63,6 +71,8 @@ def test_stream_gate_up_beside_a_q8_0_down_matches_the_oracle(monkeypatch, hidde
     sel[T // 2, 1] = -1
     w = rng.uniform(0.05, 0.6, sel.shape).astype(np.float32)
     layer = MoeLayer(H.device_weights(s), T)
+    first, last = layer.streaming()   # (2 tokens: where the matrices are large)
+    assert first == (2 if hidden * inter > 4 << 20 else 10) and T <= last
     dx, ds, dwt = torch.from_numpy(x).cuda(), torch.from_numpy(sel).cuda(), torch.from_numpy(w).cuda()
     out = layer.run(dx, None, selected_in=ds, weights_in=dwt).clone()
     again = layer.run(dx, None, selected_in=ds, weights_in=dwt)
@@ -172,3 +182,27 @@ def test_the_paths_that_a_caller_asks_for_run(monkeypatch):
         forced = run(14, lambda l: (l.set_tuning(decode_max_tokens=14, gemm_min_tokens=1 << 30), l.set_decode(form)))
         assert torch.equal(run(14, lambda l: l.set_decode(form)), forced), form
     assert not torch.equal(run(14, lambda l: None), one_launch)
+
+
+@pytest.mark.parametrize("fmt", ["mxfp4", "q8_0 shared", "q8_0 down"])
+@pytest.mark.parametrize("T", [15, 40])
+def test_a_stack_of_streaming_blocks(monkeypatch, fmt, T):
+    """h += layer(RMSNorm(h)), the residual added behind the streaming kernels and the shared expert inside or
+    beside them, in a chain: each block against the oracle, replays of a capture against eager steps."""
+    monkeypatch.setattr(MoeLayer, "v3_thresholds_below_experts", None)
+    kw = {"mxfp4": {}, "q8_0 shared": dict(sh_gate_fmt=FMT_Q8_0, sh_down_fmt=FMT_Q8_0), "q8_0 down": dict(down_fmt=FMT_Q8_0)}[fmt]
+    shapes = layer_shapes(H.Shape(2048, 512, 8, 2, seed=905, **kw, **ROUTER), 2)
+    chain = MoeChain([H.device_weights(s, block=True) for s in shapes], T)
+    for layer in chain.layers:
+        assert layer.streaming()[0] <= T <= layer.streaming()[1]
+    rng = np.random.default_rng(T)
+    chain.capture(T)
+    for step in range(3):
+        h = rng.normal(0, 1, (T, 2048)).astype(np.float32)
+        eager = chain.step(torch.from_numpy(h).cuda()).clone()
+        torch.cuda.synchronize()
+        replayed = chain.replay(torch.from_numpy(h).cuda()).clone()
+        torch.cuda.synchronize()
+        assert torch.equal(eager, replayed), step
+    final = verify_chain_stepwise(chain, shapes, h, 3 * 2e-3, min_checked=(9 * 2 * T) // 10)   # (the bar of the other chains)
+    assert np.array_equal(final, eager.cpu().numpy())
