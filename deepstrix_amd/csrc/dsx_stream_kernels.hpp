@@ -21,7 +21,13 @@
 // workgroups of one launch end within 5 % of each other at 64 tokens and 10 % at 16.  Measured and not
 // taken: the last tenth of the work claimed in chunks through a counter (64 tokens 4 % faster, 200 tokens 2
 // to 5 % slower: every chunk loads an item's columns again); a stage read into registers and its place
-// requested before the products (16 columns: no change; 32: the registers spill).
+// requested before the products (16 columns: no change; 32: the registers spill).  Scalar registers run out in
+// the instances for long rows (54 to 61 of them live in lanes of a vector register in gate/up, 33 to 36 in down;
+// no memory); what that costs was not measured.
+//
+// A shared expert of another format runs beside these on the layer's side stream although they take nearly all
+// of every CU's LDS: the layer of 256 experts 7168 x 2048 with a Q8_0 shared expert, us before / with the streaming
+// kernels: 24 tokens 750 / 674, 64: 1201 / 1061, 128: 1644 / 1274, 400: 1708 / 1457, 512: 1735 / 1486.
 #pragma once
 
 #include "dsx_device.hpp"
