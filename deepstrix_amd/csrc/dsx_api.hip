@@ -80,18 +80,32 @@ int need_init(const char *who) {
 template <bool PAIR, int NCG, typename F>
 int with_stream_kernel(uint32_t n_sb, F &&f) {
     if constexpr (PAIR) {
-        if (n_sb <= 8u) return f(k_mxfp4_stream<PAIR, 2, NCG, 2>, 2u);
+        if (n_sb <= 8u) return f(k_mxfp4_stream<PAIR, 2, NCG, 2>, 2u, 8u);
     } else {
-        if (n_sb <= 4u) return f(k_mxfp4_stream<PAIR, 1, NCG, 4>, 4u);
-        if (n_sb <= 8u) return f(k_mxfp4_stream<PAIR, 2, NCG, 2>, 2u);
+        if (n_sb <= 4u) return f(k_mxfp4_stream<PAIR, 1, NCG, 4>, 4u, 8u);
+        if (n_sb <= 8u) return f(k_mxfp4_stream<PAIR, 2, NCG, 2>, 2u, 8u);
     }
-    if (n_sb <= 16u) return f(k_mxfp4_stream<PAIR, 4, NCG, 1>, 1u);
-    return f(k_mxfp4_stream<PAIR, 7, NCG, 1>, 1u);
+    if (n_sb <= 16u) return f(k_mxfp4_stream<PAIR, 4, NCG, 1>, 1u, 8u);
+    return f(k_mxfp4_stream<PAIR, 7, NCG, 1>, 1u, 8u);
+}
+
+// The same for k_q8_0_stream (16 columns) and rows of n_sb groups of four blocks: f(kernel, row tiles per stage, waves).
+// Workgroups of four waves, two per CU, which overlap one's sums with the other's products, where half of the
+// LDS holds three stages (2048 x 1408, 64 experts, down, 4 / 40 tokens: 19 / 45 us against 22 / 48 with eight
+// waves; 7168 x 2048, two stages: 16 / 100 tokens 308 / 733 against 298 / 701) and for gate/up, whose SwiGLU takes
+// longer (2048 x 1408: 30 / 80 us against 34 / 79).
+template <bool PAIR, typename F>
+int with_q8_stream_kernel(uint32_t n_sb, F &&f) {
+    if (n_sb <= 8u) return f(k_q8_0_stream<PAIR, 8, 1, 2>, 2u, 8u);
+    if (n_sb <= (PAIR ? 16u : 12u)) return f(k_q8_0_stream<PAIR, 4, 4, 1>, 1u, 4u);
+    if constexpr (!PAIR)
+        if (n_sb <= 16u) return f(k_q8_0_stream<PAIR, 8, 2, 1>, 1u, 8u);
+    return f(k_q8_0_stream<PAIR, 8, 4, 1>, 1u, 8u);
 }
 
 template <bool PAIR>
 void stream_raise_lds_limits() {
-    auto raise = [](auto kernel, uint32_t) {
+    auto raise = [](auto kernel, uint32_t, uint32_t) {
         (void)hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kStLds);
         return 0;
     };
@@ -99,6 +113,7 @@ void stream_raise_lds_limits() {
         with_stream_kernel<PAIR, 1>(n_sb, raise);
         with_stream_kernel<PAIR, 2>(n_sb, raise);
     }
+    for (uint32_t n_sb : {8u, 12u, 16u, kStQ8MaxSb}) with_q8_stream_kernel<PAIR>(n_sb, raise);
 }
 
 void raise_lds_limits() {
@@ -198,12 +213,12 @@ static int fit_nt(uint32_t chunk, uint32_t n_blocks, int cap) {
 // optional extra group `n_expert` that holds every token (slot n_used).
 int group_build_big(hipStream_t st, int32_t *group_count, int32_t *group_offset, int32_t *members,
                     int32_t *work_items, int32_t *n_work_items, const int32_t *selected, uint32_t b,
-                    uint32_t n_used, uint32_t n_expert, uint32_t chunk, bool extra, int32_t *items2 = nullptr,
-                    int32_t *n_items2 = nullptr, uint32_t chunk2 = 0) {
-    // items2: a second list of work items, of chunk2 members
-    hipLaunchKernelGGL(k_group_tables, dim3(n_expert + (extra ? 1u : 0u) + (items2 ? 2u : 1u)), dim3(kGbThreads), 0, st,
+                    uint32_t n_used, uint32_t n_expert, uint32_t chunk, bool extra, ItemList list2 = {}, ItemList list3 = {}) {
+    // list2, list3 (with list2): further lists of work items
+    const uint32_t lists = 1u + (list2.items ? 1u : 0u) + (list3.items ? 1u : 0u);
+    hipLaunchKernelGGL(k_group_tables, dim3(n_expert + (extra ? 1u : 0u) + lists), dim3(kGbThreads), 0, st,
                        group_count, group_offset, members, work_items, n_work_items, selected, b, n_used,
-                       n_expert, chunk, extra ? 1u : 0u, items2, n_items2, chunk2);
+                       n_expert, chunk, extra ? 1u : 0u, list2, list3);
     return launched("group_tables");
 }
 
@@ -232,17 +247,19 @@ int launch_gemm(hipStream_t st, const GemmParams &p, uint32_t max_wi, bool plana
 }
 
 // Streaming launch for groups of few members (items of up to 16 ncg members), one workgroup per CU.
+// q8: Q8_0 weights and activation rows.
 template <bool PAIR>
-int launch_stream(hipStream_t st, StreamParams p, uint32_t ncg) {
-    auto go = [&](auto kernel, uint32_t rt) -> int {
+int launch_stream(hipStream_t st, StreamParams p, uint32_t ncg, bool q8 = false) {
+    auto go = [&](auto kernel, uint32_t rt, uint32_t waves) -> int {
         const uint64_t act_rows = (uint64_t)p.n_tokens * (p.n_used + 1u);
-        if (p.n_rows % (16u * rt) || p.n_sb > kStMaxSb || !stream_layout(p, PAIR, rt, ncg))
+        if (p.n_rows % (16u * rt) || p.n_sb > (q8 ? kStQ8MaxSb : kStMaxSb) || !stream_layout(p, PAIR, rt, ncg, waves))
             return fail(DSX_ERR_SHAPE, "stream: %u rows of %u super-blocks", p.n_rows, p.n_sb);
         if (act_rows * p.act_row_bytes > 0xFFFFFFFFull)
             return fail(DSX_ERR_INVALID_ARG, "stream: the activation rows exceed 4 GiB");
-        hipLaunchKernelGGL(kernel, dim3((uint32_t)g_num_cu), dim3(kStThreads), stream_lds_bytes(p, PAIR, rt, ncg), st, p);
+        hipLaunchKernelGGL(kernel, dim3((uint32_t)g_num_cu * 8u / waves), dim3(waves * 64u), stream_lds_bytes(p, PAIR, rt, ncg, waves), st, p);
         return launched(PAIR ? "gate_up stream" : "down stream");
     };
+    if (q8) return with_q8_stream_kernel<PAIR>(p.n_sb, go);   // ncg == 1
     return ncg == 1u ? with_stream_kernel<PAIR, 1>(p.n_sb, go) : with_stream_kernel<PAIR, 2>(p.n_sb, go);
 }
 

@@ -198,6 +198,19 @@ __device__ __forceinline__ void lds_dma4_v(uint32_t lds_addr, const void *ptr) {
                  :: "s"(lds_addr), "v"(ptr) : "memory");
 }
 
+// At most n of the wave's vector memory operations may still be under way (n uniform; above 31: 31).
+__device__ __forceinline__ void wait_vm(uint32_t n) {
+#define DSX_VM(k) case k: asm volatile("s_waitcnt vmcnt(" #k ")" ::: "memory"); break;
+    switch (n) {
+        DSX_VM(0) DSX_VM(1) DSX_VM(2) DSX_VM(3) DSX_VM(4) DSX_VM(5) DSX_VM(6) DSX_VM(7) DSX_VM(8) DSX_VM(9)
+        DSX_VM(10) DSX_VM(11) DSX_VM(12) DSX_VM(13) DSX_VM(14) DSX_VM(15) DSX_VM(16) DSX_VM(17) DSX_VM(18)
+        DSX_VM(19) DSX_VM(20) DSX_VM(21) DSX_VM(22) DSX_VM(23) DSX_VM(24) DSX_VM(25) DSX_VM(26) DSX_VM(27)
+        DSX_VM(28) DSX_VM(29) DSX_VM(30)
+        default: asm volatile("s_waitcnt vmcnt(31)" ::: "memory"); break;
+    }
+#undef DSX_VM
+}
+
 // Weights of one super-block for the lane's row: its two nibble blocks (halves 0 and 1,
 // block kb of each) and the 8 scale bytes.
 struct WSuper {

@@ -674,21 +674,27 @@ __device__ __forceinline__ void group_count_body(
     }
 }
 
+// A list of work items of up to `chunk` members each; items null: none.
+struct ItemList {
+    int32_t *items, *n;
+    uint32_t chunk;
+};
+
 __global__ __launch_bounds__(kGbThreads) void k_group_tables(
     int32_t *__restrict__ group_count, int32_t *__restrict__ group_offset,
     int32_t *__restrict__ members, int32_t *__restrict__ work_items,
     int32_t *__restrict__ n_work_items, const int32_t *__restrict__ selected, uint32_t b,
-    uint32_t n_used, uint32_t n_expert, uint32_t chunk, uint32_t extra, int32_t *__restrict__ items2,
-    int32_t *__restrict__ n_items2, uint32_t chunk2) {
+    uint32_t n_used, uint32_t n_expert, uint32_t chunk, uint32_t extra, const ItemList list2,
+    const ItemList list3) {
     constexpr uint32_t kWaves = kGbThreads / 64;
     __shared__ uint32_t s_mine[kWaves], s_below[kWaves];
     const uint32_t n_groups = n_expert + (extra ? 1u : 0u);
     if (blockIdx.x >= n_groups) {
-        // a second cut of the same groups (other items) has a workgroup of its own, which writes the
-        // counts and offsets too, with the same values
-        const bool second = blockIdx.x > n_groups;
-        group_count_body(group_count, group_offset, second ? items2 : work_items, second ? n_items2 : n_work_items,
-                         selected, b, n_used, n_expert, second ? chunk2 : chunk, extra);
+        // other cuts of the same groups (other items) have a workgroup each, which writes the counts and
+        // offsets too, with the same values
+        const uint32_t which = blockIdx.x - n_groups;
+        const ItemList l = which == 0u ? ItemList{work_items, n_work_items, chunk} : which == 1u ? list2 : list3;
+        group_count_body(group_count, group_offset, l.items, l.n, selected, b, n_used, n_expert, l.chunk, extra);
         return;
     }
     const uint32_t e = blockIdx.x, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63u;

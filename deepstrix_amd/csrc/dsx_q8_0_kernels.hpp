@@ -18,6 +18,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "../../include/dsx_moe.h"
 #include "dsx_device.hpp"
 #include "dsx_quant.hpp"
@@ -25,6 +27,52 @@
 namespace dsx {
 
 int q8_0_fail(int code, const char *what, const char *why);
+
+typedef int v4i32 __attribute__((ext_vector_type(4)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+
+// The products f16(d_w) * xscale of a 16 x 16 fragment and four blocks: an outer product per block, which the
+// matrix pipe makes for the four of them in one instruction (rounded once, as a vector multiplication would;
+// together with Q8Frag, 512 tokens of 2048 x 1408, 64 experts, wide tile: gate/up 151 -> 134 us, down 93 -> 85).
+// In: the lane's row (dw) or column (xs) n16 = lane % 16 of block lane / 16.  Out: [4 b + q] is row 4 (lane / 16)
+// + q of block b, column n16.  Per value and block the vector pipe is left with the convert and the fused add, two
+// instructions instead of three, and the rows' scales take one register instead of sixteen.
+__device__ __forceinline__ v16f q8_0_scales(float dw, float xs) {
+    return __builtin_amdgcn_mfma_f32_16x16x1f32(dw, xs, v16f{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f},
+                                                0, 0, 0);
+}
+
+// Four blocks of a 16 x 16 fragment: the integer sums of each and the scale products.  Started (five matrix
+// instructions) and added up (32 vector instructions) apart, so that one fragment's sums are under way while
+// another's are folded: left alone the compiler waits out every block's matrix instruction before its fold.
+struct Q8Frag {
+    // the bits of 1.5 * 2^23: an integer |s| < 2^22 added to them (32 products of int8 are below 2^20) makes the float
+    // 12582912 + s, so that a subtraction stands in for the convert (the layer of 512 tokens, 64 experts: 3 us of 145)
+    static constexpr int kMagic = 0x4B400000;
+    v4i32 s[4];
+    v16f sc;
+    __device__ __forceinline__ void start(const long (&a)[4], const long (&b)[4], float dw, float xs) {
+        sc = q8_0_scales(dw, xs);
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            s[k] = __builtin_amdgcn_mfma_i32_16x16x32_i8(a[k], b[k], v4i32{kMagic, kMagic, kMagic, kMagic}, 0, 0, 0);
+    }
+    __device__ __forceinline__ void fold(float (&acc)[4]) const {
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) acc[q] = fmaf(sc[4 * k + q], __int_as_float(s[k][q]) - 12582912.0f, acc[q]);
+    }
+    // behind start() of one fragment and fold() of the one before: a matrix instruction, six vector ones, ..
+    __device__ static __forceinline__ void interleave() {
+#pragma unroll
+        for (int k = 0; k < 5; k++) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+};
 
 constexpr int kQ8Waves = 4;
 constexpr int kQ8RowsPerWg = 16;
@@ -455,26 +503,31 @@ inline int q8_0_down_by_expert(hipStream_t st, float *partials, const uint8_t *d
 
 // ---------------------------------------------------------------------------------------
 // Expert products for many tokens per expert: grouped GEMMs on the int8 matrix instruction.
-// Work item = (expert, first member), the next up to 128 members are the token columns; a
-// workgroup (4 waves) multiplies 64 weight rows with them over all k, wave w owning rows
+// Work item = (expert, first member), the next up to 128 members are the token columns -- 32 in the narrow
+// tile; a workgroup (4 waves) multiplies 64 weight rows with them over all k, wave w owning rows
 // 16 w .. 16 w + 15 and all columns.
 //   gate/up (PAIR):  the 64 rows of gate and the same 64 rows of up; the epilogue applies the
 //                    clamped SwiGLU and the routing weight and stores f32 mid rows;
 //   down:            f32 partial rows, one per (token, slot).
 // One v_mfma_i32_16x16x32_i8 is exactly one Q8_0 block of a 16 x 16 fragment; its int32 sums
-// are folded into the f32 accumulators with f16(d_w) * xscale, as in q8_0_row_partial.
+// are folded into the f32 accumulators with f16(d_w) * xscale (Q8Frag).
 // Operands are fetched in memory order by LDS-direct loads (see lds_dma16) in chunks of 4
-// blocks (128 k), double buffered: the weights into a region private to the wave, the
+// blocks (128 k) into a ring of buffers: the weights into a region private to the wave, the
 // activations (and their scales) shared; 16-byte units are XOR-swizzled with the row so
 // that the 8-byte operand reads spread over the banks.  The extra expert (index n_expert,
 // slot n_used) like in the MXFP4 GEMM.
-// LDS: B[2][16 KB] | xs[2][2 KB] | A[4 waves][M][2][2 KB] | dw[M][64 rows][n_blocks] f16,
-// M = 2 matrices for PAIR, else 1.
+// The narrow tile is for up to 28 picks per expert, where the kernel only streams weights: its workgroups need a
+// third to two thirds of the LDS, so that three (gate/up) or four (down) of a CU wait for their chunks side by side
+// where the wide tile has two.  A value's terms and their order are those of the wide tile: the same bits.  Measured, us wide /
+// narrow: down 7168 x 2048, 256 experts, top-8: 100 tokens 871 / 681 (5.7 TB/s), 512: 1040 / 870, 850: 1163 / 990; 2048 x
+// 1408, 64 experts, top-6, both products, 64 tokens: 157 / 142, 200: 166 / 152, 300: 183 / 186.  With few columns
+// per expert it is bound by the weight stream; with 48 (512 tokens) the vector pipe is 54 % busy, the matrix pipe 22 %,
+// and the workgroups' last round is part empty.
 // ---------------------------------------------------------------------------------------
 constexpr int kQgWaves = 4;
 constexpr int kQgCols = 128;
+constexpr int kQgColsNarrow = 32;
 constexpr int kQgRows = 64;
-constexpr uint32_t kQgBOff = 0, kQgXsOff = 2 * 16384, kQgAOff = kQgXsOff + 2 * 2048;
 
 struct Q8GemmParams {
     float *out;                    // PAIR: f32 mid [dest rows, n_rows]; else partials [dest rows, n_rows]
@@ -485,26 +538,34 @@ struct Q8GemmParams {
     const float *ew;               // [n_tokens, n_used]   (PAIR)
     const int32_t *group_count, *group_offset, *members, *work_items, *n_work_items;
     uint32_t n_tokens, n_used, n_expert, n_rows, n_blocks, act_row_bytes, n_row_tiles;
+    uint32_t chunk;                // members of a work item, up to the tile's columns
     float clamp, sh_clamp;
 };
 
-// columns (double buffered) | activation scales | the waves' weight chunks (double buffered) | the
-// rows' block scales of two chunks at a time (double buffered): 72 KB with both matrices, so that
-// two workgroups share a CU
-inline size_t q8_0_gemm_lds_bytes(bool pair) {
-    const uint32_t m = pair ? 2u : 1u;
-    return kQgAOff + (size_t)kQgWaves * m * 4096u + (size_t)2u * m * kQgRows * 16u;
-}
+// DEPTH buffers of: columns | activation scales | the waves' weight chunks; two of: the rows' block scales of
+// two chunks
+// 32 columns (narrow): three buffers of down's 13 KB chunks (four workgroups per CU), two of gate/up's 21 KB
+// (three); 128: two (two workgroups per CU)
+template <bool PAIR, int COLS>
+struct Q8GemmLds {
+    static constexpr int DEPTH = COLS < 64 && !PAIR ? 3 : 2;
+    static constexpr uint32_t kM = PAIR ? 2u : 1u;
+    static constexpr uint32_t kB = (uint32_t)COLS * 128u, kXs = (uint32_t)COLS * 16u;
+    static constexpr uint32_t kXsOff = DEPTH * kB, kAOff = kXsOff + DEPTH * kXs;
+    static constexpr uint32_t kAWave = kM * DEPTH * 2048u;   // [matrix][buffer][2 KB]
+    static constexpr uint32_t kDwOff = kAOff + kQgWaves * kAWave;
+    static constexpr uint32_t kBytes = kDwOff + 2u * kM * kQgRows * 16u;
+};
 
-typedef int v4i32 __attribute__((ext_vector_type(4)));
-
-template <bool PAIR>
-__global__ __launch_bounds__(kQgWaves * 64) void k_q8_0_gemm(const Q8GemmParams p) {
+template <bool PAIR, int COLS>
+__global__ __launch_bounds__(kQgWaves * 64, COLS >= 64 ? 2 : PAIR ? 3 : 4) void k_q8_0_gemm(const Q8GemmParams p) {
     constexpr uint32_t M = PAIR ? 2u : 1u;
+    using L = Q8GemmLds<PAIR, COLS>;
+    constexpr int DEPTH = L::DEPTH;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    __shared__ uint32_t s_dest[kQgCols];
-    __shared__ uint32_t s_src[kQgCols];
-    __shared__ float s_ew[kQgCols];
+    __shared__ uint32_t s_dest[COLS];
+    __shared__ uint32_t s_src[COLS];
+    __shared__ float s_ew[COLS];
 
     const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63u;
     const uint32_t g4 = lane >> 4, n16 = lane & 15u;
@@ -527,10 +588,10 @@ __global__ __launch_bounds__(kQgWaves * 64) void k_q8_0_gemm(const Q8GemmParams 
 
     const uint32_t wi = (uint32_t)p.work_items[item];
     const uint32_t e = wi >> 16, start = wi & 0xFFFFu;
-    const uint32_t cnt = min((uint32_t)kQgCols, (uint32_t)p.group_count[e] - start);
+    const uint32_t cnt = min(p.chunk, (uint32_t)p.group_count[e] - start);
     const uint32_t mbase = (uint32_t)p.group_offset[e] + start;
     const bool extra = e >= p.n_expert;
-    if (tid < (uint32_t)kQgCols) {
+    if (tid < (uint32_t)COLS) {
         // columns past the end of the group repeat its last member; they are never stored
         const uint32_t m = (uint32_t)p.members[mbase + min(tid, cnt - 1u)];
         const uint32_t t = m >> 16, slot = m & 0xFFFFu;
@@ -546,118 +607,144 @@ __global__ __launch_bounds__(kQgWaves * 64) void k_q8_0_gemm(const Q8GemmParams 
 
     // the rows' block scales travel with the chunks: 16 bytes per row hold the scales of two chunks
     // (8 blocks), fetched by one instruction per matrix every other chunk (wave mm: lane -> row)
-    const uint32_t dw_off = kQgAOff + kQgWaves * M * 4096u;
-    const uint8_t *s_dw = smem + dw_off;   // [buffer][matrix][row][16 B]
+    const uint8_t *s_dw = smem + L::kDwOff;   // [buffer][matrix][row][16 B]
     __syncthreads();  // s_src visible
 
     const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
     const uint32_t l8 = lane >> 3, c8 = (lane & 7u) ^ l8;
     // A: wave w, matrix mm, rows 16 w + 8 i + l8, 16-byte unit c8 of the chunk's 128 bytes
-    const uint32_t a_lds = __builtin_amdgcn_readfirstlane(lds0 + kQgAOff + wave * M * 4096u);
+    const uint32_t a_lds = __builtin_amdgcn_readfirstlane(lds0 + L::kAOff + wave * L::kAWave);
     const uint32_t a_fetch = (wave * 16u + l8) * row_bytes + nb * 2u + c8 * 16u;
-    // B: wave w fetches columns 32 w + 8 ii + l8
-    const uint32_t b_lds = __builtin_amdgcn_readfirstlane(lds0 + kQgBOff + wave * 4096u);
-    uint32_t b_fetch[4];
+    // B: wave w fetches columns COLS / 4 w + 8 ii + l8
+    constexpr int kBLoads = COLS / 32;
+    const uint32_t b_lds = __builtin_amdgcn_readfirstlane(lds0 + wave * (uint32_t)kBLoads * 1024u);
+    uint32_t b_fetch[kBLoads];
 #pragma unroll
-    for (int ii = 0; ii < 4; ii++)
-        b_fetch[ii] = s_src[wave * 32u + ii * 8u + l8] * p.act_row_bytes + c8 * 16u;
-    // activation scales: waves 0 and 1, lane -> column 64 w + lane, the chunk's 4 floats
-    const uint32_t xs_lds = __builtin_amdgcn_readfirstlane(lds0 + kQgXsOff + (wave & 1u) * 1024u);
-    const uint32_t dw_lds = __builtin_amdgcn_readfirstlane(lds0 + dw_off);
+    for (int ii = 0; ii < kBLoads; ii++)
+        b_fetch[ii] = s_src[wave * (uint32_t)kBLoads * 8u + ii * 8u + l8] * p.act_row_bytes + c8 * 16u;
+    // activation scales: the first waves, lane -> column 64 w + lane, the chunk's 4 floats
+    constexpr uint32_t kXsWaves = COLS > 64 ? 2u : 1u;
+    const uint32_t xs_lds = __builtin_amdgcn_readfirstlane(lds0 + L::kXsOff + (kXsWaves == 2u ? wave & 1u : 0u) * 1024u);
+    const uint32_t dw_lds = __builtin_amdgcn_readfirstlane(lds0 + L::kDwOff);
     const uint32_t wave_u = __builtin_amdgcn_readfirstlane(wave);
     const uint8_t *dw_base = (M == 2u && wave_u == 1u) ? wbase[M - 1] : wbase[0];   // wave mm fetches matrix mm's
-    const uint32_t xs_fetch = s_src[(wave & 1u) * 64u + lane] * p.act_row_bytes + nb * 32u;
-    const bool b_live = wave * 32u < cnt;
+    const uint32_t xs_fetch = s_src[((wave & 1u) * 64u + lane) % (uint32_t)COLS] * p.act_row_bytes + nb * 32u;
+    const bool b_live = wave_u * (uint32_t)kBLoads * 8u < cnt;
     auto issue = [&](uint32_t c, uint32_t buf) {
 #pragma unroll
         for (uint32_t mm = 0; mm < M; mm++)
 #pragma unroll
             for (int i = 0; i < 2; i++)
-                lds_dma16(a_lds + mm * 4096u + buf * 2048u + (uint32_t)i * 1024u, wbase[mm],
+                lds_dma16(a_lds + (mm * DEPTH + buf) * 2048u + (uint32_t)i * 1024u, wbase[mm],
                           a_fetch + (uint32_t)i * 8u * row_bytes + c * 128u);
         if (b_live) {
 #pragma unroll
-            for (int ii = 0; ii < 4; ii++)
-                lds_dma16(b_lds + buf * 16384u + (uint32_t)ii * 1024u, p.act, b_fetch[ii] + c * 128u);
+            for (int ii = 0; ii < kBLoads; ii++)
+                lds_dma16(b_lds + buf * L::kB + (uint32_t)ii * 1024u, p.act, b_fetch[ii] + c * 128u);
         }
-        if (wave < 2u) lds_dma16(xs_lds + buf * 2048u, p.act, xs_fetch + c * 16u);
+        if (wave_u < kXsWaves && (COLS >= 64 || lane < (uint32_t)COLS)) lds_dma16(xs_lds + buf * L::kXs, p.act, xs_fetch + c * 16u);
         // (a last, single chunk reads 8 bytes past the scales, into the row's own quants)
         if ((c & 1u) == 0u && wave_u < M)
             lds_dma16(dw_lds + ((c >> 1) & 1u) * (M * kQgRows * 16u) + wave_u * (kQgRows * 16u), dw_base,
                       lane * row_bytes + (c >> 1) * 16u);
     };
 
+    // the wave's loads of a chunk, without the block scales of the even ones
+    const uint32_t my_loads = 2u * M + (b_live ? (uint32_t)kBLoads : 0u) + (wave_u < kXsWaves ? 1u : 0u);
+
     // read side: lane (row / column n16, 8-byte piece g4 of a block's 32 bytes)
     const uint32_t rd = (n16 >> 3) * 1024u + (n16 & 7u) * 128u + (g4 & 1u) * 8u;
     const uint32_t rd_sw = n16 & 7u, rd_unit = g4 >> 1;
-    const uint8_t *a_ptr = smem + kQgAOff + wave * M * 4096u;
+    const uint8_t *a_ptr = smem + L::kAOff + wave * L::kAWave;
 
-    float acc[M][8][4];
+    float acc[M][COLS / 16][4];
 #pragma unroll
     for (uint32_t mm = 0; mm < M; mm++)
 #pragma unroll
-        for (int j = 0; j < 8; j++)
+        for (int j = 0; j < COLS / 16; j++)
 #pragma unroll
             for (int q = 0; q < 4; q++) acc[mm][j][q] = 0.0f;
 
     const uint32_t n_chunks = nb / 4u;
     const uint32_t nj = (cnt + 15u) / 16u;
-    issue(0, 0);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
+    for (uint32_t c = 0; c + 1u < DEPTH; c++)
+        if (c < n_chunks) issue(c, c);
+    uint32_t buf = 0, next = DEPTH - 1u;   // buffers of chunks c and c + DEPTH - 1
     for (uint32_t c = 0; c < n_chunks; c++) {
-        const uint32_t buf = c & 1u;
-        if (c + 1u < n_chunks) issue(c + 1u, buf ^ 1u);
-        const uint8_t *bb = smem + kQgBOff + buf * 16384u;
-        const uint8_t *xb = smem + kQgXsOff + buf * 2048u;
-        // the lane's 4 rows' scales of the chunk's 4 blocks, and its A operands
-        float dw[M][4][4];
+        // the chunk has landed; the DEPTH - 2 behind it may be under way.  Behind the barrier it has for every
+        // wave, and nobody reads chunk c - 1, whose buffer the next request fills
+        if constexpr (DEPTH == 2) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        else wait_vm(c + 1u < n_chunks ? my_loads + (wave_u < M ? (c & 1u) : 0u) : 0u);
+        static_assert(DEPTH <= 3, "one chunk behind the awaited one");
+        __syncthreads();
+        if (c + DEPTH - 1u < n_chunks) issue(c + DEPTH - 1u, next);
+        const uint8_t *bb = smem + buf * L::kB;
+        const uint8_t *xb = smem + L::kXsOff + buf * L::kXs;
+        // row n16's scale of block g4, and its A operands of the chunk's 4 blocks
+        float dw[M];
         long av[M][4];
 #pragma unroll
         for (uint32_t mm = 0; mm < M; mm++) {
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const uint2 h = *(const uint2 *)(s_dw + ((size_t)((c >> 1) & 1u) * M + mm) * (kQgRows * 16u) +
-                                                 (size_t)(wave * 16u + g4 * 4u + q) * 16u + (c & 1u) * 8u);
-                dw[mm][q][0] = __half2float(__ushort_as_half((uint16_t)(h.x & 0xFFFFu)));
-                dw[mm][q][1] = __half2float(__ushort_as_half((uint16_t)(h.x >> 16)));
-                dw[mm][q][2] = __half2float(__ushort_as_half((uint16_t)(h.y & 0xFFFFu)));
-                dw[mm][q][3] = __half2float(__ushort_as_half((uint16_t)(h.y >> 16)));
-            }
-            const uint8_t *ab = a_ptr + mm * 4096u + buf * 2048u;
+            dw[mm] = __half2float(__ushort_as_half(*(const uint16_t *)(
+                s_dw + ((size_t)((c >> 1) & 1u) * M + mm) * (kQgRows * 16u) + (size_t)(wave * 16u + n16) * 16u + (c & 1u) * 8u + g4 * 2u)));
+            const uint8_t *ab = a_ptr + (mm * DEPTH + buf) * 2048u;
 #pragma unroll
             for (int b = 0; b < 4; b++)
                 av[mm][b] = *(const long *)(ab + rd + (((uint32_t)(2 * b) + rd_unit) ^ rd_sw) * 16u);
         }
+        // fragment f = M j + mm; the columns' operands of a group are read two fragments ahead, the
+        // products started one ahead
+        auto columns = [&](int j, long (&bv)[4], float &xs) __attribute__((always_inline)) {
+            const uint8_t *bj = bb + (size_t)j * 2048u + rd;
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            if ((uint32_t)j < nj) {  // uniform
-                const float4 xs = *(const float4 *)(xb + (size_t)(j * 16u + n16) * 16u);
-                const float xsv[4] = {xs.x, xs.y, xs.z, xs.w};
-                const uint8_t *bj = bb + (size_t)j * 2048u + rd;
+            for (int b = 0; b < 4; b++) bv[b] = *(const long *)(bj + (((uint32_t)(2 * b) + rd_unit) ^ rd_sw) * 16u);
+            xs = *(const float *)(xb + (size_t)((uint32_t)j * 16u + n16) * 16u + g4 * 4u);
+        };
+        auto step = [&](auto groups) __attribute__((always_inline)) {
+            constexpr int kFrags = (int)M * decltype(groups)::value;
+            long bv[2][4];
+            float xs[2];
+            Q8Frag fr[2];
+            columns(0, bv[0], xs[0]);
+            if (kFrags > (int)M) columns(1, bv[1], xs[1]);
+            fr[0].start(av[0], bv[0], dw[0], xs[0]);
+            if (M == 1u && kFrags > 2) columns(2, bv[0], xs[0]);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int b = 0; b < 4; b++) {
-                    const long bv = *(const long *)(bj + (((uint32_t)(2 * b) + rd_unit) ^ rd_sw) * 16u);
-#pragma unroll
-                    for (uint32_t mm = 0; mm < M; mm++) {
-                        const v4i32 s = __builtin_amdgcn_mfma_i32_16x16x32_i8(av[mm][b], bv, v4i32{0, 0, 0, 0}, 0, 0, 0);
-                        // three vector instructions per value: scale product, convert, fused add
-                        acc[mm][j][0] = fmaf(dw[mm][0][b] * xsv[b], (float)s.x, acc[mm][j][0]);
-                        acc[mm][j][1] = fmaf(dw[mm][1][b] * xsv[b], (float)s.y, acc[mm][j][1]);
-                        acc[mm][j][2] = fmaf(dw[mm][2][b] * xsv[b], (float)s.z, acc[mm][j][2]);
-                        acc[mm][j][3] = fmaf(dw[mm][3][b] * xsv[b], (float)s.w, acc[mm][j][3]);
-                    }
+            for (int f = 0; f < kFrags; f++) {
+                if (f + 1 < kFrags) {
+                    const int j = (f + 1) / (int)M, mm = (f + 1) % (int)M;
+                    fr[(f + 1) & 1].start(av[mm], bv[j & 1], dw[mm], xs[j & 1]);
+                    // (the group's last use was just issued)
+                    if (mm == (int)M - 1 && (j + 2) * (int)M < kFrags) columns(j + 2, bv[j & 1], xs[j & 1]);
                 }
+                fr[f & 1].fold(acc[f % (int)M][f / (int)M]);
+                Q8Frag::interleave();
+            }
+        };
+        if constexpr (COLS == 32) {
+            if (nj == 1u) step(std::integral_constant<int, 1>{});   // uniform
+            else step(std::integral_constant<int, 2>{});
+        } else {
+            switch (nj) {
+                case 1: step(std::integral_constant<int, 1>{}); break;
+                case 2: step(std::integral_constant<int, 2>{}); break;
+                case 3: step(std::integral_constant<int, 3>{}); break;
+                case 4: step(std::integral_constant<int, 4>{}); break;
+                case 5: step(std::integral_constant<int, 5>{}); break;
+                case 6: step(std::integral_constant<int, 6>{}); break;
+                case 7: step(std::integral_constant<int, 7>{}); break;
+                default: step(std::integral_constant<int, 8>{}); break;
             }
         }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
+        buf = buf + 1u == DEPTH ? 0u : buf + 1u;
+        next = next + 1u == DEPTH ? 0u : next + 1u;
     }
 
     // the lane holds rows 16 w + 4 g4 + q of columns 16 j + n16
     const float clamp = extra ? p.sh_clamp : p.clamp;
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
+    for (int j = 0; j < COLS / 16; j++) {
         const uint32_t col = j * 16u + n16;
         if (col >= cnt) continue;
         float *dst = p.out + (uint64_t)s_dest[col] * p.n_rows + rt * kQgRows + wave * 16u + g4 * 4u;
@@ -675,25 +762,34 @@ __global__ __launch_bounds__(kQgWaves * 64) void k_q8_0_gemm(const Q8GemmParams 
 
 // Raised once per device by the library's set-up, with the device current.
 inline void q8_0_gemm_raise_lds_limits() {
-    (void)hipFuncSetAttribute((const void *)k_q8_0_gemm<true>, hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
-    (void)hipFuncSetAttribute((const void *)k_q8_0_gemm<false>, hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
+    (void)hipFuncSetAttribute((const void *)k_q8_0_gemm<true, kQgCols>, hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
+    (void)hipFuncSetAttribute((const void *)k_q8_0_gemm<false, kQgCols>, hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
+    (void)hipFuncSetAttribute((const void *)k_q8_0_gemm<true, kQgColsNarrow>, hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
+    (void)hipFuncSetAttribute((const void *)k_q8_0_gemm<false, kQgColsNarrow>, hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
 }
 
-template <bool PAIR>
-inline int q8_0_gemm(hipStream_t st, const Q8GemmParams &p, uint32_t max_wi) {
+template <bool PAIR, int COLS>
+inline int q8_0_gemm_launch(hipStream_t st, const Q8GemmParams &p, uint32_t max_wi) {
     if (max_wi == 0) return DSX_OK;
     if (p.n_rows % kQgRows || p.n_blocks % 4 || p.n_blocks == 0)
         return q8_0_fail(DSX_ERR_SHAPE, "q8_0 gemm", "n_rows must be a multiple of 64, k of 128");
     const uint64_t act_rows = (uint64_t)p.n_tokens * (p.n_used + 1u);
     if ((uint64_t)p.n_rows * p.n_blocks * 34u > 0xFFFFFFFFull || act_rows * p.act_row_bytes > 0xFFFFFFFFull)
         return q8_0_fail(DSX_ERR_INVALID_ARG, "q8_0 gemm", "a weight matrix or the activation rows exceed 4 GiB");
-    const size_t lds = q8_0_gemm_lds_bytes(PAIR);
+    const size_t lds = Q8GemmLds<PAIR, COLS>::kBytes;
     const uint32_t per_xcd = (max_wi + 7u) / 8u;
     const uint64_t grid = (uint64_t)8u * per_xcd * p.n_row_tiles;
     if (grid > 0x7FFFFFFFull) return q8_0_fail(DSX_ERR_INVALID_ARG, "q8_0 gemm", "grid too large");
-    hipLaunchKernelGGL(k_q8_0_gemm<PAIR>, dim3((uint32_t)grid), dim3(kQgWaves * 64), lds, st, p);
+    hipLaunchKernelGGL((k_q8_0_gemm<PAIR, COLS>), dim3((uint32_t)grid), dim3(kQgWaves * 64), lds, st, p);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? DSX_OK : q8_0_fail((int)e, "q8_0 gemm", hipGetErrorString(e));
+}
+
+// The tile follows from the members of a work item.
+template <bool PAIR>
+inline int q8_0_gemm(hipStream_t st, const Q8GemmParams &p, uint32_t max_wi) {
+    return p.chunk <= (uint32_t)kQgColsNarrow ? q8_0_gemm_launch<PAIR, kQgColsNarrow>(st, p, max_wi)
+                                              : q8_0_gemm_launch<PAIR, kQgCols>(st, p, max_wi);
 }
 
 }  // namespace dsx

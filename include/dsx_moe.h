@@ -338,6 +338,9 @@ int dsx_moe_layer_set_profile_events(dsx_moe_layer *layer, void *gate_up_begin, 
  * (dsx_moe_layer_get_streaming) in front of what the values below say -- until the caller sets one of them, to
  * whatever value: by_expert_chunk, gemm_min_tokens and gemm_narrow_members end the streaming of the layer,
  * decode_max_tokens that of an all-MXFP4 layer up to so many tokens.
+ * A Q8_0 down matrix behind MXFP4 gate/up and both products of an all-Q8_0 layer likewise run, until the caller
+ * sets by_expert_chunk or gemm_min_tokens, on streaming kernels up to a number of tokens (all-Q8_0: 2 tokens to
+ * below 4 picks per expert) and on a 32-column GEMM up to 28 picks per expert.
  * by_expert_chunk (1..16): token columns per work item of the small-batch by-expert path.
  * gemm_min_tokens (default for an all-MXFP4 layer: 3.5 picks per expert [112 tokens], 7 where
  * n_expert * inter / 256 < 512; MXFP4 gate/up with a Q8_0 down matrix 2 [64], 4 for
@@ -364,7 +367,7 @@ int dsx_moe_layer_get_tuning(const dsx_moe_layer *layer, uint32_t out[6]);
 /* The token counts that take the streaming kernels: out[0] the first, out[1] the last, both 0 where there are
  * none (planar weights, Q8_0 gate/up, weights that are not 8-byte aligned, rows of more than 7168 values, values
  * set by the caller as above).  By default, all-MXFP4: from 9 tokens at the earliest to below 18 picks per
- * expert, 28 where a matrix has up to 4 M elements [9 .. 575]; beside a Q8_0 down matrix gate/up alone, from 2
+ * expert, 28 where a matrix has up to 4 M elements [9 .. 575]; beside a Q8_0 down matrix (whose own path is not reported), from 2
  * tokens to below 28 picks per expert [2 .. 895]; few picks in all and matrices under 4 M elements start later.  Where the same
  * token count would take a grouped GEMM otherwise, the device chooses between the two by the picks. */
 int dsx_moe_layer_get_streaming(const dsx_moe_layer *layer, uint32_t out[2]);
