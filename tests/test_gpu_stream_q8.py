@@ -53,10 +53,10 @@ def test_all_q8_0_layer_matches_the_oracle(monkeypatch, hidden, inter, T):
     assert torch.equal(out, old) == (T >= 16)
 
 
-@pytest.mark.parametrize("hidden,inter", [(512, 256), (1280, 768), (2048, 2048), (7168, 512)])
+@pytest.mark.parametrize("hidden,inter,shared", [(512, 256, "none"), (1280, 768, "same"), (1280, 768, "q8_0"),
+                                                 (2048, 2048, "none"), (7168, 512, "same")])
 @pytest.mark.parametrize("T", [10, 15, 16, 23, 24, 111])
-@pytest.mark.parametrize("shared,planar", [("none", False), ("same", False), ("q8_0", True)])
-def test_q8_0_down_behind_mxfp4_gate_up_matches_the_oracle(monkeypatch, hidden, inter, T, shared, planar):
+def test_q8_0_down_behind_mxfp4_gate_up_matches_the_oracle(monkeypatch, hidden, inter, shared, T):
     fmts = dict(sh_gate_fmt=FMT_Q8_0, sh_down_fmt=FMT_Q8_0) if shared == "q8_0" else {}
     s = H.Shape(hidden, inter, 8, 2, down_fmt=FMT_Q8_0, shared=shared != "none", seed=820 + T, **fmts, **ROUTER)
     _run(s, T, T, monkeypatch)
@@ -67,3 +67,24 @@ def test_rows_longer_than_the_registers_take_the_older_paths(monkeypatch):
     s = H.Shape(4224, 256, 8, 2, FMT_Q8_0, FMT_Q8_0, shared=False, seed=850, **ROUTER)
     out, old = _run(s, 15, 5, monkeypatch)
     assert torch.equal(out, old)
+
+
+@pytest.mark.parametrize("hidden", [128, 384, 1152])
+@pytest.mark.parametrize("T", [1, 3, 33])
+def test_front_launch_of_q8_0_layers(hidden, T):
+    """Router, activation rows and status word in one launch: rows that are no multiple of the wave's 256 elements;
+    given logits and the same picks pinned make the same bits."""
+    s = H.Shape(hidden, 256, 16, 3, FMT_Q8_0, FMT_Q8_0, shared=False, seed=860, **ROUTER)
+    x, logits, bias = H.host_inputs(s, T)
+    layer = MoeLayer(H.device_weights(s), T)
+    dx = torch.from_numpy(x).cuda()
+    out, sel, w = (t.clone() for t in layer.run(dx, torch.from_numpy(logits).cuda(), want_routing=True))
+    pinned = layer.run(dx, None, selected_in=sel, weights_in=w)
+    torch.cuda.synchronize()
+    assert torch.equal(out, pinned)
+    rsel, _ = H.oracle_route(s, logits, bias)
+    _, scores = ref.router_scores(logits, bias, s.router_mode, s.n_group, s.topk_group)
+    sel, w = sel.cpu().numpy(), w.cpu().numpy()
+    assert H.routing_mismatch_explained(sel, rsel, scores, s.n_used) == []
+    want = ref.moe_forward(H.host_weights(s), x, sel, w)
+    H.assert_parity_up_to_rounding_steps(out.cpu().numpy(), want, H.host_weights(s), sel, f"{hidden} T={T}")
