@@ -504,7 +504,7 @@ inline int q8_0_down_by_expert(hipStream_t st, float *partials, const uint8_t *d
 // ---------------------------------------------------------------------------------------
 // Expert products for many tokens per expert: grouped GEMMs on the int8 matrix instruction.
 // Work item = (expert, first member), the next up to 128 members are the token columns -- 32 in the narrow
-// tile; a workgroup (4 waves) multiplies 64 weight rows with them over all k, wave w owning rows
+// tile, 64 in the middle one; a workgroup (4 waves) multiplies 64 weight rows with them over all k, wave w owning rows
 // 16 w .. 16 w + 15 and all columns.
 //   gate/up (PAIR):  the 64 rows of gate and the same 64 rows of up; the epilogue applies the
 //                    clamped SwiGLU and the routing weight and stores f32 mid rows;
@@ -523,9 +523,13 @@ inline int q8_0_down_by_expert(hipStream_t st, float *partials, const uint8_t *d
 // 1408, 64 experts, top-6, both products, 64 tokens: 157 / 142, 200: 166 / 152, 300: 183 / 186.  With few columns
 // per expert it is bound by the weight stream; with 48 (512 tokens) the vector pipe is 54 % busy, the matrix pipe 22 %,
 // and the workgroups' last round is part empty.
+// The middle tile is down's for the picks behind that, while most experts still make one item of 64: three workgroups per
+// CU for the wide tile's two (7168 x 2048, 256 experts, 1000 tokens: the layer 2349 -> 2143 us; four per CU spilled 24
+// registers).  Gate/up of 64 columns would need 54 KB and stay at two per CU.
 // ---------------------------------------------------------------------------------------
 constexpr int kQgWaves = 4;
 constexpr int kQgCols = 128;
+constexpr int kQgColsMiddle = 64;   // down only
 constexpr int kQgColsNarrow = 32;
 constexpr int kQgRows = 64;
 
@@ -544,6 +548,7 @@ struct Q8GemmParams {
 
 // DEPTH buffers of: columns | activation scales | the waves' weight chunks; two of: the rows' block scales of
 // two chunks
+// 64 columns: two buffers, three workgroups per CU (three buffers would not fit three times)
 // 32 columns (narrow): three buffers of down's 13 KB chunks (four workgroups per CU), two of gate/up's 21 KB
 // (three); 128: two (two workgroups per CU)
 template <bool PAIR, int COLS>
@@ -558,7 +563,7 @@ struct Q8GemmLds {
 };
 
 template <bool PAIR, int COLS>
-__global__ __launch_bounds__(kQgWaves * 64, COLS >= 64 ? 2 : PAIR ? 3 : 4) void k_q8_0_gemm(const Q8GemmParams p) {
+__global__ __launch_bounds__(kQgWaves * 64, COLS > 64 ? 2 : PAIR || COLS > 32 ? 3 : 4) void k_q8_0_gemm(const Q8GemmParams p) {
     constexpr uint32_t M = PAIR ? 2u : 1u;
     using L = Q8GemmLds<PAIR, COLS>;
     constexpr int DEPTH = L::DEPTH;
@@ -725,6 +730,13 @@ __global__ __launch_bounds__(kQgWaves * 64, COLS >= 64 ? 2 : PAIR ? 3 : 4) void 
         if constexpr (COLS == 32) {
             if (nj == 1u) step(std::integral_constant<int, 1>{});   // uniform
             else step(std::integral_constant<int, 2>{});
+        } else if constexpr (COLS == 64) {
+            switch (nj) {
+                case 1: step(std::integral_constant<int, 1>{}); break;
+                case 2: step(std::integral_constant<int, 2>{}); break;
+                case 3: step(std::integral_constant<int, 3>{}); break;
+                default: step(std::integral_constant<int, 4>{}); break;
+            }
         } else {
             switch (nj) {
                 case 1: step(std::integral_constant<int, 1>{}); break;
@@ -764,6 +776,7 @@ __global__ __launch_bounds__(kQgWaves * 64, COLS >= 64 ? 2 : PAIR ? 3 : 4) void 
 inline void q8_0_gemm_raise_lds_limits() {
     (void)hipFuncSetAttribute((const void *)k_q8_0_gemm<true, kQgCols>, hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
     (void)hipFuncSetAttribute((const void *)k_q8_0_gemm<false, kQgCols>, hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
+    (void)hipFuncSetAttribute((const void *)k_q8_0_gemm<false, kQgColsMiddle>, hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
     (void)hipFuncSetAttribute((const void *)k_q8_0_gemm<true, kQgColsNarrow>, hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
     (void)hipFuncSetAttribute((const void *)k_q8_0_gemm<false, kQgColsNarrow>, hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
 }
@@ -788,8 +801,10 @@ inline int q8_0_gemm_launch(hipStream_t st, const Q8GemmParams &p, uint32_t max_
 // The tile follows from the members of a work item.
 template <bool PAIR>
 inline int q8_0_gemm(hipStream_t st, const Q8GemmParams &p, uint32_t max_wi) {
-    return p.chunk <= (uint32_t)kQgColsNarrow ? q8_0_gemm_launch<PAIR, kQgColsNarrow>(st, p, max_wi)
-                                              : q8_0_gemm_launch<PAIR, kQgCols>(st, p, max_wi);
+    if (p.chunk <= (uint32_t)kQgColsNarrow) return q8_0_gemm_launch<PAIR, kQgColsNarrow>(st, p, max_wi);
+    if constexpr (!PAIR)
+        if (p.chunk <= (uint32_t)kQgColsMiddle) return q8_0_gemm_launch<PAIR, kQgColsMiddle>(st, p, max_wi);
+    return q8_0_gemm_launch<PAIR, kQgCols>(st, p, max_wi);
 }
 
 }  // namespace dsx

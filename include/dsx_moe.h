@@ -340,7 +340,8 @@ int dsx_moe_layer_set_profile_events(dsx_moe_layer *layer, void *gate_up_begin, 
  * decode_max_tokens that of an all-MXFP4 layer up to so many tokens.
  * A Q8_0 down matrix behind MXFP4 gate/up and both products of an all-Q8_0 layer likewise run, until the caller
  * sets by_expert_chunk or gemm_min_tokens, on streaming kernels up to a number of tokens (all-Q8_0: 2 tokens to
- * below 4 picks per expert) and on a 32-column GEMM up to 28 picks per expert.
+ * below 4 picks per expert) and on GEMMs of 32 columns up to 28 picks
+ * per expert and (down) of 64 up to 42 or, large matrices, 56.
  * by_expert_chunk (1..16): token columns per work item of the small-batch by-expert path.
  * gemm_min_tokens (default for an all-MXFP4 layer: 3.5 picks per expert [112 tokens], 7 where
  * n_expert * inter / 256 < 512; MXFP4 gate/up with a Q8_0 down matrix 2 [64], 4 for

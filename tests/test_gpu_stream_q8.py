@@ -1,13 +1,13 @@
 """Q8_0 products on few members per expert against the CPU oracle and the older paths: the streaming kernels
 (16-column items, dsx_stream_kernels.hpp) on rows of an odd and an even number of 128-value groups and in each
-instance by row length (up to 8, 12, 16 and 32 groups), and the 32-column int8 GEMM; items with one column and with
+instance by row length (up to 8, 12, 16 and 32 groups), and the 32- and 64-column int8 GEMMs; items with one column and with
 an empty column group, empty slots, an expert that nearly every token names (several items)."""
 import numpy as np
 import pytest
 
 torch = pytest.importorskip("torch")
 
-from deepstrix_amd.capi import FMT_Q8_0
+from deepstrix_amd.capi import FMT_MXFP4, FMT_Q8_0
 from deepstrix_amd.executor import MoeLayer
 from oracle import ref
 from tests import helpers as H
@@ -60,6 +60,30 @@ def test_q8_0_down_behind_mxfp4_gate_up_matches_the_oracle(monkeypatch, hidden, 
     fmts = dict(sh_gate_fmt=FMT_Q8_0, sh_down_fmt=FMT_Q8_0) if shared == "q8_0" else {}
     s = H.Shape(hidden, inter, 8, 2, down_fmt=FMT_Q8_0, shared=shared != "none", seed=820 + T, **fmts, **ROUTER)
     _run(s, T, T, monkeypatch)
+
+
+@pytest.mark.parametrize("down_fmt", ["all", "down"])
+@pytest.mark.parametrize("T", [112, 129, 167, 168])
+def test_middle_tile_of_the_down_gemm_matches_the_oracle(monkeypatch, down_fmt, T):
+    """28 to 42 picks per expert: down by 64-column items, several of the expert that most tokens name, with one to
+    four column groups; the wide tile's bits."""
+    s = H.Shape(512, 512, 8, 2, FMT_Q8_0 if down_fmt == "all" else FMT_MXFP4, FMT_Q8_0, seed=840 + T, **ROUTER)
+    out, old = _run(s, T, T, monkeypatch)
+    if down_fmt == "all":
+        assert torch.equal(out, old)
+
+
+def test_middle_tile_on_many_workgroups(monkeypatch):
+    """48 picks per expert and enough row tiles for many rounds: the middle tile again, the wide one's bits."""
+    monkeypatch.setattr(MoeLayer, "v3_thresholds_below_experts", None)
+    s = H.Shape(4096, 128, 128, 8, FMT_Q8_0, FMT_Q8_0, shared=True, seed=845, **ROUTER)
+    x, logits, _ = H.host_inputs(s, 768)
+    dw = H.device_weights(s)
+    layer, older = MoeLayer(dw, 768), MoeLayer(dw, 768)
+    older.set_tuning(by_expert_chunk=4)
+    dx, dl = torch.from_numpy(x).cuda(), torch.from_numpy(logits).cuda()
+    out = layer.run(dx, dl).clone()
+    assert torch.equal(out, older.run(dx, dl)) and torch.isfinite(out).all()
 
 
 def test_rows_longer_than_the_registers_take_the_older_paths(monkeypatch):
