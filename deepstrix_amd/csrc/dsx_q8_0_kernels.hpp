@@ -35,8 +35,8 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 // matrix pipe makes for the four of them in one instruction (rounded once, as a vector multiplication would;
 // together with Q8Frag, 512 tokens of 2048 x 1408, 64 experts, wide tile: gate/up 151 -> 134 us, down 93 -> 85).
 // In: the lane's row (dw) or column (xs) n16 = lane % 16 of block lane / 16.  Out: [4 b + q] is row 4 (lane / 16)
-// + q of block b, column n16.  Per value and block the vector pipe is left with the convert and the fused add, two
-// instructions instead of three, and the rows' scales take one register instead of sixteen.
+// + q of block b, column n16.  Per value and block the vector pipe is left with a subtraction (Q8Frag) and the fused add,
+// two instructions instead of three, and the rows' scales take one register instead of sixteen.
 __device__ __forceinline__ v16f q8_0_scales(float dw, float xs) {
     return __builtin_amdgcn_mfma_f32_16x16x1f32(dw, xs, v16f{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f},
                                                 0, 0, 0);
