@@ -334,19 +334,18 @@ int dsx_moe_layer_set_profile_events(dsx_moe_layer *layer, void *gate_up_begin, 
 /* Tuning knobs with no counterpart in the reference; 0 keeps the current value.  The defaults follow
  * from the layer's shape: which path a token count takes depends on the picks an expert receives,
  * T * n_used / n_expert (in brackets: the DeepSeek-V3 shape, 256 experts, top-8).
- * On the engine's rows a layer with MXFP4 gate/up takes the streaming kernels over a range of token counts
- * (dsx_moe_layer_get_streaming) in front of what the values below say -- until the caller sets one of them, to
- * whatever value: by_expert_chunk, gemm_min_tokens and gemm_narrow_members end the streaming of the layer,
- * decode_max_tokens that of an all-MXFP4 layer up to so many tokens.
- * A Q8_0 down matrix behind MXFP4 gate/up and both products of an all-Q8_0 layer likewise run, until the caller
- * sets by_expert_chunk or gemm_min_tokens, on streaming kernels up to a number of tokens (all-Q8_0: 2 tokens to
- * below 4 picks per expert) and on GEMMs of 32 columns up to 28 picks
- * per expert and (down) of 64 up to 42 or, large matrices, 56.
+ * On the engine's rows a layer with MXFP4 gate/up, and an all-Q8_0 layer, takes the streaming kernels over a range of
+ * token counts (dsx_moe_layer_get_streaming) in front of what the values below say -- until the caller sets one of them, to
+ * whatever value: by_expert_chunk, gemm_min_tokens and gemm_narrow_members end the streaming of the layer
+ * (gemm_narrow_members: not of an all-Q8_0 one), decode_max_tokens that of an all-MXFP4 layer up to so many tokens.
+ * Until the caller sets by_expert_chunk or gemm_min_tokens, a Q8_0 down matrix behind MXFP4 gate/up streams where gate/up
+ * does, below gemm_min_tokens, and the int8 GEMMs behind the streaming ranges have 32 columns per work item up to 28 picks
+ * per expert and (down) 64 up to 42, or up to 56 where n_expert * hidden / 64 is at least 24 times the CUs.
  * by_expert_chunk (1..16): token columns per work item of the small-batch by-expert path.
  * gemm_min_tokens (default for an all-MXFP4 layer: 3.5 picks per expert [112 tokens], 7 where
  * n_expert * inter / 256 < 512; MXFP4 gate/up with a Q8_0 down matrix 2 [64], 4 for
- * matrices under 4 M elements; all-Q8_0 layers 1.5; on planar weights right behind the decode path
- * [17]): from this many tokens
+ * matrices under 4 M elements; all-Q8_0 layers 1.5, and there behind the streaming range; on planar weights
+ * right behind the decode path [17]): from this many tokens
  * on, a layer with MXFP4 gate/up runs the grouped-GEMM path (128 token columns per work item,
  * shared expert as an extra group; a Q8_0 down matrix takes the int8 grouped GEMM) and an all-Q8_0
  * layer the int8 grouped GEMMs; an all-MXFP4 layer whose GEMMs use the narrow tile (below)
@@ -362,15 +361,16 @@ int dsx_moe_layer_set_profile_events(dsx_moe_layer *layer, void *gate_up_begin, 
 int dsx_moe_layer_set_tuning(dsx_moe_layer *layer, uint32_t by_expert_chunk, uint32_t gemm_min_tokens,
                              uint32_t decode_max_tokens, uint32_t gemm_narrow_members);
 /* The current values: out[0] by_expert_chunk, [1] gemm_min_tokens, [2] the same for layers whose
- * GEMMs are int8 (all-Q8_0), [3] decode_max_tokens, [4] gemm_narrow_members, [5] the token count
- * from which the one-launch decode path pairs tokens that name one expert (0: never). */
+ * GEMMs are int8 (all-Q8_0: where the streaming range reaches further, they begin behind it), [3]
+ * decode_max_tokens, [4] gemm_narrow_members, [5] the token count from which the one-launch decode path pairs tokens that name one expert (0: never). */
 int dsx_moe_layer_get_tuning(const dsx_moe_layer *layer, uint32_t out[6]);
 /* The token counts that take the streaming kernels: out[0] the first, out[1] the last, both 0 where there are
- * none (planar weights, Q8_0 gate/up, weights that are not 8-byte aligned, rows of more than 7168 values, values
- * set by the caller as above).  By default, all-MXFP4: from 9 tokens at the earliest to below 18 picks per
- * expert, 28 where a matrix has up to 4 M elements [9 .. 575]; beside a Q8_0 down matrix (whose own path is not reported), from 2
- * tokens to below 28 picks per expert [2 .. 895]; few picks in all and matrices under 4 M elements start later.  Where the same
- * token count would take a grouped GEMM otherwise, the device chooses between the two by the picks. */
+ * none (planar weights, Q8_0 gate/up with an MXFP4 down matrix, weights that are not 8-byte aligned, rows of more
+ * than 7168 values -- Q8_0: 4096 -- values set by the caller as above).  By default, all-MXFP4: from 9 tokens at the
+ * earliest to below 18 picks per expert, 28 where a matrix has up to 4 M elements [9 .. 575]; beside a Q8_0 down
+ * matrix the range of gate/up, from 2 tokens to below 28 picks per expert [2 .. 895]; few picks in all and matrices
+ * under 4 M elements start later; all-Q8_0: from 2 tokens to below 4 picks per expert.  Where the same token count
+ * would take a grouped GEMM otherwise, the device chooses between the two by the picks (all-Q8_0: not). */
 int dsx_moe_layer_get_streaming(const dsx_moe_layer *layer, uint32_t out[2]);
 /* Decode path of an all-MXFP4 layer (up to decode_max_tokens tokens, or to where streaming begins); no
  * counterpart in the reference.  fused: 1 = gate/up, mid quantization, down and the slot-order sum in ONE launch

@@ -268,6 +268,18 @@ def test_values_that_the_caller_sets_are_not_passed_over_by_streaming():
     assert _streaming(decode=1, **_V3) == (9, 575)
 
 
+def test_streaming_range_of_an_all_q8_0_layer_is_reported():
+    Q = capi.FMT_Q8_0
+    q8 = dict(hidden=2048, inter=1408, n_expert=64, n_used=6, gate_fmt=Q, up_fmt=Q, down_fmt=Q)
+    first, last = _streaming(**q8)
+    assert first == 2 and 15 <= last < 43   # (below 1.5 and 4 picks per expert)
+    for tuning in [(4, 0, 0, 0), (0, 16, 0, 0)]:
+        assert _streaming(tuning, **q8) == (0, 0)
+    assert _streaming((0, 0, 8, 1), **q8) == (first, last)   # (values of MXFP4 paths)
+    for odd in (dict(gate=0x1004), dict(down=0x1004), dict(up_bpe=12), dict(hidden=4224), dict(inter=4224)):
+        assert _streaming(**{**q8, **odd}) == (0, 0), odd
+
+
 @pytest.mark.parametrize("odd", [dict(gate=0x1004), dict(up=0x1004), dict(down=0x1004), dict(gate_bpe=12), dict(up_bpe=12),
                                  dict(down_bpe=12), dict(sh_gate=0x1004), dict(sh_up=0x1004), dict(sh_down=0x1004),
                                  dict(hidden=7424), dict(inter=7424, sh_inter=7424),
