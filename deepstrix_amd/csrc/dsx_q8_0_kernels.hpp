@@ -22,6 +22,7 @@
 
 #include "../../include/dsx_moe.h"
 #include "dsx_device.hpp"
+#include "dsx_q8_0_rules.hpp"
 #include "dsx_quant.hpp"
 
 namespace dsx {
@@ -543,6 +544,7 @@ struct Q8GemmParams {
     const int32_t *group_count, *group_offset, *members, *work_items, *n_work_items;
     uint32_t n_tokens, n_used, n_expert, n_rows, n_blocks, act_row_bytes, n_row_tiles;
     uint32_t chunk;                // members of a work item, up to the tile's columns
+    StreamChoice choice;           // a streaming launch offers the same product
     float clamp, sh_clamp;
 };
 
@@ -574,6 +576,8 @@ __global__ __launch_bounds__(kQgWaves * 64, COLS > 64 ? 2 : PAIR || COLS > 32 ? 
 
     const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63u;
     const uint32_t g4 = lane >> 4, n16 = lane & 15u;
+
+    if (COLS == kQgColsNarrow && p.choice.offered() && p.choice.streams()) return;   // uniform
 
     // the row tiles of a work item run on one XCD (they share the activations in its L2); the
     // items are dealt to the XCDs like cards, which spreads the wide groups of skewed routing

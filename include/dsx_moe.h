@@ -369,8 +369,9 @@ int dsx_moe_layer_get_tuning(const dsx_moe_layer *layer, uint32_t out[6]);
  * than 7168 values -- Q8_0: 4096 -- values set by the caller as above).  By default, all-MXFP4: from 9 tokens at the
  * earliest to below 18 picks per expert, 28 where a matrix has up to 4 M elements [9 .. 575]; beside a Q8_0 down
  * matrix the range of gate/up, from 2 tokens to below 28 picks per expert [2 .. 895]; few picks in all and matrices
- * under 4 M elements start later; all-Q8_0: from 2 tokens to below 4 picks per expert.  Where the same token count
- * would take a grouped GEMM otherwise, the device chooses between the two by the picks (all-Q8_0: not). */
+ * under 4 M elements start later; all-Q8_0: from 2 tokens to below 4 picks per expert, 1.5 where a matrix has up to
+ * 2 M elements.  Where the same token count would take a grouped GEMM otherwise, the device chooses between the two by
+ * the picks (all-Q8_0: for more than 16 tokens where n_expert * hidden * inter is at least 256 M). */
 int dsx_moe_layer_get_streaming(const dsx_moe_layer *layer, uint32_t out[2]);
 /* Decode path of an all-MXFP4 layer (up to decode_max_tokens tokens, or to where streaming begins); no
  * counterpart in the reference.  fused: 1 = gate/up, mid quantization, down and the slot-order sum in ONE launch

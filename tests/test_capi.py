@@ -280,6 +280,17 @@ def test_streaming_range_of_an_all_q8_0_layer_is_reported():
         assert _streaming(**{**q8, **odd}) == (0, 0), odd
 
 
+@pytest.mark.parametrize("shape,last", [
+    # (hidden, inter, experts, top), last token count: 1.5 picks per expert where the int8 GEMM was measured faster from there on, else 4
+    ((2048, 1408, 64, 6), 42), ((1024, 512, 64, 4), 23), ((1024, 512, 128, 8), 23), ((512, 2048, 64, 4), 23),
+    ((512, 4096, 32, 4), 11), ((1024, 512, 32, 4), 11), ((2048, 512, 32, 4), 11), ((2048, 768, 128, 8), 23),
+    ((4096, 1024, 32, 4), 31), ((4096, 1024, 128, 8), 63), ((4096, 1536, 128, 8), 63), ((2560, 1792, 96, 4), 95), ((3072, 2048, 64, 4), 63)])
+def test_all_q8_0_streaming_ends_where_it_is_slower(shape, last):
+    Q = capi.FMT_Q8_0
+    got = _streaming(**dict(zip(("hidden", "inter", "n_expert", "n_used"), shape)), gate_fmt=Q, up_fmt=Q, down_fmt=Q)
+    assert got == (2, last)
+
+
 @pytest.mark.parametrize("odd", [dict(gate=0x1004), dict(up=0x1004), dict(down=0x1004), dict(gate_bpe=12), dict(up_bpe=12),
                                  dict(down_bpe=12), dict(sh_gate=0x1004), dict(sh_up=0x1004), dict(sh_down=0x1004),
                                  dict(hidden=7424), dict(inter=7424, sh_inter=7424),

@@ -17,11 +17,12 @@ pytestmark = pytest.mark.gpu
 ROUTER = dict(router_mode=1, route_scale=2.5, bias_sigma=0.01, clamp=10.0)
 
 
-def _run(s, T, seed, monkeypatch):
+def _run(s, T, seed, monkeypatch, named=None):
+    """Picks on the first `named` experts (None: all).  Also returns the streaming range."""
     monkeypatch.setattr(MoeLayer, "v3_thresholds_below_experts", None)   # the library's own thresholds
     x, _, _ = H.host_inputs(s, T)
     rng = np.random.default_rng(seed)
-    sel = np.stack([rng.permutation(s.n_expert)[:2] for _ in range(T)]).astype(np.int32)
+    sel = np.stack([rng.permutation(named or s.n_expert)[:2] for _ in range(T)]).astype(np.int32)
     few = rng.random(T) < 0.6                       # most tokens name expert 3: several items
     sel[few, 0] = np.where(sel[few, 1] == 3, sel[few, 0], 3)
     sel[T // 2, 1] = -1                             # an empty slot
@@ -35,22 +36,91 @@ def _run(s, T, seed, monkeypatch):
     old = older.run(dx, None, selected_in=ds, weights_in=dwt)
     torch.cuda.synchronize()
     assert torch.equal(out, again)
-    want = ref.moe_forward(H.host_weights(s), x, sel, w)
+    hw = H.host_weights(s, experts=range(named or s.n_expert))
+    want = ref.moe_forward(hw, x, sel, w)
     # the dots are exact: other orders of the f32 sums, and a mid value at a rounding boundary that takes the
     # neighbouring int8 step (fitted to a column of a down matrix)
-    H.assert_parity_up_to_rounding_steps(out.cpu().numpy(), want, H.host_weights(s), sel, f"{s.hidden} x {s.inter} T={T}")
-    return out, old
+    H.assert_parity_up_to_rounding_steps(out.cpu().numpy(), want, hw, sel, f"{s.hidden} x {s.inter} T={T}")
+    return out, old, layer.streaming()
 
 
 # (hidden, inter): gate/up rows of hidden / 128 groups, down rows of inter / 128
 @pytest.mark.parametrize("hidden,inter", [(128, 256), (384, 1152), (1024, 640), (1152, 128), (2048, 1408), (2304, 2176), (4096, 512), (512, 4096)])
-@pytest.mark.parametrize("T", [2, 15, 16, 60, 111])
+@pytest.mark.parametrize("T", [2, 5, 15, 16, 60, 111])
 def test_all_q8_0_layer_matches_the_oracle(monkeypatch, hidden, inter, T):
-    """2 and 15 tokens: the streaming kernels; from 16 (4 picks per expert) to 111: the narrow GEMM, which has the
-    bits of the wide one."""
+    """2 and 5 tokens (1.25 picks per expert): the streaming kernels, which serve matrices over 2 M elements at 15 as
+    well; behind them, to 111, the narrow GEMM, which has the bits of the wide one."""
     s = H.Shape(hidden, inter, 8, 2, FMT_Q8_0, FMT_Q8_0, shared=hidden != 1024, seed=800, **ROUTER)
-    out, old = _run(s, T, T, monkeypatch)
-    assert torch.equal(out, old) == (T >= 16)
+    out, old, streaming = _run(s, T, T, monkeypatch)
+    assert streaming == (2, 15 if hidden * inter > 2 << 20 else 5)
+    assert torch.equal(out, old) == (T > streaming[1])
+
+
+@pytest.mark.parametrize("hidden,inter", [(256, 1280), (384, 1536), (640, 1664), (512, 1792), (1280, 2048), (4096, 384)])
+@pytest.mark.parametrize("T", [17, 23])
+def test_all_q8_0_streaming_with_several_items_of_an_expert(monkeypatch, hidden, inter, T):
+    """Under 1.5 picks per expert on 32 experts, but most tokens name one and all of them the shared one: their second
+    items begin at member 16 and have one to seven columns.  Down rows of 10 and 12 groups (four waves, padded rows), 13, 14 and 16 (eight
+    waves, of which some are a group short)."""
+    s = H.Shape(hidden, inter, 32, 2, FMT_Q8_0, FMT_Q8_0, shared=inter != 1664, seed=810, **ROUTER)
+    out, old, streaming = _run(s, T, T, monkeypatch, named=6)
+    assert streaming == (2, 63 if hidden * inter > 2 << 20 else 23)
+    assert H.max_rel(out.cpu().numpy(), old.cpu().numpy()) < 1e-3
+
+
+def _choice_case(T):
+    """64 experts of 2048 x 2048, top-4: streaming to 63 tokens, from 24 on beside the narrow GEMM."""
+    s = H.Shape(2048, 2048, 64, 4, FMT_Q8_0, FMT_Q8_0, seed=870, **ROUTER)
+    dw = H.device_weights(s)
+    layer, gemm = MoeLayer(dw, T), MoeLayer(dw, T)
+    gemm.set_tuning(gemm_min_tokens=1)   # the int8 GEMM alone
+    assert layer.streaming() == (2, 63) and gemm.streaming() == (0, 0)
+    rng = np.random.default_rng(T)
+    sets = {}
+    for kind, named in (("few", 5), ("spread", 64)):
+        sel = np.stack([rng.choice(named, 4, replace=False) for _ in range(T)]).astype(np.int32)
+        sets[kind] = (sel, rng.uniform(0.05, 0.6, sel.shape).astype(np.float32))
+    return s, dw, layer, gemm, torch.from_numpy(H.host_inputs(s, T)[0]).cuda(), sets
+
+
+@pytest.mark.parametrize("T", [24, 33, 63])
+def test_all_q8_0_picks_on_a_few_experts_take_the_gemm(T):
+    """From 1.5 picks per expert on the device chooses: picks on a few experts go to the int8 GEMM, whose bits a layer
+    that only has it reproduces, spread ones to the streaming kernels (another order of the sums)."""
+    s, dw, layer, gemm, x, sets = _choice_case(T)
+    for kind in ("few", "spread", "few"):   # one workspace: the counts of one call say nothing to the next
+        sel, w = sets[kind]
+        run = lambda l: l.run(x, None, selected_in=torch.from_numpy(sel).cuda(), weights_in=torch.from_numpy(w).cuda()).cpu().numpy()
+        out, want = run(layer), run(gemm)
+        assert np.array_equal(out, want) == (kind == "few"), kind
+        assert H.max_rel(out, want) < 1e-3
+        n = T if kind == "few" else 3   # (spread: the experts of three tokens are enough on the host)
+        hw = H.host_weights_from_device(s, dw, experts=np.unique(sel[-n:]))
+        H.assert_parity_up_to_rounding_steps(out[-n:], ref.moe_forward(hw, x.cpu().numpy()[-n:], sel[-n:], w[-n:]), hw, sel[-n:], kind)
+
+
+def test_a_captured_all_q8_0_pass_chooses_at_every_replay():
+    s, dw, layer, gemm, x, sets = _choice_case(40)
+    sets = [tuple(torch.from_numpy(a).cuda() for a in sets[kind]) for kind in ("few", "spread")]
+    eager = [layer.run(x, None, selected_in=sel, weights_in=w).clone() for sel, w in sets]
+    sel, w = (t.clone() for t in sets[0])
+    out = torch.empty_like(x)
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        layer.run(x, None, out=out, selected_in=sel, weights_in=w)
+        side.synchronize()
+        with torch.cuda.graph(graph, stream=side):
+            layer.run(x, None, out=out, selected_in=sel, weights_in=w)
+    torch.cuda.synchronize()
+    for rep in range(4):
+        sel.copy_(sets[rep % 2][0])
+        w.copy_(sets[rep % 2][1])
+        out.fill_(float(rep))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager[rep % 2]), rep
 
 
 @pytest.mark.parametrize("hidden,inter,shared", [(512, 256, "none"), (1280, 768, "same"), (1280, 768, "q8_0"),
@@ -68,7 +138,7 @@ def test_middle_tile_of_the_down_gemm_matches_the_oracle(monkeypatch, down_fmt, 
     """28 to 42 picks per expert: down by 64-column items, several of the expert that most tokens name, with one to
     four column groups; the wide tile's bits."""
     s = H.Shape(512, 512, 8, 2, FMT_Q8_0 if down_fmt == "all" else FMT_MXFP4, FMT_Q8_0, seed=840 + T, **ROUTER)
-    out, old = _run(s, T, T, monkeypatch)
+    out, old, _ = _run(s, T, T, monkeypatch)
     if down_fmt == "all":
         assert torch.equal(out, old)
 
@@ -89,7 +159,7 @@ def test_middle_tile_on_many_workgroups(monkeypatch):
 def test_rows_longer_than_the_registers_take_the_older_paths(monkeypatch):
     """Gate/up rows of 33 groups: the older paths' bits."""
     s = H.Shape(4224, 256, 8, 2, FMT_Q8_0, FMT_Q8_0, shared=False, seed=850, **ROUTER)
-    out, old = _run(s, 15, 5, monkeypatch)
+    out, old, _ = _run(s, 15, 5, monkeypatch)
     assert torch.equal(out, old)
 
 
