@@ -529,10 +529,6 @@ inline int q8_0_down_by_expert(hipStream_t st, float *partials, const uint8_t *d
 // registers).  Gate/up of 64 columns would need 54 KB and stay at two per CU.
 // ---------------------------------------------------------------------------------------
 constexpr int kQgWaves = 4;
-constexpr int kQgCols = 128;
-constexpr int kQgColsMiddle = 64;   // down only
-constexpr int kQgColsNarrow = 32;
-constexpr int kQgRows = 64;
 
 struct Q8GemmParams {
     float *out;                    // PAIR: f32 mid [dest rows, n_rows]; else partials [dest rows, n_rows]

@@ -8,6 +8,8 @@
 namespace dsx {
 
 constexpr uint32_t kQ8StreamMembers = 16;   // members of a streaming work item (dsx_stream_kernels.hpp)
+// columns of the int8 GEMM's tiles (k_q8_0_gemm), rows of them all
+constexpr uint32_t kQgCols = 128, kQgColsMiddle = 64 /* down only */, kQgColsNarrow = 32, kQgRows = 64;
 
 struct Q8Shape {
     uint32_t hidden, inter, n_expert, n_used;
@@ -36,6 +38,30 @@ inline bool q8_all_streams(const Q8Shape &s, uint32_t T) {
 // ones (2048 x 1408: 24 tokens 131 / 136, 40: 143 / 149) than they do on the same ones (old / streaming 24: 52 / 53, 32: 53 / 55, 40: 60 / 61).
 inline bool q8_stream_choice(const Q8Shape &s, uint32_t T) {
     return T > kQ8StreamMembers && !s.picks_below_halves(T, 3u) && s.n_expert * s.elements() >= (256ull << 20);
+}
+
+// Columns per work item of the int8 GEMMs of T tokens on n_cu CUs.
+//
+// Narrow: few members per expert.  An item reads its rows of the weights whatever its members, so that an expert which every token
+// names is read T / 32 times: over 256 tokens the middle tile (64: down in 64 columns, gate/up in 128) is no slower on spread picks and much
+// faster on the same ones (all-Q8_0 layer, spread / same picks, old; narrow; middle: 7168 x 2048, 256 experts, top-8: 256 tokens
+// 2546 / 609; 2397 / 599; 2385 / 471, 512: 2753 / 937; 2613 / 1180; 2564 / 769, 768: 3271 / 1283; 2884 / 1780; 2847 / 1138; 5120 x 1536, 160
+// experts, top-6: 512: 1027 / 446; 987 / 480; 946 / 360; 3072 x 2048, 64 experts, top-4: 384: 360 / 194; 354 / 213; 338 / 160; MXFP4 gate/up, 7168 x
+// 2048: 512: 1882 / -; 1747 / 612; 1746 / 533).  Up to 2 M elements it stays the faster one (2048 x 768, 128 experts, top-8: 384 tokens 217 /
+// 127; 190 / 98; 194 / 107).  It ends at 28 picks per expert (4096 x 1536, 128 experts, top-8, 24: narrow 656 / middle 633, 32: 773 / 679; 2048 x
+// 1408, 64 experts, top-6, 24: 185 / 184, 36: 238 / 202), at 42 on up to 16 experts whose down product makes less than a round of three
+// workgroups per CU, of which an item more or less per expert is a large part (4096 x 14336, 8 experts, top-2, 32 picks: old 705, narrow 584, middle
+// 650, wide 610; MXFP4 gate/up: 528, 482, 551, 503; but 1024 x 2048, 32 experts, top-4, 32: 110, 92, 88; 512 x 2048, 64 experts, 40: 122, 111, 96).
+//
+// Middle: to 42 picks per expert, 56 where down makes many rounds (us per layer, wide / middle: 7168 x 2048, 256 experts, MXFP4 gate/up,
+// 1000 tokens [31 picks per expert] 2349 / 2143, 1700 [53] 2723 / 2504, 2100 [66: most experts make two items] 2906 / 2999; all-Q8_0 2048 x 1408,
+// 64 experts: 300 tokens [28] 196 / 191, 420 [39] 220 / 214, 512 [48] 234 / 239, 700 [66] 265 / 277: its 2048 workgroups are then four full
+// rounds of the wide tile's two per CU, but 2.7 of the middle one's three; 4096 x 1536, 128 experts, 48: 830 / 815).
+inline uint32_t q8_gemm_columns(const Q8Shape &s, uint32_t T, uint32_t n_cu) {
+    const uint64_t workgroups = (uint64_t)s.n_expert * (s.hidden / kQgRows);   // down's, a work item per expert
+    const uint32_t narrow = s.n_expert <= 16u && workgroups < 3u * n_cu ? 84u : 56u;
+    if ((T <= 256u || s.elements() <= (2ull << 20)) && s.picks_below_halves(T, narrow)) return kQgColsNarrow;
+    return s.picks_below_halves(T, workgroups >= 24u * n_cu ? 112u : 84u) ? kQgColsMiddle : kQgCols;
 }
 
 }  // namespace dsx

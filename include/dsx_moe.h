@@ -340,7 +340,8 @@ int dsx_moe_layer_set_profile_events(dsx_moe_layer *layer, void *gate_up_begin, 
  * (gemm_narrow_members: not of an all-Q8_0 one), decode_max_tokens that of an all-MXFP4 layer up to so many tokens.
  * Until the caller sets by_expert_chunk or gemm_min_tokens, a Q8_0 down matrix behind MXFP4 gate/up streams where gate/up
  * does, below gemm_min_tokens, and the int8 GEMMs behind the streaming ranges have 32 columns per work item up to 28 picks
- * per expert and (down) 64 up to 42, or up to 56 where n_expert * hidden / 64 is at least 24 times the CUs.
+ * per expert and 256 tokens (any number where a matrix has up to 2 M elements), and (down) 64 up to 42, or up to 56 where
+ * n_expert * hidden / 64 is at least 24 times the CUs; on up to 16 experts, where it is below 3 times the CUs, 32 up to 42.
  * by_expert_chunk (1..16): token columns per work item of the small-batch by-expert path.
  * gemm_min_tokens (default for an all-MXFP4 layer: 3.5 picks per expert [112 tokens], 7 where
  * n_expert * inter / 256 < 512; MXFP4 gate/up with a Q8_0 down matrix 2 [64], 4 for

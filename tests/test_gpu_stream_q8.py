@@ -135,9 +135,10 @@ def test_q8_0_down_behind_mxfp4_gate_up_matches_the_oracle(monkeypatch, hidden, 
 @pytest.mark.parametrize("down_fmt", ["all", "down"])
 @pytest.mark.parametrize("T", [112, 129, 167, 168])
 def test_middle_tile_of_the_down_gemm_matches_the_oracle(monkeypatch, down_fmt, T):
-    """28 to 42 picks per expert: down by 64-column items, several of the expert that most tokens name, with one to
-    four column groups; the wide tile's bits."""
-    s = H.Shape(512, 512, 8, 2, FMT_Q8_0 if down_fmt == "all" else FMT_MXFP4, FMT_Q8_0, seed=840 + T, **ROUTER)
+    """28 to 42 picks per expert on a layer whose down product makes a round of workgroups (fewer
+    take the narrow tile): down by 64-column items, several of the expert that most tokens name, with one to four column
+    groups; the wide tile's bits."""
+    s = H.Shape(6144, 256, 8, 2, FMT_Q8_0 if down_fmt == "all" else FMT_MXFP4, FMT_Q8_0, seed=840 + T, **ROUTER)
     out, old, _ = _run(s, T, T, monkeypatch)
     if down_fmt == "all":
         assert torch.equal(out, old)
