@@ -64,4 +64,17 @@ inline uint32_t q8_gemm_columns(const Q8Shape &s, uint32_t T, uint32_t n_cu) {
     return s.picks_below_halves(T, workgroups >= 24u * n_cu ? 112u : 84u) ? kQgColsMiddle : kQgCols;
 }
 
+// Columns per work item of a dense Q8_0 expert of b tokens (dsx_dense_ffn; both products, one list): 32 where the wide tile would
+// leave workgroup slots empty in gate/up (two per CU) -- over 128 tokens unless the items, each of which reads gate and up whole,
+// come to about a gigabyte of reads, in brackets (us, wide / narrow: 7168 x 2048: 96 tokens 162 / 84, 512 [0.5] 203 / 129, 768 [0.75] 203 / 194,
+// 1000 [1.0] 204 / 269, 1900 [1.9] 328 / 514; 7168 x 3072: 512 [0.75] 297 / 197, 640 [0.94] 299 / 291, 1000 [1.5] 301 / 401; 5120 x 1536: 1500
+// [0.79] 218 / 194, 1900 [1.0] 222 / 256; 7168 x 512: 3000 [0.73] 204 / 181, 4096 [1.0] 230 / 238; 2048 x 1408: 1900 [0.37] 98 / 94; 7168 x 18432:
+// 128 [1.1] 1366 / 624).
+inline uint32_t q8_dense_columns(uint32_t hidden, uint32_t inter, uint32_t b, uint32_t n_cu) {
+    const uint64_t wide = (uint64_t)((b + kQgCols - 1u) / kQgCols) * (inter / kQgRows);
+    const uint64_t item = 2u * (uint64_t)hidden * inter / 32u * 34u;
+    const bool few_reads = b <= kQgCols || (b + kQgColsNarrow - 1u) / kQgColsNarrow * item < 950000000u;
+    return wide < 2u * n_cu && few_reads ? kQgColsNarrow : kQgCols;
+}
+
 }  // namespace dsx

@@ -276,3 +276,29 @@ def test_config5_full_size_T512_adversarial_and_uniform_routing():
         # the streaming kernel (items of 32 and of 16 columns): the same integer dots summed in a different f32 order, so a mid value next to a rounding
         # boundary of the Q8_0 quantization may move one int8 step
         assert H.max_rel(out_h[sub], got.cpu().numpy()) < 1e-3, name
+
+
+@pytest.mark.parametrize("hidden,inter,b", [(256, 4096, 96), (256, 4096, 129), (256, 4096, 896), (256, 4096, 1000), (1024, 128, 200), (128, 1408, 3000)])
+def test_dense_q8_0_expert_of_many_tokens(hidden, inter, b):
+    """The int8 GEMMs of a dense expert in 32 and, from 512 wide workgroups on (1000 tokens at inter 4096, 3000 at 1408), in
+    128 columns: the oracle's values, and a token's bits do not depend on the tile (its half of the batch takes the narrow one)."""
+    s = H.Shape(hidden, inter, 1, 1, FMT_Q8_0, FMT_Q8_0, shared=False, clamp=5.0, seed=77)
+    w = H.host_weights(s)
+    x = synth.normal_host(9, synth.T_X, b * hidden).reshape(b, hidden)
+    gate, up, down = dev(w.gate), dev(w.up), dev(w.down)
+
+    def run(xs):
+        n = xs.shape[0]
+        out = torch.empty((n, hidden), dtype=torch.float32, device="cuda")
+        scratch = torch.empty(dispatch.dense_ffn_scratch_bytes(n, hidden, inter), dtype=torch.uint8, device="cuda")
+        dispatch.dense_ffn(FMT_Q8_0, FMT_Q8_0, FMT_Q8_0, out, gate, up, down, dev(xs), n, hidden, inter, s.clamp, scratch)
+        torch.cuda.synchronize()
+        return out.cpu().numpy()
+
+    out = run(x)
+    if b >= 256:
+        assert np.array_equal(out[: b // 2], run(x[: b // 2]))
+    rows = np.r_[0:24, b - 24:b]   # (the first and the ragged last items on the host)
+    sel = np.zeros((rows.size, 1), np.int32)
+    want = ref.moe_forward(w, x[rows], sel, np.ones((rows.size, 1), np.float32))
+    H.assert_parity_up_to_rounding_steps(out[rows], want, w, sel, f"dense {hidden} x {inter} b={b}")

@@ -32,3 +32,15 @@ def ask(lines):
     ((1024, 2048, 32, 4), {192: 32, 256: 64})])
 def test_columns_of_the_int8_gemm(shape, columns):
     assert dict(zip(columns, ask([("gemm", *shape, T, CUS) for T in columns]))) == columns
+
+
+@pytest.mark.parametrize("shape,columns", [
+    ((7168, 2048), {96: 32, 768: 32, 1000: 128, 1900: 128, 2000: 128}),
+    ((7168, 3072), {512: 32, 640: 32, 1000: 128}),
+    ((5120, 1536), {1500: 32, 1900: 128}),
+    ((2048, 1408), {96: 32, 1900: 32, 4096: 128}),
+    ((7168, 512), {3000: 32, 4096: 128}),
+    ((7168, 18432), {96: 32, 128: 32, 512: 128}),
+    ((128, 128), {65535: 128}), ((65536, 128), {129: 32, 65535: 128})])   # (no overflow at the ends of the range)
+def test_columns_of_a_dense_expert(shape, columns):
+    assert dict(zip(columns, ask([("dense", *shape, 0, 0, b, CUS) for b in columns]))) == columns
