@@ -1,16 +1,19 @@
 """Q8_0 products on few members per expert against the CPU oracle and the older paths: the streaming kernels
 (16-column items, dsx_stream_kernels.hpp) on rows of an odd and an even number of 128-value groups and in each
-instance by row length (up to 8, 12, 16 and 32 groups), and the 32- and 64-column int8 GEMMs; items with one column and with
-an empty column group, empty slots, an expert that nearly every token names (several items)."""
+instance by row length (up to 8, 12, 16 and 32 groups), with second items of an expert, beside the GEMM with the device's choice, in
+captures, blocks and the hyper-connection combine; the 32- and 64-column int8 GEMMs with several items of an expert that nearly
+every token names; items with one column and with an empty column group, empty slots."""
 import numpy as np
 import pytest
 
 torch = pytest.importorskip("torch")
 
 from deepstrix_amd.capi import FMT_MXFP4, FMT_Q8_0
-from deepstrix_amd.executor import MoeLayer
+from deepstrix_amd.executor import MoeChain, MoeLayer
 from oracle import ref
 from tests import helpers as H
+from tests.test_gpu_chain import layer_shapes, verify_chain_stepwise
+from tests.test_gpu_hc_post import _layer_case
 
 pytestmark = pytest.mark.gpu
 
@@ -130,6 +133,48 @@ def test_q8_0_down_behind_mxfp4_gate_up_matches_the_oracle(monkeypatch, hidden, 
     fmts = dict(sh_gate_fmt=FMT_Q8_0, sh_down_fmt=FMT_Q8_0) if shared == "q8_0" else {}
     s = H.Shape(hidden, inter, 8, 2, down_fmt=FMT_Q8_0, shared=shared != "none", seed=820 + T, **fmts, **ROUTER)
     _run(s, T, T, monkeypatch)
+
+
+@pytest.mark.parametrize("hidden,inter,shared", [(4096, 1280, "none"), (3072, 1536, "same"), (4096, 1792, "q8_0"), (2048, 2048, "same")])
+@pytest.mark.parametrize("T", [2, 5, 7])
+def test_q8_0_down_streams_behind_mxfp4_gate_up(monkeypatch, hidden, inter, shared, T):
+    """Below two picks per expert down takes the streaming kernel as well: rows of 10 and 12 groups (four waves), 14 and 16."""
+    fmts = dict(sh_gate_fmt=FMT_Q8_0, sh_down_fmt=FMT_Q8_0) if shared == "q8_0" else {}
+    s = H.Shape(hidden, inter, 8, 2, down_fmt=FMT_Q8_0, shared=shared != "none", seed=830 + T, **fmts, **ROUTER)
+    monkeypatch.setattr(MoeLayer, "v3_thresholds_below_experts", None)
+    layer = MoeLayer(H.device_weights(s), 8)
+    assert layer.streaming()[0] == 2 and layer.tuning()["gemm_q8_min_tokens"] == 8
+    _run(s, T, T, monkeypatch)
+
+
+@pytest.mark.parametrize("T", [3, 15])
+def test_a_stack_of_all_q8_0_streaming_blocks(monkeypatch, T):
+    """h += layer(RMSNorm(h)) in a chain: each block against the oracle, replays of a capture against eager steps."""
+    monkeypatch.setattr(MoeLayer, "v3_thresholds_below_experts", None)
+    shapes = layer_shapes(H.Shape(2304, 1024, 8, 2, FMT_Q8_0, FMT_Q8_0, seed=880, **ROUTER), 2)
+    chain = MoeChain([H.device_weights(s, block=True) for s in shapes], T)
+    for layer in chain.layers:
+        assert layer.streaming() == (2, 15)
+    rng = np.random.default_rng(T)
+    chain.capture(T)
+    for step in range(3):
+        h = rng.normal(0, 1, (T, 2304)).astype(np.float32)
+        eager = chain.step(torch.from_numpy(h).cuda()).clone()
+        torch.cuda.synchronize()
+        replayed = chain.replay(torch.from_numpy(h).cuda()).clone()
+        torch.cuda.synchronize()
+        assert torch.equal(eager, replayed), step
+    final = verify_chain_stepwise(chain, shapes, h, 3 * 2e-3, min_checked=(9 * 2 * T) // 10)   # (the bar of the other chains)
+    assert np.array_equal(final, eager.cpu().numpy())
+
+
+@pytest.mark.parametrize("T", [2, 15])
+def test_hyper_connection_combine_behind_all_q8_0_streaming(monkeypatch, T):
+    monkeypatch.setattr(MoeLayer, "v3_thresholds_below_experts", None)
+    s = H.Shape(2304, 1024, 8, 2, FMT_Q8_0, FMT_Q8_0, seed=885, **ROUTER)
+    layer = MoeLayer(H.device_weights(s), T)
+    assert layer.streaming() == (2, 15)
+    _layer_case(s, layer, T)
 
 
 @pytest.mark.parametrize("down_fmt", ["all", "down"])
