@@ -89,11 +89,15 @@ int with_stream_kernel(uint32_t n_sb, F &&f) {
     return f(k_mxfp4_stream<PAIR, 7, NCG, 1>, 1u, 8u);
 }
 
-// The same for k_q8_0_stream (16 columns) and rows of n_sb groups of four blocks: f(kernel, row tiles per stage, waves).
-// Workgroups of four waves, two per CU, which overlap one's sums with the other's products, where half of the
-// LDS holds three stages (2048 x 1408, 64 experts, down, 4 / 40 tokens: 19 / 45 us against 22 / 48 with eight
-// waves; 7168 x 2048, two stages: 16 / 100 tokens 308 / 733 against 298 / 701) and for gate/up, whose SwiGLU takes
-// longer (2048 x 1408: 30 / 80 us against 34 / 79).
+// The same for k_q8_0_stream (16 columns) and rows of n_sb groups of four blocks: f(kernel, row tiles per stage,
+// waves). Workgroups of four waves, two per CU, which overlap one's sums with the other's products, for gate/up, whose
+// SwiGLU takes longer (2048 x 1408, 64 experts, 4 / 40 tokens: 30 / 80 us against 34 / 79 with eight waves), and for
+// down up to 12 groups (four / eight waves, us: 2048 x 1408, 11 groups: 4 tokens 19 / 22, 40: 45 / 48; layers with 12
+// groups, 4096 x 1536, 128 experts, all-Q8_0: 2 tokens 87.3 / 89.8, 4: 134.9 / 136.5, 16: 325 / 325, 48: 472 / 467;
+// behind MXFP4 gate/up: 2: 66.8 / 70.5, 24: 279.9 / 277.6).  At 13 to 16 groups the two are as close (layers, 2560 x
+// 1792, 14 groups: 4 tokens 69.3 / 71.7, 16: 157 / 158, 48: 269 / 267; 3072 x 2048, 16 groups: 4: 81.6 / 83.6, 48: 263
+// / 261), 7168 x 2048 down alone slower with four (16 / 100 tokens 308 / 733 against 298 / 701).  Rows of up to 8
+// groups are two row tiles per stage with eight waves.
 template <bool PAIR, typename F>
 int with_q8_stream_kernel(uint32_t n_sb, F &&f) {
     if (n_sb <= 8u) return f(k_q8_0_stream<PAIR, 8, 1, 2>, 2u, 8u);
@@ -246,7 +250,8 @@ int launch_gemm(hipStream_t st, const GemmParams &p, uint32_t max_wi, bool plana
     return launched(PAIR ? "gate_up gemm" : "down gemm");
 }
 
-// Streaming launch for groups of few members (items of up to 16 ncg members), one workgroup per CU.
+// Streaming launch for groups of few members (items of up to 16 ncg members): as many workgroups as are resident, one
+// of eight waves or two of four per CU.
 // q8: Q8_0 weights and activation rows.
 template <bool PAIR>
 int launch_stream(hipStream_t st, StreamParams p, uint32_t ncg, bool q8 = false) {

@@ -517,14 +517,16 @@ inline int q8_0_down_by_expert(hipStream_t st, float *partials, const uint8_t *d
 // activations (and their scales) shared; 16-byte units are XOR-swizzled with the row so
 // that the 8-byte operand reads spread over the banks.  The extra expert (index n_expert,
 // slot n_used) like in the MXFP4 GEMM.
-// The narrow tile is for up to 28 picks per expert, where the kernel only streams weights: its workgroups need a
+// Which tile a layer takes: q8_gemm_columns (dsx_q8_0_rules.hpp).
+// The narrow tile is for few picks per expert, where the kernel only streams weights: its workgroups need a
 // third to two thirds of the LDS, so that three (gate/up) or four (down) of a CU wait for their chunks side by side
 // where the wide tile has two.  A value's terms and their order are those of the wide tile: the same bits.  Measured, us wide /
-// narrow: down 7168 x 2048, 256 experts, top-8: 100 tokens 871 / 681 (5.7 TB/s), 512: 1040 / 870, 850: 1163 / 990; 2048 x
-// 1408, 64 experts, top-6, both products, 64 tokens: 157 / 142, 200: 166 / 152, 300: 183 / 186.  With few columns
-// per expert it is bound by the weight stream; with 48 (512 tokens) the vector pipe is 54 % busy, the matrix pipe 22 %,
-// and the workgroups' last round is part empty.
-// The middle tile is down's for the picks behind that, while most experts still make one item of 64: three workgroups per
+// narrow: down 7168 x 2048, 256 experts, top-8: 100 tokens 871 / 681 (5.7 TB/s); 2048 x 1408, 64 experts, top-6, both
+// products, 64 tokens: 157 / 142, 200: 166 / 152.  There (19 picks per expert) the vector pipe is 31 % busy in gate/up and 25 % in
+// down, the matrix pipe 14 and 10 %.
+// The wide tile with 48 picks per expert (the same layer, 512 tokens): 54 % and 22 % busy in gate/up, 41 % and 16 % in
+// down, whose last round of workgroups (4.25 rounds) is part empty.
+// The middle tile is down's for the picks between, while most experts still make one item of 64: three workgroups per
 // CU for the wide tile's two (7168 x 2048, 256 experts, 1000 tokens: the layer 2349 -> 2143 us; four per CU spilled 24
 // registers).  Gate/up of 64 columns would need 54 KB and stay at two per CU.
 // ---------------------------------------------------------------------------------------

@@ -2,13 +2,13 @@
 // weights, and they read them as whole row tiles.
 //
 // A tile of 16 of the engine's rows is one contiguous stretch of 16 n_sb 136 bytes (a super-block of 256 MXFP4
-// values, four blocks of 32 Q8_0 values).  A workgroup (8 waves, one per CU: it takes nearly all of the LDS) streams such
-// stretches through a ring of LDS stages with LDS-direct loads, so that every cache line is requested
+// values, four blocks of 32 Q8_0 values).  A workgroup (8 waves, one per CU: it takes nearly all of the LDS; for some Q8_0
+// rows 4 waves, two per CU: with_q8_stream_kernel) streams such stretches through a ring of LDS stages with LDS-direct loads, so that every cache line is requested
 // once and 60-120 KB per CU are under way at any time; what differs from the grouped GEMM
 // (dsx_gemm_kernels.hpp), which walks 512 rows in step and asks for 136 bytes of each at a time (two
 // lines for 1.06 lines' worth, and every step waits for its own loads).
 //
-// The roles of the operands are swapped for that: the columns stay, the weights pass.  The eight waves
+// The roles of the operands are swapped for that: the columns stay, the weights pass.  MXFP4: the eight waves
 // split k by half super-blocks -- wave w takes half w % 2 of super-blocks w / 2, w / 2 + 4, .. -- and
 // hold the columns' operands of their share in registers for as long as the work item (expert, up to
 // 16 NCG members) lasts.  Of a tile they each multiply their share, and the eight partial sums per
@@ -17,8 +17,8 @@
 // The work, (items) x (row tiles), is cut into one contiguous range per workgroup, so that a workgroup
 // changes its item only once or twice.
 //
-// Q8_0: wave w takes every eighth (fourth) group of four blocks.  Against the by-expert kernels and the 128-column int8
-// GEMM, us: 2048 x 1408, 64 experts, top-6, gate/up + down: 4 tokens 35 + 26 / 30 + 19, 16: 70 + 49 / 63 + 36; 7168
+// Q8_0: of W waves, wave w takes every W-th group of four blocks.  Against the by-expert kernels and the 128-column int8
+// GEMM (whole layers: dsx_q8_0_rules.hpp), us: 2048 x 1408, 64 experts, top-6, gate/up + down: 4 tokens 35 + 26 / 30 + 19, 16: 70 + 49 / 63 + 36; 7168
 // x 2048, 256 experts, down, 16 tokens: 413 / 298.  32 and 64 columns per item lost to the int8 GEMM's narrow tile (512
 // tokens, down 7168 x 2048, 32 columns: 915 / 870): a stage's products, sums and two barriers then outlast its loads.
 //
@@ -28,7 +28,7 @@
 // taken: the last tenth of the work claimed in chunks through a counter (64 tokens 4 % faster, 200 tokens 2
 // to 5 % slower: every chunk loads an item's columns again); a stage read into registers and its place
 // requested before the products (16 columns: no change; 32: the registers spill).  Scalar registers run out in
-// the instances for long rows (54 to 61 of them live in lanes of a vector register in gate/up, 33 to 36 in down;
+// the instances for long rows (45 to 53 of them live in lanes of a vector register in gate/up, 32 to 36 in down;
 // no memory); what that costs was not measured.
 //
 // A shared expert of another format runs beside these on the layer's side stream although they take nearly all
@@ -269,7 +269,7 @@ __device__ __forceinline__ void stream_body(const StreamParams &p) {
 
     // ---- requesting stages ----------------------------------------------------------------------
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)smem) + kStages;
-    const uint32_t n_loads = PAIR && !kTurns ? 2u * p.loads : p.loads;   // of a stage; the wave's: wave, wave + 8, ..
+    const uint32_t n_loads = PAIR && !kTurns ? 2u * p.loads : p.loads;   // of a stage; the wave's: wave, wave + kW, ..
     const uint32_t my_loads = (n_loads + (uint32_t)kW - 1u - wave) / (uint32_t)kW;
     const uint32_t unit_bytes = kTiles * 16u * n_sb * (uint32_t)kSuperBytes;
     const uint32_t last_piece = unit_bytes / 16u - 1u;
@@ -349,7 +349,7 @@ __device__ __forceinline__ void stream_body(const StreamParams &p) {
     uint32_t n_st = 0, st_hist = 0;   // stores of the last `depth` stages, four bits each, and their sum
 
     // Adds up partial sums, wave after wave: thread -> (column tid / 16, row tid % 16) of a fragment, and on by
-    // 512 values.  gate: the first of two stages in turn, whose sums wait in registers for the second's.
+    // kThreads values.  gate: the first of two stages in turn, whose sums wait in registers for the second's.
     constexpr uint32_t kOuts = (PAIR ? 1u : (uint32_t)RT) * NCG * 256u;
     constexpr uint32_t kRounds = (kOuts + kThreads - 1u) / kThreads;
     float gate_sum[kTurns ? kRounds : 1];
