@@ -22,8 +22,10 @@
 // x 2048, 256 experts, down, 16 tokens: 413 / 298.  32 and 64 columns per item lost to the int8 GEMM's narrow tile (512
 // tokens, down 7168 x 2048, 32 columns: 915 / 870): a stage's products, sums and two barriers then outlast its loads.
 //
-// MXFP4: bound by the weight stream.  7168 x 2048, 256 experts, top-8, on the engine's rows: gate/up at 64 tokens
-// 615 us = 5.5 TB/s (by-expert kernels: 720), down 334 us = 5.0 (382); at 200 tokens 739 and 417 us.  The
+// MXFP4: bound by the weight stream.  Every line of it is asked for once, whole and by one instruction (but the ends of
+// a unit), so the loads are non-temporal: whole layers, us with ordinary loads / with these: 7168 x 2048, 256 experts,
+// top-8: 16 tokens 453 / 389, 64: 966 / 865, 300: 1249 / 1226; 4096 x 1024, 128 experts, 37 tokens 188 / 171; all-Q8_0
+// 2048 x 1408: 4 tokens 66 / 61, 40: 140 / 124.  The
 // workgroups of one launch end within 5 % of each other at 64 tokens and 10 % at 16.  Measured and not
 // taken: the last tenth of the work claimed in chunks through a counter (64 tokens 4 % faster, 200 tokens 2
 // to 5 % slower: every chunk loads an item's columns again); a stage read into registers and its place
@@ -294,7 +296,7 @@ __device__ __forceinline__ void stream_body(const StreamParams &p) {
             uint32_t piece = s - run * p.pitch;
             piece = min(piece, p.run - 1u);   // a row's padding repeats its last piece
             // (slots past the last row fetch the unit's last piece: the load stays in the unit)
-            lds_dma16(dst + L * 1024u, second ? src1 : src0, min(run * p.run + piece, last_piece) * 16u);
+            lds_dma16<true>(dst + L * 1024u, second ? src1 : src0, min(run * p.run + piece, last_piece) * 16u);
         }
         q_left--;
         q_slot = q_slot + 1u == p.depth ? 0u : q_slot + 1u;
