@@ -207,16 +207,28 @@ __device__ __forceinline__ void lds_dma4_v(uint32_t lds_addr, const void *ptr) {
                  :: "s"(lds_addr), "v"(ptr) : "memory");
 }
 
-// At most n of the wave's vector memory operations may still be under way (n uniform; above 31: 31).
+// At most n of the wave's vector memory operations may still be under way (n uniform; above 30: 31, or with LONG above
+// 62: 63 -- the choice is a tree of branches, and two levels more of it cost a short stage 1 %).
+template <bool LONG = false>
 __device__ __forceinline__ void wait_vm(uint32_t n) {
 #define DSX_VM(k) case k: asm volatile("s_waitcnt vmcnt(" #k ")" ::: "memory"); break;
-    switch (n) {
-        DSX_VM(0) DSX_VM(1) DSX_VM(2) DSX_VM(3) DSX_VM(4) DSX_VM(5) DSX_VM(6) DSX_VM(7) DSX_VM(8) DSX_VM(9)
-        DSX_VM(10) DSX_VM(11) DSX_VM(12) DSX_VM(13) DSX_VM(14) DSX_VM(15) DSX_VM(16) DSX_VM(17) DSX_VM(18)
-        DSX_VM(19) DSX_VM(20) DSX_VM(21) DSX_VM(22) DSX_VM(23) DSX_VM(24) DSX_VM(25) DSX_VM(26) DSX_VM(27)
-        DSX_VM(28) DSX_VM(29) DSX_VM(30)
-        default: asm volatile("s_waitcnt vmcnt(31)" ::: "memory"); break;
+#define DSX_VM4(a, b, c, d) DSX_VM(a) DSX_VM(b) DSX_VM(c) DSX_VM(d)
+    if constexpr (LONG) {
+        switch (n) {
+            DSX_VM4(0, 1, 2, 3) DSX_VM4(4, 5, 6, 7) DSX_VM4(8, 9, 10, 11) DSX_VM4(12, 13, 14, 15)
+            DSX_VM4(16, 17, 18, 19) DSX_VM4(20, 21, 22, 23) DSX_VM4(24, 25, 26, 27) DSX_VM4(28, 29, 30, 31)
+            DSX_VM4(32, 33, 34, 35) DSX_VM4(36, 37, 38, 39) DSX_VM4(40, 41, 42, 43) DSX_VM4(44, 45, 46, 47)
+            DSX_VM4(48, 49, 50, 51) DSX_VM4(52, 53, 54, 55) DSX_VM4(56, 57, 58, 59) DSX_VM(60) DSX_VM(61) DSX_VM(62)
+            default: asm volatile("s_waitcnt vmcnt(63)" ::: "memory"); break;
+        }
+    } else {
+        switch (n) {
+            DSX_VM4(0, 1, 2, 3) DSX_VM4(4, 5, 6, 7) DSX_VM4(8, 9, 10, 11) DSX_VM4(12, 13, 14, 15)
+            DSX_VM4(16, 17, 18, 19) DSX_VM4(20, 21, 22, 23) DSX_VM4(24, 25, 26, 27) DSX_VM(28) DSX_VM(29) DSX_VM(30)
+            default: asm volatile("s_waitcnt vmcnt(31)" ::: "memory"); break;
+        }
     }
+#undef DSX_VM4
 #undef DSX_VM
 }
 

@@ -97,6 +97,7 @@ inline size_t stream_lds_bytes(const StreamParams &p, bool pair, uint32_t rt, ui
 template <int NI, int NCG>
 struct StreamMxfp4 {
     static constexpr int kWaves = 8;
+    static constexpr bool kRoles = true;   // (below, stream_body)
     static constexpr uint32_t kPart = stream_part_bytes(kWaves) / 4u;
     // operand (super-block sb0 + 4 i, the wave's half) of column n16 of a column group; a super-block past
     // the row's end has zero codes and d = 0
@@ -175,6 +176,7 @@ struct StreamMxfp4 {
 template <int W, int NI>
 struct StreamQ8 {
     static constexpr int kWaves = W;
+    static constexpr bool kRoles = false;
     static constexpr uint32_t kPart = stream_part_bytes(kWaves) / 4u;
     long codes[NI][4];   // bytes 8 g4 .. of block b of a group: column n16
     float xs[NI];        // scale of block g4 of the group; a group past the row's end has zero codes and scales
@@ -240,7 +242,12 @@ template <typename COLS, bool PAIR, int NCG, int RT>
 __device__ __forceinline__ void stream_body(const StreamParams &p) {
     static_assert(!PAIR || RT <= 2, "one row tile of either matrix");
     constexpr int kW = COLS::kWaves;
-    constexpr uint32_t kThreads = (uint32_t)kW * 64u;
+    // Between two stages a wave requests the next one or adds up and stores the last one's sums.  MXFP4: the first half of
+    // the waves does the one, the second half the other, at the same time and without a load that waits behind a store
+    // (vmcnt counts them in order); Q8_0: every wave does its part of both (half each: 2048 x 1408, 40 tokens 124 / 126 us).
+    constexpr uint32_t kLoaders = COLS::kRoles ? (uint32_t)kW / 2u : (uint32_t)kW;
+    constexpr uint32_t kSummer0 = COLS::kRoles ? kLoaders : 0u;               // the first wave that sums
+    constexpr uint32_t kSummers = ((uint32_t)kW - kSummer0) * 64u;            // threads that do
     constexpr bool kTurns = PAIR && RT == 1;
     constexpr uint32_t kTiles = PAIR ? 1u : (uint32_t)RT;   // row tiles of a unit
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
@@ -271,8 +278,9 @@ __device__ __forceinline__ void stream_body(const StreamParams &p) {
 
     // ---- requesting stages ----------------------------------------------------------------------
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)smem) + kStages;
-    const uint32_t n_loads = PAIR && !kTurns ? 2u * p.loads : p.loads;   // of a stage; the wave's: wave, wave + kW, ..
-    const uint32_t my_loads = (n_loads + (uint32_t)kW - 1u - wave) / (uint32_t)kW;
+    const bool loader = !COLS::kRoles || wave < kLoaders, summer = !COLS::kRoles || !loader;
+    const uint32_t n_loads = PAIR && !kTurns ? 2u * p.loads : p.loads;   // of a stage; the wave's: wave, wave + kLoaders, ..
+    const uint32_t my_loads = (n_loads + kLoaders - 1u - wave) / kLoaders;
     const uint32_t unit_bytes = kTiles * 16u * n_sb * (uint32_t)kSuperBytes;
     const uint32_t last_piece = unit_bytes / 16u - 1u;
     uint32_t q_item = item0, q_ut = ut0, q_m = 0, q_slot = 0, q_left = n_stages;   // the next stage to request
@@ -289,7 +297,7 @@ __device__ __forceinline__ void stream_body(const StreamParams &p) {
         const uint8_t *src1 = PAIR && !kTurns ? q_base[1] + (uint64_t)q_ut * unit_bytes : nullptr;
         const uint32_t dst = lds0 + q_slot * p.stage_bytes;
         // (the offsets are the same for every stage, but there are no registers to keep them in)
-        for (uint32_t L = wave; L < n_loads; L += (uint32_t)kW) {
+        for (uint32_t L = wave; L < n_loads; L += kLoaders) {
             const bool second = PAIR && !kTurns && L >= p.loads;
             const uint32_t s = (second ? L - p.loads : L) * 64u + lane;
             const uint32_t run = __umulhi(s, p.pitch_magic);   // s / pitch
@@ -336,9 +344,10 @@ __device__ __forceinline__ void stream_body(const StreamParams &p) {
     };
 
     // the first stage is requested ahead of the look-ups, the others behind them: loads return in order
-    request();
+    if (loader) request();
     load_item(item0);
-    for (uint32_t d = 1; d < p.depth && q_left; d++) request();
+    if (loader)
+        for (uint32_t d = 1; d < p.depth && q_left; d++) request();
 
     // ---- the stages ----------------------------------------------------------------------------
     // read side: row n16 of a tile
@@ -348,23 +357,24 @@ __device__ __forceinline__ void stream_body(const StreamParams &p) {
     // that the lanes' 16-byte writes spread over the banks
     float *part_w = s_part + wave * 256u + n16 * 16u + ((g4 + (n16 >> 2)) & 3u) * 4u;
     uint32_t c_item = item0, c_ut = ut0, slot = 0;
-    uint32_t n_st = 0, st_hist = 0;   // stores of the last `depth` stages, four bits each, and their sum
+    // a loader that stores: its stores of the last `depth` stages, four bits each, and their sum
+    uint32_t n_st = 0, st_hist = 0;
 
-    // Adds up partial sums, wave after wave: thread -> (column tid / 16, row tid % 16) of a fragment, and on by
-    // kThreads values.  gate: the first of two stages in turn, whose sums wait in registers for the second's.
-    constexpr uint32_t kOuts = (PAIR ? 1u : (uint32_t)RT) * NCG * 256u;
-    constexpr uint32_t kRounds = (kOuts + kThreads - 1u) / kThreads;
+    // Adds up partial sums, wave after wave: a thread's values in the order (column, row tile, row), so that the rows of a
+    // unit's tiles, which follow each other in a result row, are stored in whole lines where there is more than one tile
+    // (7168 x 2048, 256 experts, 300 tokens, layer: 1186 / 1170 us).
+    // gate: the first of two stages in turn, whose sums wait in registers for the second's.
+    constexpr uint32_t kOuts = kTiles * NCG * 256u;
+    constexpr uint32_t kRounds = (kOuts + kSummers - 1u) / kSummers;
     float gate_sum[kTurns ? kRounds : 1];
     auto finish = [&](bool gate) __attribute__((always_inline)) {
 #pragma unroll
         for (uint32_t r = 0; r < kRounds; r++) {
-            const uint32_t o0 = r * kThreads, o = o0 + tid;
-            if (kOuts % kThreads != 0u && o >= kOuts) break;
-            const uint32_t frag0 = (o0 >> 8) + (wave >> 2);   // the wave's fragment; its columns start at 4 (wave % 4)
-            const uint32_t cg = PAIR ? frag0 : frag0 % NCG;
-            if (cg * 16u + (wave & 3u) * 4u >= cnt) continue;   // uniform: no member among them
-            const uint32_t col16 = (o >> 4) & 15u, row = o & 15u, col = cg * 16u + col16;
-            const float *f = s_part + frag0 * COLS::kPart + col16 * 16u + ((row + (col16 & 12u)) & 15u);
+            const uint32_t ow = r * kSummers + (wave - kSummer0) * 64u;   // the wave's first value
+            const uint32_t colw = ow / (16u * kTiles);
+            if ((kOuts % kSummers != 0u && ow >= kOuts) || colw >= cnt) continue;   // uniform: no member among its columns
+            const uint32_t col = colw + lane / (16u * kTiles), tile = g4 % kTiles, col16 = col & 15u;
+            const float *f = s_part + (tile * NCG + (col >> 4)) * COLS::kPart + col16 * 16u + ((n16 + (col16 & 12u)) & 15u);
             float a = f[0], b = 0.0f;
 #pragma unroll
             for (int w = 1; w < kW; w++) a += f[w * 256];
@@ -381,14 +391,15 @@ __device__ __forceinline__ void stream_body(const StreamParams &p) {
 #pragma unroll
                 for (int w = 1; w < kW; w++) b += f[w * 256];
             }
-            n_st++;
-            st_hist++;
+            if (kSummer0 == 0u) {
+                n_st++;
+                st_hist++;
+            }
             if (col < cnt) {
-                float *dst = p.out + (uint64_t)s_dest[col] * p.n_rows + (c_ut * kTiles + (PAIR ? 0u : frag0 / NCG)) * 16u + row;
+                float *dst = p.out + (uint64_t)s_dest[col] * p.n_rows + (c_ut * kTiles + tile) * 16u + n16;
                 *dst = PAIR ? swiglu_clamp(a, b, clamp, s_ew[col]) : a;
             }
         }
-        if (!gate) c_ut++;
     };
 
     uint32_t m = 0;   // which matrix the stage is of (in turn)
@@ -399,10 +410,12 @@ __device__ __forceinline__ void stream_body(const StreamParams &p) {
         // the stage's loads have landed; what this wave sent after them may be under way: the younger
         // stages' loads and the stores of the last `depth` stages (counted exactly: a store more than
         // allowed for would be made up by a load of the next stage, most of a stage's time later)
-        wait_vm(min(n_stages - 1u - j, p.depth - 1u) * my_loads + n_st);
+        if (loader) wait_vm<COLS::kRoles>(min(n_stages - 1u - j, p.depth - 1u) * my_loads + n_st);
         __syncthreads();
-        n_st -= (st_hist >> (4u * p.depth - 4u)) & 15u;
-        st_hist <<= 4;
+        if (kSummer0 == 0u) {
+            n_st -= (st_hist >> (4u * p.depth - 4u)) & 15u;
+            st_hist <<= 4;
+        }
         const uint8_t *st = smem + kStages + slot * p.stage_bytes;
 #pragma unroll
         for (int rt = 0; rt < RT; rt++) {
@@ -410,9 +423,11 @@ __device__ __forceinline__ void stream_body(const StreamParams &p) {
                       part_w + (kTurns ? 0u : (uint32_t)rt * NCG) * COLS::kPart);
         }
         __syncthreads();   // the partial sums are there, and nobody reads the stage any more
-        if (q_left) request();
         slot = slot + 1u == p.depth ? 0u : slot + 1u;
-        finish(kTurns && m == 0u);
+        if (loader && q_left) request();
+        const bool gate = kTurns && m == 0u;
+        if (summer) finish(gate);
+        if (!gate) c_ut++;
         m ^= 1u;
         if (c_ut == n_ut && j + 1u < n_stages) {
             c_ut = 0;
