@@ -26,7 +26,8 @@
 // operands of a super-block (half x plane) back to back through one register quad per weight
 // fragment and folds it into the accumulator with the column's d once per super-block (one FMA
 // per value, placed between the next column group's first matrix instructions); the narrow
-// tile, whose operands arrive by half super-blocks, folds once per half.
+// tile, whose operands arrive by half super-blocks, chains the halves the same way, so that both
+// tiles give the same bits.
 #pragma once
 
 #include <type_traits>
@@ -257,19 +258,25 @@ __global__ __launch_bounds__(kGemmWaves * 64, MT == kGemmMT ? 2 : 4) void k_mxfp
     constexpr int kALoads = 4 * kGemmRF + 2;  // per wave and super-block
     // load L of those: 0..7 the halves of the four fragments, 8 and 9 the scales of the row sets
     // (row runs: loads 0..4 the first row set, 5..9 the second)
-    auto issue_a_one = [&](int L, uint32_t sb) __attribute__((always_inline)) {
+    // NT: non-temporal loads.  Planar weights in the narrow tile of a group that has no other: every line is then fetched
+    // once and whole (7168 x 2048, 256 experts, layer us without / with: 16 tokens 473 / 429, 100: 1033 / 960, 200: 1105 /
+    // 1077; 4096 x 1024, 128 experts, 37: 168 / 147).  Groups of several tiles find each other's lines in the L2 (400
+    // tokens, with such loads throughout: 1240 / 1290), the engine's rows their neighbours' (4096 tokens 3095 / 4085).
+    auto issue_a_one = [&](auto ntc, int L, uint32_t sb) __attribute__((always_inline)) {
+        constexpr bool NT = decltype(ntc)::value;
         if constexpr (kRun) {
             const int m = L / 5, i = L - 5 * m;
             lds_dma16(a_lds + (uint32_t)(m * 5120 + i * 1024), wbase[m] + (a_slab[0][m] + sb * kStepW), run_off[i]);
         } else if (L < 4 * kGemmRF) {
             const int f = L >> 1, i = L & 1, r = f >> 1, m = f & 1;
-            lds_dma16(a_lds + (uint32_t)(f * 2048 + i * 1024),
+            lds_dma16<NT>(a_lds + (uint32_t)(f * 2048 + i * 1024),
                       wbase[m] + (a_slab[r][m] + (uint32_t)i * 8u * row_stride + sb * kStepW), a_fetch);
         } else {
             const int m = L - 4 * kGemmRF;
             lds_dma4(a_lds + kScaleOff + (uint32_t)m * 256u, wbase[m] + (a_slab[0][m] + sb * kStepW), sc_fetch);
         }
     };
+    constexpr std::integral_constant<bool, false> kNoNt{};
     constexpr int kAFirst = 8;  // of them requested during the first half of a super-block
     // read side: lane (row n16, block g4) of fragment f: chunk g4 (first half), 4 + g4 (second)
     const uint32_t sw = ((n16 & 7u) * 8u + (g4 ^ (n16 & 7u))) * 16u;  // within a 1 KB slab
@@ -423,16 +430,16 @@ __global__ __launch_bounds__(kGemmWaves * 64, MT == kGemmMT ? 2 : 4) void k_mxfp
                 if constexpr (gp < ALoads) {
                     // literal indices: the load's registers are picked at compile time
                     constexpr int kA = AFrom;
-                    if (gp == 0) issue_a_one(kA + 0 < kALoads ? kA + 0 : 0, sb + 1u);
-                    if (gp == 1) issue_a_one(kA + 1 < kALoads ? kA + 1 : 0, sb + 1u);
-                    if (gp == 2) issue_a_one(kA + 2 < kALoads ? kA + 2 : 0, sb + 1u);
-                    if (gp == 3) issue_a_one(kA + 3 < kALoads ? kA + 3 : 0, sb + 1u);
-                    if (gp == 4) issue_a_one(kA + 4 < kALoads ? kA + 4 : 0, sb + 1u);
-                    if (gp == 5) issue_a_one(kA + 5 < kALoads ? kA + 5 : 0, sb + 1u);
-                    if (gp == 6) issue_a_one(kA + 6 < kALoads ? kA + 6 : 0, sb + 1u);
-                    if (gp == 7) issue_a_one(kA + 7 < kALoads ? kA + 7 : 0, sb + 1u);
-                    if (gp == 8) issue_a_one(kA + 8 < kALoads ? kA + 8 : 0, sb + 1u);
-                    if (gp == 9) issue_a_one(kA + 9 < kALoads ? kA + 9 : 0, sb + 1u);
+                    if (gp == 0) issue_a_one(kNoNt, kA + 0 < kALoads ? kA + 0 : 0, sb + 1u);
+                    if (gp == 1) issue_a_one(kNoNt, kA + 1 < kALoads ? kA + 1 : 0, sb + 1u);
+                    if (gp == 2) issue_a_one(kNoNt, kA + 2 < kALoads ? kA + 2 : 0, sb + 1u);
+                    if (gp == 3) issue_a_one(kNoNt, kA + 3 < kALoads ? kA + 3 : 0, sb + 1u);
+                    if (gp == 4) issue_a_one(kNoNt, kA + 4 < kALoads ? kA + 4 : 0, sb + 1u);
+                    if (gp == 5) issue_a_one(kNoNt, kA + 5 < kALoads ? kA + 5 : 0, sb + 1u);
+                    if (gp == 6) issue_a_one(kNoNt, kA + 6 < kALoads ? kA + 6 : 0, sb + 1u);
+                    if (gp == 7) issue_a_one(kNoNt, kA + 7 < kALoads ? kA + 7 : 0, sb + 1u);
+                    if (gp == 8) issue_a_one(kNoNt, kA + 8 < kALoads ? kA + 8 : 0, sb + 1u);
+                    if (gp == 9) issue_a_one(kNoNt, kA + 9 < kALoads ? kA + 9 : 0, sb + 1u);
                 }
                 // Nothing moves across the end of an operand's products: the request of the next
                 // operand stays right ahead of them, the folds beside them.  (The empty statement
@@ -478,7 +485,7 @@ __global__ __launch_bounds__(kGemmWaves * 64, MT == kGemmMT ? 2 : 4) void k_mxfp
                 issue_phase(sb + 1u, 0, (sb + 1u) & 1u);
                 issue_yd(sb + 1u);
                 // fewer operands than weight loads: the rest of the loads in front
-                gemm_static_for<4 * NJ, kALoads>([&](auto lc) __attribute__((always_inline)) { issue_a_one(decltype(lc)::value, sb + 1u); });
+                gemm_static_for<4 * NJ, kALoads>([&](auto lc) __attribute__((always_inline)) { issue_a_one(kNoNt, decltype(lc)::value, sb + 1u); });
             }
             constexpr int kBeside = !more ? 0 : 4 * NJ < kALoads ? 4 * NJ : kALoads;
             compute_phase(njc, I0{}, I0{}, std::integral_constant<int, kBeside>{}, sb & 1u, sb);
@@ -572,46 +579,31 @@ __global__ __launch_bounds__(kGemmWaves * 64, MT == kGemmMT ? 2 : 4) void k_mxfp
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
 
-        const uint32_t nj = (cnt + 15u) / 16u;  // column groups that hold a real column
-        // One half super-block with NJ column groups (compile-time, so the code below is one
-        // straight line): for every group, the two pieces (high and low plane) against the wave's
-        // four fragments, then the fold acc += d * c -- placed right before each fragment's
-        // temporary is overwritten by the next group's first piece.  The next piece's B operand is
-        // requested from LDS one piece ahead of its use (deeper changes nothing).  Empty asm
-        // statements pin that order; they emit no instruction, so the compiler still sees every
-        // real one and keeps its hazards.  Left alone it hoists every LDS read of the half to its
-        // top, which overflows the registers, pulls each fold up to the instruction that produces
-        // its input, where it waits, and with the group count as a run-time condition waits for
-        // each operand right after requesting it (layer at T=4096: 4.5 -> 4.0 ms).
+        // One half super-block of the tile's column group: its two operands (high and low plane) against the wave's four
+        // fragments, chained through c with the other half's as in the wide tile, then (second half) the fold acc += d * c.
+        // An operand is requested from LDS ahead of the products of the one before it.  Empty asm statements pin that
+        // order; they emit no instruction, so the compiler still sees every real one and keeps its hazards.
+        v4f c[kGemmRF][2];
     #define DSX_PIN() asm volatile("" ::: "memory")
-        auto compute_half = [&](auto hc, auto njc, const uint32_t sb, const bool more) {
+        auto compute_half = [&](auto ntc, auto hc, const uint32_t sb, const bool more) {
             constexpr int h = decltype(hc)::value;
-            constexpr int NJ = decltype(njc)::value;
             const uint8_t *half = tiles + h * kHeadsBytes;
             const uint8_t *tails = tiles + kTailsOff + (sb & 1u) * kTailsBytes;
-            const float *yds = s_yd + ((sb >> 2) & 1u) * (uint32_t)(kYdBytes / 4) + (sb & 3u);
-            // the operand of (column group j, plane q): 16 bytes of head, 8 of tail
-            auto load_piece = [&](int j, int q) -> v8i {
-                const uint32_t cb = (((uint32_t)(2 * j) + (n16 >> 3)) * 1024u + sw) ^ ((uint32_t)q * 64u);
-                const uint4 hd = *(const uint4 *)(half + cb);
-                const uint2 tl = *(const uint2 *)(tails + (uint32_t)j * 2048u +
-                                                  (bt_rd ^ ((uint32_t)q * 32u) ^ ((uint32_t)h * 64u)));
+            // the operand of plane q: 16 bytes of head, 8 of tail
+            auto load_piece = [&](int q) -> v8i {
+                const uint4 hd = *(const uint4 *)(half + (((n16 >> 3) * 1024u + sw) ^ ((uint32_t)q * 64u)));
+                const uint2 tl = *(const uint2 *)(tails + (bt_rd ^ ((uint32_t)q * 32u) ^ ((uint32_t)h * 64u)));
                 return v8i{(int)hd.x, (int)hd.y, (int)hd.z, (int)hd.w, (int)tl.x, (int)tl.y, 0, 0};
             };
-            v4f c[kGemmRF][2];
-            // piece p = 2 j + q alternates between two operand registers
-            constexpr int NP = 2 * NJ;
             v8i ring[2];
-            ring[0] = load_piece(0, 0);
-            float yd_prev = 0.0f, yd = 0.0f;
+            ring[0] = load_piece(0);
+            const float yd = h == 1 ? s_yd[((sb >> 2) & 1u) * (uint32_t)(kYdBytes / 4) + (sb & 3u) + n16 * 4u] : 0.0f;
             DSX_PIN();
-    #pragma unroll
-            for (int pc = 0; pc < NP; pc++) {
-                const int j = pc >> 1, q = pc & 1;
-                if (q == 0) yd = yds[(j * 16u + n16) * 4u];
-                if (pc + 1 < NP) ring[(pc + 1) & 1] = load_piece((pc + 1) >> 1, (pc + 1) & 1);
+            gemm_static_for<0, 2>([&](auto qc) __attribute__((always_inline)) {
+                constexpr int q = decltype(qc)::value;
+                if (q == 0) ring[1] = load_piece(1);
                 DSX_PIN();
-                v8i &bq = ring[pc & 1];
+                v8i &bq = ring[q];
                 asm volatile("" : "+v"(bq));  // the products with this piece stay behind the request above
     #pragma unroll
                 for (int r = 0; r < kGemmRF; r++)
@@ -620,70 +612,41 @@ __global__ __launch_bounds__(kGemmWaves * 64, MT == kGemmMT ? 2 : 4) void k_mxfp
                         const GemmAFrag &w = a_cur[r][m];
                         const uint4 &aw = h == 0 ? w.a0 : w.a1;
                         const v8i av = {(int)aw.x, (int)aw.y, (int)aw.z, (int)aw.w, 0, 0, 0, 0};
-                        if (q == 0) {
-                            if (j > 0) {
-                                asm volatile("" : "+v"(c[r][m]));
-                                v4f &a = acc[r][m][j > 0 ? j - 1 : 0];
-                                a.x = fmaf(yd_prev, c[r][m].x, a.x);
-                                a.y = fmaf(yd_prev, c[r][m].y, a.y);
-                                a.z = fmaf(yd_prev, c[r][m].z, a.z);
-                                a.w = fmaf(yd_prev, c[r][m].w, a.w);
-                                asm volatile("" : "+v"(a));
-                            }
-                            c[r][m] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
-                                av, bq, v4f{0.f, 0.f, 0.f, 0.f}, 4, 2, h, (int)w.sc, 0, kScaleB6High);
-                        } else {
-                            c[r][m] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
-                                av, bq, c[r][m], 4, 2, h, (int)w.sc, 0, kScaleB6Low);
-                        }
+                        const v4f from = h == 0 && q == 0 ? v4f{0.f, 0.f, 0.f, 0.f} : c[r][m];
+                        c[r][m] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+                            av, bq, from, 4, 2, h, (int)w.sc, 0, q == 0 ? kScaleB6High : kScaleB6Low);
                     }
-                if (q == 1) yd_prev = yd;
-                // the next super-block's weights, a load or two behind each piece's products: a
-                // request that has to wait for room in the memory pipeline then holds back nothing
-                // that the matrix pipe does not already have
-                {
-                    constexpr int kFrom = h == 0 ? 0 : kAFirst, kCnt = h == 0 ? kAFirst : kALoads - kAFirst;
-                    // behind the first pieces of a half: 8 of the 10 in the first half, one per piece (a
-                    // few per cent faster than 6 + 4 and than all 10 at once, measured at 4096 tokens)
-                    constexpr int kSpan = h == 0 ? (NP < 8 ? NP : 8) : (NP + 1) / 2;
-                    const int lo = pc * kCnt / kSpan, hi = (pc + 1) * kCnt / kSpan;
-                    if (pc < kSpan && more) {
-                        // literal indices: the load's registers are picked at compile time
-                        if (0 < kCnt && lo <= 0 && 0 < hi) issue_a_one(kFrom + 0, sb + 1u);
-                        if (1 < kCnt && lo <= 1 && 1 < hi) issue_a_one(kFrom + 1, sb + 1u);
-                        if (2 < kCnt && lo <= 2 && 2 < hi) issue_a_one(kFrom + 2, sb + 1u);
-                        if (3 < kCnt && lo <= 3 && 3 < hi) issue_a_one(kFrom + 3, sb + 1u);
-                        if (4 < kCnt && lo <= 4 && 4 < hi) issue_a_one(kFrom + 4, sb + 1u);
-                        if (5 < kCnt && lo <= 5 && 5 < hi) issue_a_one(kFrom + 5, sb + 1u);
-                        if (6 < kCnt && lo <= 6 && 6 < hi) issue_a_one(kFrom + 6, sb + 1u);
-                        if (7 < kCnt && lo <= 7 && 7 < hi) issue_a_one(kFrom + 7, sb + 1u);
-                        if (8 < kCnt && lo <= 8 && 8 < hi) issue_a_one(kFrom + 8, sb + 1u);
-                        if (9 < kCnt && lo <= 9 && 9 < hi) issue_a_one(kFrom + 9, sb + 1u);
-                    }
+                // the next super-block's weights behind the products: a request that has to wait for room in the
+                // memory pipeline then holds back nothing that the matrix pipe does not already have
+                if (more) {
+                    constexpr int kPart = h == 0 ? kAFirst / 2 : q == 0 ? kALoads - kAFirst : 0;
+                    constexpr int kFrom = h == 0 ? q * kPart : kAFirst;
+                    gemm_static_for<0, kPart>([&](auto lc) __attribute__((always_inline)) { issue_a_one(ntc, kFrom + decltype(lc)::value, sb + 1u); });
                 }
+            });
+            if (h == 1) {
+    #pragma unroll
+                for (int r = 0; r < kGemmRF; r++)
+    #pragma unroll
+                    for (int m = 0; m < 2; m++) {
+                        v4f &a = acc[r][m][0];
+                        a.x = fmaf(yd, c[r][m].x, a.x);
+                        a.y = fmaf(yd, c[r][m].y, a.y);
+                        a.z = fmaf(yd, c[r][m].z, a.z);
+                        a.w = fmaf(yd, c[r][m].w, a.w);
+                    }
             }
-            // fold the last group
-    #pragma unroll
-            for (int r = 0; r < kGemmRF; r++)
-    #pragma unroll
-                for (int m = 0; m < 2; m++) {
-                    v4f &a = acc[r][m][NJ - 1];
-                    a.x = fmaf(yd_prev, c[r][m].x, a.x);
-                    a.y = fmaf(yd_prev, c[r][m].y, a.y);
-                    a.z = fmaf(yd_prev, c[r][m].z, a.z);
-                    a.w = fmaf(yd_prev, c[r][m].w, a.w);
-                }
         };
     #undef DSX_PIN
 
-        auto main_loop = [&](auto njc) {
+        auto main_loop = [&](auto ntc) {
             for (uint32_t sb = 0; sb < p.n_sb; sb++) {
                 const bool more = sb + 1u < p.n_sb;
                 read_a();
                 // the wave's A region is free again once its reads have returned
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
                 issue_b(sb, 1);
-                compute_half(std::integral_constant<int, 0>{}, njc, sb, more);
+                compute_half(ntc, std::integral_constant<int, 0>{}, sb, more);
                 // the second half of B has landed (the younger weight loads may still be on their way)
                 if (more) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(kAFirst) : "memory");
                 else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -693,29 +656,16 @@ __global__ __launch_bounds__(kGemmWaves * 64, MT == kGemmMT ? 2 : 4) void k_mxfp
                     issue_bt(sb + 1u);
                     issue_yd(sb + 1u);
                 }
-                compute_half(std::integral_constant<int, 1>{}, njc, sb, more);
+                compute_half(ntc, std::integral_constant<int, 1>{}, sb, more);
                 // everything this wave fetched for the next super-block has landed before the others
                 // may read it
                 asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
                 __syncthreads();
             }
         };
-        // the number of column groups that hold a real column picks the instantiation
-        if constexpr (kGemmCG == 1) {
-            main_loop(std::integral_constant<int, 1>{});
-        } else {
-            switch (nj) {
-                case 1: main_loop(std::integral_constant<int, 1>{}); break;
-                case 2: main_loop(std::integral_constant<int, 2>{}); break;
-                case 3: main_loop(std::integral_constant<int, 3>{}); break;
-                case 4: main_loop(std::integral_constant<int, 4>{}); break;
-                case 5: main_loop(std::integral_constant<int, 5>{}); break;
-                case 6: main_loop(std::integral_constant<int, 6>{}); break;
-                case 7: main_loop(std::integral_constant<int, 7>{}); break;
-                default: main_loop(std::integral_constant<int, 8>{}); break;
-            }
-        }
-
+        static_assert(kGemmCG == 1, "the narrow tile has one column group");
+        if (PLANAR && (uint32_t)p.group_count[e] <= (uint32_t)MT) main_loop(std::integral_constant<bool, PLANAR>{});   // uniform
+        else main_loop(kNoNt);
     }
 
     // ---- epilogue ---------------------------------------------------------------------
