@@ -217,12 +217,13 @@ static int fit_nt(uint32_t chunk, uint32_t n_blocks, int cap) {
 // optional extra group `n_expert` that holds every token (slot n_used).
 int group_build_big(hipStream_t st, int32_t *group_count, int32_t *group_offset, int32_t *members,
                     int32_t *work_items, int32_t *n_work_items, const int32_t *selected, uint32_t b,
-                    uint32_t n_used, uint32_t n_expert, uint32_t chunk, bool extra, ItemList list2 = {}, ItemList list3 = {}) {
-    // list2, list3 (with list2): further lists of work items
+                    uint32_t n_used, uint32_t n_expert, uint32_t chunk, bool extra, ItemList list2 = {}, ItemList list3 = {},
+                    GroupSplit split = {}) {
+    // list2, list3 (with list2): further lists of work items; split: which groups the first two of them have
     const uint32_t lists = 1u + (list2.items ? 1u : 0u) + (list3.items ? 1u : 0u);
     hipLaunchKernelGGL(k_group_tables, dim3(n_expert + (extra ? 1u : 0u) + lists), dim3(kGbThreads), 0, st,
                        group_count, group_offset, members, work_items, n_work_items, selected, b, n_used,
-                       n_expert, chunk, extra ? 1u : 0u, list2, list3);
+                       n_expert, chunk, extra ? 1u : 0u, list2, list3, split);
     return launched("group_tables");
 }
 

@@ -602,20 +602,21 @@ __global__ __launch_bounds__(256) void k_q8_0_quantize(int8_t *__restrict__ xq,
 // ---------------------------------------------------------------------------------------
 constexpr int kGbThreads = 1024;
 
-// Exclusive prefix sums of count[0..n) into off[0..n] and of the groups' work items,
-// ceil(count / chunk), into wi_off[0..n] (entry n: the totals), by the first wave of the workgroup:
+// Exclusive prefix sums of count[0..n) into off[0..n] and of the groups' work items, ceil(count / chunk) (groups
+// of more than `above` and up to `most` members, others none), into wi_off[0..n] (entry n: the totals), by the first wave of the workgroup:
 // a lane adds up its share of consecutive groups, the lanes scan their sums with shuffles, and
 // every lane writes its groups' offsets (one thread walking 257 groups through LDS took 8 us).
 // The caller puts a barrier on either side.
 __device__ __forceinline__ void gb_scan(const int *s_count, int *s_off, int *s_wi_off, uint32_t n,
-                                        uint32_t chunk, uint32_t tid) {
+                                        uint32_t chunk, uint32_t above, uint32_t most, uint32_t tid) {
     if (tid >= 64u) return;
+    auto items = [&](int c) { return (uint32_t)c > above && (uint32_t)c <= most ? (c + (int)chunk - 1) / (int)chunk : 0; };
     const uint32_t per = (n + 63u) / 64u;
     const uint32_t b = min(n, tid * per), e = min(n, b + per);
     int sa = 0, sw = 0;
     for (uint32_t i = b; i < e; i++) {
         sa += s_count[i];
-        sw += (s_count[i] + (int)chunk - 1) / (int)chunk;
+        sw += items(s_count[i]);
     }
     int ia = sa, iw = sw;   // inclusive scan over the lanes
 #pragma unroll
@@ -631,7 +632,7 @@ __device__ __forceinline__ void gb_scan(const int *s_count, int *s_off, int *s_w
         s_off[i] = ea;
         s_wi_off[i] = ew;
         ea += s_count[i];
-        ew += (s_count[i] + (int)chunk - 1) / (int)chunk;
+        ew += items(s_count[i]);
     }
     if (tid == 63u) {
         s_off[n] = ia;
@@ -646,18 +647,37 @@ __device__ __forceinline__ void gb_scan(const int *s_count, int *s_off, int *s_w
 // e < n_groups places the members of group e.  A placing workgroup reads every pick anyway, so it
 // counts the picks of lower groups itself (its group's offset) and waits for nobody.
 // ---------------------------------------------------------------------------------------
+
+// Two lists with items of different widths, `most` and wide_chunk members: the groups of up to `most` members go to the
+// narrow one, the others to the wide one -- or all groups to the narrow one where that is less work: a wide item weighs
+// 3/2 of a narrow one and wide items come `round` at a time (7168 x 2048, 256 experts, planar weights, 200 tokens: on
+// picks skewed like Zipf's 30 wide items take 24 us off 991; all tokens on the same picks: 117 narrow items take 265 us, 18 wide
+// ones 185).  Fewer than min_narrow narrow items go to the wide list as well.
+struct GroupSplit {
+    uint32_t most, wide_chunk, round, min_narrow;   // most 0: no split, every list has all groups
+};
+
+// A list of work items of up to `chunk` members each; items null: none.
+struct ItemList {
+    int32_t *items, *n;
+    uint32_t chunk;
+};
+
 __device__ __forceinline__ void group_count_body(
-    int32_t *__restrict__ group_count, int32_t *__restrict__ group_offset,
-    int32_t *__restrict__ work_items, int32_t *__restrict__ n_work_items,
-    const int32_t *__restrict__ selected, uint32_t b, uint32_t n_used, uint32_t n_expert,
-    uint32_t chunk, uint32_t extra) {
+    int32_t *__restrict__ group_count, int32_t *__restrict__ group_offset, const ItemList l,
+    const int32_t *__restrict__ selected, uint32_t b, uint32_t n_used, uint32_t n_expert, uint32_t extra,
+    const GroupSplit split) {
+    int32_t *const work_items = l.items, *const n_work_items = l.n;
+    const uint32_t chunk = l.chunk;
     __shared__ int s_count[DSX_MAX_EXPERTS_K + 1];
     __shared__ int s_off[DSX_MAX_EXPERTS_K + 2];
     __shared__ int s_wi_off[DSX_MAX_EXPERTS_K + 2];
+    __shared__ int s_split[3];
     const uint32_t tid = threadIdx.x;
     const uint32_t total = b * n_used;
     const uint32_t n_groups = n_expert + (extra ? 1u : 0u);
     for (uint32_t e = tid; e < n_groups; e += kGbThreads) s_count[e] = 0;
+    if (tid < 3u) s_split[tid] = 0;
     __syncthreads();
     auto count = [&](int e) {
         if (e >= 0 && (uint32_t)e < n_expert) atomicAdd(&s_count[e], 1);
@@ -673,7 +693,29 @@ __device__ __forceinline__ void group_count_body(
     for (uint32_t i = 4u * n4 + tid; i < total; i += kGbThreads) count(selected[i]);
     if (extra && tid == 0) s_count[n_expert] = (int)b;
     __syncthreads();
-    gb_scan(s_count, s_off, s_wi_off, n_groups, chunk, tid);
+    uint32_t above = 0u, most = ~0u;
+    if (split.most) {   // uniform
+        // items of the groups over `most`, groups up to it, narrow items with all groups
+        int n[3] = {0, 0, 0};
+        for (uint32_t e = tid; e < n_groups; e += kGbThreads) {
+            const uint32_t c = (uint32_t)s_count[e], tiles = (c + split.most - 1u) / split.most;
+            n[c > split.most ? 0 : 1] += c > split.most ? (int)((c + split.wide_chunk - 1u) / split.wide_chunk) : (int)tiles;
+            n[2] += (int)tiles;
+        }
+#pragma unroll
+        for (int q = 0; q < 3; q++) {
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) n[q] += __shfl_xor(n[q], o, 64);
+            if ((tid & 63u) == 0u && n[q]) atomicAdd(&s_split[q], n[q]);
+        }
+        __syncthreads();
+        const uint32_t n_wide = (uint32_t)s_split[0], n_small = (uint32_t)s_split[1], n_narrow = (uint32_t)s_split[2];
+        const bool wide = 3u * max(n_wide, split.round) + 2u * n_small < 2u * n_narrow;
+        const bool narrow = !wide || n_small >= split.min_narrow;
+        if (chunk == split.wide_chunk) above = wide ? (narrow ? split.most : 0u) : ~0u;
+        else most = narrow ? (wide ? split.most : ~0u) : 0u;
+    }
+    gb_scan(s_count, s_off, s_wi_off, n_groups, chunk, above, most, tid);
     __syncthreads();
     if (tid == 0) *n_work_items = s_wi_off[n_groups];
     for (uint32_t e = tid; e < n_groups; e += kGbThreads) {
@@ -694,18 +736,12 @@ __device__ __forceinline__ void group_count_body(
     }
 }
 
-// A list of work items of up to `chunk` members each; items null: none.
-struct ItemList {
-    int32_t *items, *n;
-    uint32_t chunk;
-};
-
 __global__ __launch_bounds__(kGbThreads) void k_group_tables(
     int32_t *__restrict__ group_count, int32_t *__restrict__ group_offset,
     int32_t *__restrict__ members, int32_t *__restrict__ work_items,
     int32_t *__restrict__ n_work_items, const int32_t *__restrict__ selected, uint32_t b,
     uint32_t n_used, uint32_t n_expert, uint32_t chunk, uint32_t extra, const ItemList list2,
-    const ItemList list3) {
+    const ItemList list3, const GroupSplit split) {
     constexpr uint32_t kWaves = kGbThreads / 64;
     __shared__ uint32_t s_mine[kWaves], s_below[kWaves];
     const uint32_t n_groups = n_expert + (extra ? 1u : 0u);
@@ -714,7 +750,7 @@ __global__ __launch_bounds__(kGbThreads) void k_group_tables(
         // offsets too, with the same values
         const uint32_t which = blockIdx.x - n_groups;
         const ItemList l = which == 0u ? ItemList{work_items, n_work_items, chunk} : which == 1u ? list2 : list3;
-        group_count_body(group_count, group_offset, l.items, l.n, selected, b, n_used, n_expert, l.chunk, extra);
+        group_count_body(group_count, group_offset, l, selected, b, n_used, n_expert, extra, split);
         return;
     }
     const uint32_t e = blockIdx.x, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63u;
