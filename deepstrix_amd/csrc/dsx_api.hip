@@ -688,15 +688,15 @@ int dsx_moe_down_by_expert(dsx_stream_t stream, int dtype, float *partials, cons
 
 static int reduce_impl(hipStream_t st, float *out, const float *partials, const int32_t *selected,
                        const float *add, uint32_t n_used, uint32_t n_rows, uint32_t b,
-                       const HcPost &hc = HcPost{}) {
+                       const HcPost &hc = HcPost{}, const float *residual = nullptr) {
     if (b == 0) return DSX_OK;
     if ((!out && !hc.n_hc) || !partials) return fail(DSX_ERR_INVALID_ARG, "moe_reduce_partials: null pointer");
     if (n_rows == 0 || n_rows % 4 != 0 || !aligned(out, 16) || !aligned(partials, 16) ||
-        (add && !aligned(add, 16)))
+        (add && !aligned(add, 16)) || (residual && !aligned(residual, 16)))
         return fail(DSX_ERR_SHAPE, "moe_reduce_partials: n_rows=%u must be a multiple of 4, buffers 16-byte aligned", n_rows);
     const uint64_t n4 = (uint64_t)b * (n_rows / 4);
     hipLaunchKernelGGL(k_reduce_partials, dim3((uint32_t)((n4 + 255) / 256)), dim3(256), 0, st, out,
-                       partials, selected, add, n_used, n_rows, b, hc);
+                       partials, selected, add, residual, n_used, n_rows, b, hc);
     return launched("moe_reduce_partials");
 }
 

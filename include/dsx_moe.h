@@ -372,7 +372,10 @@ int dsx_moe_layer_get_tuning(const dsx_moe_layer *layer, uint32_t out[6]);
  * matrix the range of gate/up, from 2 tokens to below 28 picks per expert [2 .. 895]; few picks in all and matrices
  * under 4 M elements start later; all-Q8_0: from 2 tokens to below 4 picks per expert, 1.5 where a matrix has up to
  * 2 M elements.  Where the same token count would take a grouped GEMM otherwise, the device chooses between the two by
- * the picks (all-Q8_0: for more than 16 tokens where n_expert * hidden * inter is at least 256 M). */
+ * the picks (all-Q8_0: for more than 16 tokens where n_expert * hidden * inter is at least 256 M).
+ * Below out[0] the decode path of an all-MXFP4 layer on the engine's rows uses the same kernels from 28 picks on (48 where a
+ * matrix has under 8 M elements, 112 under 3 M; beside a shared expert of another format from 7 tokens at the earliest)
+ * [4 .. 8 tokens], until the caller sets decode_max_tokens or a decode form other than 1. */
 int dsx_moe_layer_get_streaming(const dsx_moe_layer *layer, uint32_t out[2]);
 /* Decode path of an all-MXFP4 layer (up to decode_max_tokens tokens, or to where streaming begins); no
  * counterpart in the reference.  fused: 1 = gate/up, mid quantization, down and the slot-order sum in ONE launch

@@ -206,3 +206,50 @@ def test_a_stack_of_streaming_blocks(monkeypatch, fmt, T):
         assert torch.equal(eager, replayed), step
     final = verify_chain_stepwise(chain, shapes, h, 3 * 2e-3, min_checked=(9 * 2 * T) // 10)   # (the bar of the other chains)
     assert np.array_equal(final, eager.cpu().numpy())
+
+
+@pytest.mark.parametrize("hidden,inter,E,k,T", [(4096, 2048, 16, 8, 4), (4096, 2048, 16, 8, 8), (7168, 2048, 64, 8, 4), (2048, 1536, 16, 6, 8),
+                                                (1536, 1536, 64, 6, 19), (2048, 1536, 16, 6, 7), (4096, 2048, 16, 8, 3)])
+@pytest.mark.parametrize("shared", ["none", "same", "q8_0"])
+def test_few_tokens_stream_in_the_decode_launch_s_place(monkeypatch, hidden, inter, E, k, T, shared):
+    """From 28, 48 or 112 picks on by size of a matrix (the last two: one token short of it); a decode limit set by the
+    caller brings the one-launch form back, the same sums in another order."""
+    monkeypatch.setattr(MoeLayer, "v3_thresholds_below_experts", None)
+    fmts = dict(sh_gate_fmt=FMT_Q8_0, sh_down_fmt=FMT_Q8_0) if shared == "q8_0" else {}
+    s = H.Shape(hidden, inter, E, k, shared=shared != "none", seed=950 + T, **fmts, **ROUTER)
+    dw = H.device_weights(s)
+    layer, launch = MoeLayer(dw, T), MoeLayer(dw, T)
+    launch.set_tuning(decode_max_tokens=16)
+    x, _, _ = H.host_inputs(s, T)
+    rng = np.random.default_rng(T)
+    sel = np.stack([rng.permutation(E)[:k] for _ in range(T)]).astype(np.int32)
+    sel[T // 2, 1] = -1
+    w = rng.uniform(0.05, 0.6, sel.shape).astype(np.float32)
+    dx, ds, dwt = torch.from_numpy(x).cuda(), torch.from_numpy(sel).cuda(), torch.from_numpy(w).cuda()
+    out = layer.run(dx, None, selected_in=ds, weights_in=dwt).clone()
+    again = layer.run(dx, None, selected_in=ds, weights_in=dwt)
+    if T <= 16:
+        other = launch.run(dx, None, selected_in=ds, weights_in=dwt)
+        assert layer.status() == 0 and launch.status() == 0
+        assert H.max_rel(out.cpu().numpy(), other.cpu().numpy()) < 1e-3
+    torch.cuda.synchronize()
+    assert torch.equal(out, again)
+    H.assert_close(out.cpu().numpy(), ref.moe_forward(H.host_weights(s), x, sel, w), 2e-3, f"{hidden} x {inter} T={T} {shared}")
+
+
+def test_a_stack_of_few_token_streaming_blocks(monkeypatch):
+    """The residual is added by the slot-order sum, in place."""
+    monkeypatch.setattr(MoeLayer, "v3_thresholds_below_experts", None)
+    shapes = layer_shapes(H.Shape(4096, 2048, 16, 8, seed=960, **ROUTER), 2)
+    chain = MoeChain([H.device_weights(s, block=True) for s in shapes], 5)
+    rng = np.random.default_rng(5)
+    chain.capture(5)
+    for step in range(3):
+        h = rng.normal(0, 1, (5, 4096)).astype(np.float32)
+        eager = chain.step(torch.from_numpy(h).cuda()).clone()
+        torch.cuda.synchronize()
+        replayed = chain.replay(torch.from_numpy(h).cuda()).clone()
+        torch.cuda.synchronize()
+        assert torch.equal(eager, replayed), step
+    final = verify_chain_stepwise(chain, shapes, h, 3 * 2e-3, min_checked=(9 * 2 * 5) // 10)
+    assert np.array_equal(final, eager.cpu().numpy())
