@@ -847,14 +847,26 @@ __global__ __launch_bounds__(256) void k_reduce_partials(float *out, const float
     const uint64_t per_row = n_rows / 4u;
     if (i >= (uint64_t)b * per_row) return;
     const uint64_t t = i / per_row, c = i - t * per_row;
+    // eight slots at a time, all of their loads ahead of the sums (an empty slot's row is read and not added)
+    constexpr uint32_t kAhead = 8;
     float4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (uint32_t s = 0; s < n_used; s++) {
-        if (selected != nullptr && selected[t * n_used + s] < 0) continue;
-        const v4f v = __builtin_nontemporal_load((const v4f *)(partials + ((t * n_used + s) * n_rows) + c * 4u));
-        acc.x += v.x;
-        acc.y += v.y;
-        acc.z += v.z;
-        acc.w += v.w;
+    const float *rows = partials + t * n_used * n_rows + c * 4u;
+    for (uint32_t s0 = 0; s0 < n_used; s0 += kAhead) {
+        v4f v[kAhead];
+        bool live[kAhead];
+#pragma unroll
+        for (uint32_t q = 0; q < kAhead; q++) {
+            const uint32_t s = min(s0 + q, n_used - 1u);
+            live[q] = s0 + q < n_used && (selected == nullptr || selected[t * n_used + s] >= 0);
+            v[q] = __builtin_nontemporal_load((const v4f *)(rows + (uint64_t)s * n_rows));
+        }
+#pragma unroll
+        for (uint32_t q = 0; q < kAhead; q++) {
+            acc.x = live[q] ? acc.x + v[q].x : acc.x;
+            acc.y = live[q] ? acc.y + v[q].y : acc.y;
+            acc.z = live[q] ? acc.z + v[q].z : acc.z;
+            acc.w = live[q] ? acc.w + v[q].w : acc.w;
+        }
     }
     for (const float *a : {add, residual}) {
         if (a == nullptr) continue;
