@@ -517,18 +517,18 @@ inline int q8_0_down_by_expert(hipStream_t st, float *partials, const uint8_t *d
 // activations (and their scales) shared; 16-byte units are XOR-swizzled with the row so
 // that the 8-byte operand reads spread over the banks.  The extra expert (index n_expert,
 // slot n_used) like in the MXFP4 GEMM.
-// Which tile a layer takes: q8_gemm_columns (dsx_q8_0_rules.hpp).
-// The narrow tile is for few picks per expert, where the kernel only streams weights: its workgroups need a
-// third to two thirds of the LDS, so that three (gate/up) or four (down) of a CU wait for their chunks side by side
-// where the wide tile has two.  A value's terms and their order are those of the wide tile: the same bits.  Measured, us wide /
+// Which tile a layer takes: q8_gemm_columns and q8_gate_up_columns (dsx_q8_0_rules.hpp).
+// The narrow tile is for few picks per expert, where the kernel only streams weights: its workgroups need less
+// LDS, so that three of a CU wait for their chunks side by side where the wide tile has two.  A value's terms and their order are those of the wide tile: the same bits.  Measured, us wide /
 // narrow: down 7168 x 2048, 256 experts, top-8: 100 tokens 871 / 681 (5.7 TB/s); 2048 x 1408, 64 experts, top-6, both
 // products, 64 tokens: 157 / 142, 200: 166 / 152.  There (19 picks per expert) the vector pipe is 31 % busy in gate/up and 25 % in
 // down, the matrix pipe 14 and 10 %.
-// The wide tile with 48 picks per expert (the same layer, 512 tokens): 54 % and 22 % busy in gate/up, 41 % and 16 % in
-// down, whose last round of workgroups (4.25 rounds) is part empty.
-// The middle tile is down's for the picks between, while most experts still make one item of 64: three workgroups per
+// Non-temporal weight loads where a row's quants are whole lines and its group is one item, which then reads every line
+// once: MXFP4 gate/up, 7168 x 2048, 512 tokens 1751 / 1662; 2048 x 1408, 100 tokens 163 / 157.
+// The middle tile is for the picks between, while most experts still make one item of 64: down has three workgroups per
 // CU for the wide tile's two (7168 x 2048, 256 experts, 1000 tokens: the layer 2349 -> 2143 us; four per CU spilled 24
-// registers).  Gate/up of 64 columns would need 54 KB and stay at two per CU.
+// registers), gate/up two of each, with twice the scales at a time and less to request and fold for columns that are not
+// there (2048 x 1408, 64 experts, 512 tokens: the layer 222 -> 212; 4096 x 1536, 128 experts, 768: 804 -> 758).
 // ---------------------------------------------------------------------------------------
 constexpr int kQgWaves = 4;
 
@@ -542,35 +542,50 @@ struct Q8GemmParams {
     const int32_t *group_count, *group_offset, *members, *work_items, *n_work_items;
     uint32_t n_tokens, n_used, n_expert, n_rows, n_blocks, act_row_bytes, n_row_tiles;
     uint32_t chunk;                // members of a work item, up to the tile's columns
+    uint32_t whole_lines;          // every 128-byte piece of a routed row's quants is one cache line
     StreamChoice choice;           // a streaming launch offers the same product
     float clamp, sh_clamp;
 };
 
-// DEPTH buffers of: columns | activation scales | the waves' weight chunks; two of: the rows' block scales of
-// two chunks
-// 64 columns: two buffers, three workgroups per CU (three buffers would not fit three times)
-// 32 columns (narrow): three buffers of down's 13 KB chunks (four workgroups per CU), two of gate/up's 21 KB
-// (three); 128: two (two workgroups per CU)
+// depth buffers of: columns | the waves' weight chunks; two of: activation scales of xu chunks | the rows' block scales of
+// 2 du chunks; per_cu workgroups of a CU side by side.  What binds is requests in flight, not bytes: a load that brings
+// every row or column 16 bytes of scales makes as many requests as one that brings it a whole line.  Scales of one chunk
+// (columns) and two (rows) at a time / as below, us per layer: 2048 x 1408, 64 experts, top-6: 100 tokens 157 / 146, 512: 228
+// / 224; MXFP4 gate/up, 7168 x 2048, 256 experts, 512: 1662 / 1612; scales of one chunk for the rows as well: 184, 233, 1765.
+// More workgroups beat more buffers (down's 64 columns with three buffers, two per CU: 1780 for 1643 at 512 tokens of the
+// mixed layer; gate/up's with three: 187 for 179 at 300 of the small one), except in down's 32 columns (two buffers, four
+// per CU: 154 for 146 at 100 tokens).
+struct Q8GemmTune {
+    int depth;
+    uint32_t xu, du;
+    int per_cu;
+};
 template <bool PAIR, int COLS>
 struct Q8GemmLds {
-    static constexpr int DEPTH = COLS < 64 && !PAIR ? 3 : 2;
+    static constexpr Q8GemmTune kT = COLS == 32 ? (PAIR ? Q8GemmTune{2, 4, 2, 3} : Q8GemmTune{3, 8, 4, 3})
+                                   : COLS == 64 ? (PAIR ? Q8GemmTune{2, 8, 4, 2} : Q8GemmTune{2, 4, 4, 3})
+                                                : (PAIR ? Q8GemmTune{2, 2, 2, 2} : Q8GemmTune{2, 4, 4, 2});
+    static constexpr int DEPTH = kT.depth, kPerCu = kT.per_cu;
+    static constexpr uint32_t XU = kT.xu, DU = kT.du;
     static constexpr uint32_t kM = PAIR ? 2u : 1u;
-    static constexpr uint32_t kB = (uint32_t)COLS * 128u, kXs = (uint32_t)COLS * 16u;
-    static constexpr uint32_t kXsOff = DEPTH * kB, kAOff = kXsOff + DEPTH * kXs;
+    static constexpr uint32_t kB = (uint32_t)COLS * 128u, kXs = (uint32_t)COLS * XU * 16u;   // one buffer
+    static constexpr uint32_t kDw = kM * kQgRows * DU * 16u;
+    static constexpr uint32_t kXsOff = DEPTH * kB, kAOff = kXsOff + 2u * kXs;
     static constexpr uint32_t kAWave = kM * DEPTH * 2048u;   // [matrix][buffer][2 KB]
     static constexpr uint32_t kDwOff = kAOff + kQgWaves * kAWave;
-    static constexpr uint32_t kBytes = kDwOff + 2u * kM * kQgRows * 16u;
+    static constexpr uint32_t kBytes = kDwOff + 2u * kDw;
+    static_assert(kPerCu * ((kBytes + 1279u) / 1280u * 1280u) <= 160u * 1024u, "the workgroups of a CU fit into its LDS");
 };
 
 template <bool PAIR, int COLS>
-__global__ __launch_bounds__(kQgWaves * 64, COLS > 64 ? 2 : PAIR || COLS > 32 ? 3 : 4) void k_q8_0_gemm(const Q8GemmParams p) {
+__global__ __launch_bounds__(kQgWaves * 64, (Q8GemmLds<PAIR, COLS>::kPerCu)) void k_q8_0_gemm(const Q8GemmParams p) {
     constexpr uint32_t M = PAIR ? 2u : 1u;
     using L = Q8GemmLds<PAIR, COLS>;
     constexpr int DEPTH = L::DEPTH;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    __shared__ uint32_t s_dest[COLS];
-    __shared__ uint32_t s_src[COLS];
-    __shared__ float s_ew[COLS];
+    // what the columns are sits in the LDS before the first loads go out, and again when the last chunk has been used
+    uint32_t *s_col = (uint32_t *)smem;
+    float *s_ew = (float *)(smem + COLS * 4);
 
     const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63u;
     const uint32_t g4 = lane >> 4, n16 = lane & 15u;
@@ -598,24 +613,23 @@ __global__ __launch_bounds__(kQgWaves * 64, COLS > 64 ? 2 : PAIR || COLS > 32 ? 
     const uint32_t cnt = min(p.chunk, (uint32_t)p.group_count[e] - start);
     const uint32_t mbase = (uint32_t)p.group_offset[e] + start;
     const bool extra = e >= p.n_expert;
+    uint32_t my_dest = 0;
+    float my_ew = 1.0f;
     if (tid < (uint32_t)COLS) {
         // columns past the end of the group repeat its last member; they are never stored
         const uint32_t m = (uint32_t)p.members[mbase + min(tid, cnt - 1u)];
         const uint32_t t = m >> 16, slot = m & 0xFFFFu;
         const uint32_t dest = slot >= p.n_used ? p.n_tokens * p.n_used + t : t * p.n_used + slot;
-        s_dest[tid] = dest;
-        s_src[tid] = PAIR ? t : dest;
-        if (PAIR) s_ew[tid] = slot >= p.n_used ? 1.0f : p.ew[dest];
+        my_dest = dest;
+        s_col[tid] = PAIR ? t : dest;
+        if (PAIR && slot < p.n_used) my_ew = p.ew[dest];
     }
     const uint32_t nb = p.n_blocks, row_bytes = nb * 34u;
     const uint8_t *wbase[M];
     wbase[0] = (extra ? p.sh_w0 : p.w0 + (uint64_t)e * p.bpe0) + (uint64_t)(rt * kQgRows) * row_bytes;
     if (PAIR) wbase[M - 1] = (extra ? p.sh_w1 : p.w1 + (uint64_t)e * p.bpe1) + (uint64_t)(rt * kQgRows) * row_bytes;
 
-    // the rows' block scales travel with the chunks: 16 bytes per row hold the scales of two chunks
-    // (8 blocks), fetched by one instruction per matrix every other chunk (wave mm: lane -> row)
-    const uint8_t *s_dw = smem + L::kDwOff;   // [buffer][matrix][row][16 B]
-    __syncthreads();  // s_src visible
+    __syncthreads();  // s_col visible
 
     const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
     const uint32_t l8 = lane >> 3, c8 = (lane & 7u) ^ l8;
@@ -628,36 +642,68 @@ __global__ __launch_bounds__(kQgWaves * 64, COLS > 64 ? 2 : PAIR || COLS > 32 ? 
     uint32_t b_fetch[kBLoads];
 #pragma unroll
     for (int ii = 0; ii < kBLoads; ii++)
-        b_fetch[ii] = s_src[wave * (uint32_t)kBLoads * 8u + ii * 8u + l8] * p.act_row_bytes + c8 * 16u;
-    // activation scales: the first waves, lane -> column 64 w + lane, the chunk's 4 floats
-    constexpr uint32_t kXsWaves = COLS > 64 ? 2u : 1u;
-    const uint32_t xs_lds = __builtin_amdgcn_readfirstlane(lds0 + L::kXsOff + (kXsWaves == 2u ? wave & 1u : 0u) * 1024u);
-    const uint32_t dw_lds = __builtin_amdgcn_readfirstlane(lds0 + L::kDwOff);
+        b_fetch[ii] = s_col[wave * (uint32_t)kBLoads * 8u + ii * 8u + l8] * p.act_row_bytes + c8 * 16u;
+    // Scales come in segments of several chunks: a request of 16 bytes per row or column and chunk costs the memory pipe
+    // as much as one of a whole line.  Activation scales: units of 16 bytes (a chunk), XU per column, 64 / XU columns per
+    // load, dealt to the waves; the units of a column swapped so that 16 columns' reads spread over the banks.
+    constexpr uint32_t XU = L::XU, DU = L::DU, kXsCols = 64u / XU;
+    constexpr uint32_t kXsLoads = ((uint32_t)COLS / kXsCols + kQgWaves - 1u) / kQgWaves;   // of a wave
+    const uint32_t xs_lds = __builtin_amdgcn_readfirstlane(lds0 + L::kXsOff + wave * 1024u);
     const uint32_t wave_u = __builtin_amdgcn_readfirstlane(wave);
-    const uint8_t *dw_base = (M == 2u && wave_u == 1u) ? wbase[M - 1] : wbase[0];   // wave mm fetches matrix mm's
-    const uint32_t xs_fetch = s_src[((wave & 1u) * 64u + lane) % (uint32_t)COLS] * p.act_row_bytes + nb * 32u;
+    const uint32_t n_chunks = nb / 4u;
+    uint32_t xs_fetch[kXsLoads], xs_unit = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < kXsLoads; i++) {
+        const uint32_t col = ((i * kQgWaves + wave) * kXsCols + lane / XU) % (uint32_t)COLS;
+        xs_fetch[i] = s_col[col] * p.act_row_bytes + nb * 32u;
+        xs_unit = lane % XU ^ (col % 16u) / (16u / XU) % XU;   // (the same for every load: four loads are whole turns of the swap)
+    }
+    // the rows' block scales: units of 16 bytes (two chunks), DU per row, load q: rows 64 / DU (q % DU) .. of matrix q / DU
+    constexpr uint32_t kDwLoads = (M * DU + kQgWaves - 1u) / kQgWaves;   // of a wave: wave, wave + 4
+    static_assert(kDwLoads == 1u || kQgWaves % DU == 0u, "a wave's loads are the same rows of both matrices");
+    const uint32_t dw_lds = __builtin_amdgcn_readfirstlane(lds0 + L::kDwOff + wave * 1024u);
+    const uint32_t dw_row = (wave % DU) * (64u / DU) + lane / DU, dw_unit = (lane % DU) ^ (dw_row * DU / 16u % DU);
+    const uint32_t dw_fetch = dw_row * row_bytes, dw_last = (n_chunks - 1u) / 2u;
+    const uint32_t dw_live = wave_u < M * DU ? kDwLoads : 0u;
+    const uint8_t *s_dw = smem + L::kDwOff;   // [buffer][matrix][row][unit]
+    __syncthreads();  // s_col has been read
     const bool b_live = wave_u * (uint32_t)kBLoads * 8u < cnt;
+    const uint32_t xs_all = (cnt + kXsCols - 1u) / kXsCols, xs_live = xs_all > wave_u ? (xs_all - wave_u + kQgWaves - 1u) / kQgWaves : 0u;
+    const bool nt = p.whole_lines && !extra && (uint32_t)p.group_count[e] <= p.chunk;   // uniform
     auto issue = [&](uint32_t c, uint32_t buf) {
 #pragma unroll
         for (uint32_t mm = 0; mm < M; mm++)
 #pragma unroll
-            for (int i = 0; i < 2; i++)
-                lds_dma16(a_lds + (mm * DEPTH + buf) * 2048u + (uint32_t)i * 1024u, wbase[mm],
-                          a_fetch + (uint32_t)i * 8u * row_bytes + c * 128u);
+            for (int i = 0; i < 2; i++) {
+                const uint32_t dst = a_lds + (mm * DEPTH + buf) * 2048u + (uint32_t)i * 1024u;
+                const uint32_t src = a_fetch + (uint32_t)i * 8u * row_bytes + c * 128u;
+                if (nt) lds_dma16<true>(dst, wbase[mm], src);
+                else lds_dma16(dst, wbase[mm], src);
+            }
         if (b_live) {
 #pragma unroll
             for (int ii = 0; ii < kBLoads; ii++)
                 lds_dma16(b_lds + buf * L::kB + (uint32_t)ii * 1024u, p.act, b_fetch[ii] + c * 128u);
         }
-        if (wave_u < kXsWaves && (COLS >= 64 || lane < (uint32_t)COLS)) lds_dma16(xs_lds + buf * L::kXs, p.act, xs_fetch + c * 16u);
-        // (a last, single chunk reads 8 bytes past the scales, into the row's own quants)
-        if ((c & 1u) == 0u && wave_u < M)
-            lds_dma16(dw_lds + ((c >> 1) & 1u) * (M * kQgRows * 16u) + wave_u * (kQgRows * 16u), dw_base,
-                      lane * row_bytes + (c >> 1) * 16u);
+        if (c % XU == 0u) {
+#pragma unroll
+            for (uint32_t i = 0; i < kXsLoads; i++)
+                if (i < xs_live)   // (units past the row's end repeat its last one)
+                    lds_dma16(xs_lds + (c / XU & 1u) * L::kXs + i * (kQgWaves * 1024u), p.act, xs_fetch[i] + min(c + xs_unit, n_chunks - 1u) * 16u);
+        }
+        // (the last unit of an odd number of chunks reads 8 bytes past the scales, into the row's own quants)
+        if (c % (2u * DU) == 0u && dw_live) {
+#pragma unroll
+            for (uint32_t i = 0; i < kDwLoads; i++)
+                lds_dma16(dw_lds + (c / (2u * DU) & 1u) * L::kDw + i * (kQgWaves * 1024u),
+                          M == 2u && wave_u + i * kQgWaves >= DU ? wbase[M - 1] : wbase[0], dw_fetch + min(c / 2u + dw_unit, dw_last) * 16u);
+        }
     };
 
-    // the wave's loads of a chunk, without the block scales of the even ones
-    const uint32_t my_loads = 2u * M + (b_live ? (uint32_t)kBLoads : 0u) + (wave_u < kXsWaves ? 1u : 0u);
+    // the wave's loads of a chunk
+    auto loads_of = [&](uint32_t c) {
+        return 2u * M + (b_live ? (uint32_t)kBLoads : 0u) + (c % XU == 0u ? xs_live : 0u) + (c % (2u * DU) == 0u ? dw_live : 0u);
+    };
 
     // read side: lane (row / column n16, 8-byte piece g4 of a block's 32 bytes)
     const uint32_t rd = (n16 >> 3) * 1024u + (n16 & 7u) * 128u + (g4 & 1u) * 8u;
@@ -672,7 +718,6 @@ __global__ __launch_bounds__(kQgWaves * 64, COLS > 64 ? 2 : PAIR || COLS > 32 ? 
 #pragma unroll
             for (int q = 0; q < 4; q++) acc[mm][j][q] = 0.0f;
 
-    const uint32_t n_chunks = nb / 4u;
     const uint32_t nj = (cnt + 15u) / 16u;
     for (uint32_t c = 0; c + 1u < DEPTH; c++)
         if (c < n_chunks) issue(c, c);
@@ -681,19 +726,20 @@ __global__ __launch_bounds__(kQgWaves * 64, COLS > 64 ? 2 : PAIR || COLS > 32 ? 
         // the chunk has landed; the DEPTH - 2 behind it may be under way.  Behind the barrier it has for every
         // wave, and nobody reads chunk c - 1, whose buffer the next request fills
         if constexpr (DEPTH == 2) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        else wait_vm(c + 1u < n_chunks ? my_loads + (wave_u < M ? (c & 1u) : 0u) : 0u);
+        else wait_vm(c + 1u < n_chunks ? loads_of(c + 1u) : 0u);
         static_assert(DEPTH <= 3, "one chunk behind the awaited one");
         __syncthreads();
         if (c + DEPTH - 1u < n_chunks) issue(c + DEPTH - 1u, next);
         const uint8_t *bb = smem + buf * L::kB;
-        const uint8_t *xb = smem + L::kXsOff + buf * L::kXs;
+        const uint8_t *xb = smem + L::kXsOff + (c / XU & 1u) * L::kXs + ((c % XU) ^ n16 / (16u / XU) % XU) * 16u;
         // row n16's scale of block g4, and its A operands of the chunk's 4 blocks
         float dw[M];
         long av[M][4];
 #pragma unroll
         for (uint32_t mm = 0; mm < M; mm++) {
-            dw[mm] = __half2float(__ushort_as_half(*(const uint16_t *)(
-                s_dw + ((size_t)((c >> 1) & 1u) * M + mm) * (kQgRows * 16u) + (size_t)(wave * 16u + n16) * 16u + (c & 1u) * 8u + g4 * 2u)));
+            const uint32_t dw_at = (c / (2u * DU) & 1u) * L::kDw + (mm * kQgRows + wave * 16u + n16) * (DU * 16u) +
+                                   ((c / 2u % DU) ^ (n16 * DU / 16u % DU)) * 16u + (c & 1u) * 8u + g4 * 2u;
+            dw[mm] = __half2float(__ushort_as_half(*(const uint16_t *)(s_dw + dw_at)));
             const uint8_t *ab = a_ptr + (mm * DEPTH + buf) * 2048u;
 #pragma unroll
             for (int b = 0; b < 4; b++)
@@ -705,7 +751,7 @@ __global__ __launch_bounds__(kQgWaves * 64, COLS > 64 ? 2 : PAIR || COLS > 32 ? 
             const uint8_t *bj = bb + (size_t)j * 2048u + rd;
 #pragma unroll
             for (int b = 0; b < 4; b++) bv[b] = *(const long *)(bj + (((uint32_t)(2 * b) + rd_unit) ^ rd_sw) * 16u);
-            xs = *(const float *)(xb + (size_t)((uint32_t)j * 16u + n16) * 16u + g4 * 4u);
+            xs = *(const float *)(xb + (size_t)((uint32_t)j * 16u + n16) * (XU * 16u) + g4 * 4u);
         };
         auto step = [&](auto groups) __attribute__((always_inline)) {
             constexpr int kFrags = (int)M * decltype(groups)::value;
@@ -755,13 +801,19 @@ __global__ __launch_bounds__(kQgWaves * 64, COLS > 64 ? 2 : PAIR || COLS > 32 ? 
         next = next + 1u == DEPTH ? 0u : next + 1u;
     }
 
+    __syncthreads();  // the last chunk has been used
+    if (tid < (uint32_t)COLS) {
+        s_col[tid] = my_dest;
+        if (PAIR) s_ew[tid] = my_ew;
+    }
+    __syncthreads();
     // the lane holds rows 16 w + 4 g4 + q of columns 16 j + n16
     const float clamp = extra ? p.sh_clamp : p.clamp;
 #pragma unroll
     for (int j = 0; j < COLS / 16; j++) {
         const uint32_t col = j * 16u + n16;
         if (col >= cnt) continue;
-        float *dst = p.out + (uint64_t)s_dest[col] * p.n_rows + rt * kQgRows + wave * 16u + g4 * 4u;
+        float *dst = p.out + (uint64_t)s_col[col] * p.n_rows + rt * kQgRows + wave * 16u + g4 * 4u;
         if (PAIR) {
             const float ew = s_ew[col];
             *(float4 *)dst = make_float4(swiglu_clamp(acc[0][j][0], acc[M - 1][j][0], clamp, ew),
@@ -778,19 +830,22 @@ __global__ __launch_bounds__(kQgWaves * 64, COLS > 64 ? 2 : PAIR || COLS > 32 ? 
 inline void q8_0_gemm_raise_lds_limits() {
     (void)hipFuncSetAttribute((const void *)k_q8_0_gemm<true, kQgCols>, hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
     (void)hipFuncSetAttribute((const void *)k_q8_0_gemm<false, kQgCols>, hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
+    (void)hipFuncSetAttribute((const void *)k_q8_0_gemm<true, kQgColsMiddle>, hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
     (void)hipFuncSetAttribute((const void *)k_q8_0_gemm<false, kQgColsMiddle>, hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
     (void)hipFuncSetAttribute((const void *)k_q8_0_gemm<true, kQgColsNarrow>, hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
     (void)hipFuncSetAttribute((const void *)k_q8_0_gemm<false, kQgColsNarrow>, hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
 }
 
 template <bool PAIR, int COLS>
-inline int q8_0_gemm_launch(hipStream_t st, const Q8GemmParams &p, uint32_t max_wi) {
+inline int q8_0_gemm_launch(hipStream_t st, Q8GemmParams p, uint32_t max_wi) {
     if (max_wi == 0) return DSX_OK;
     if (p.n_rows % kQgRows || p.n_blocks % 4 || p.n_blocks == 0)
         return q8_0_fail(DSX_ERR_SHAPE, "q8_0 gemm", "n_rows must be a multiple of 64, k of 128");
     const uint64_t act_rows = (uint64_t)p.n_tokens * (p.n_used + 1u);
     if ((uint64_t)p.n_rows * p.n_blocks * 34u > 0xFFFFFFFFull || act_rows * p.act_row_bytes > 0xFFFFFFFFull)
         return q8_0_fail(DSX_ERR_INVALID_ARG, "q8_0 gemm", "a weight matrix or the activation rows exceed 4 GiB");
+    p.whole_lines = p.n_blocks % 64u == 0u && p.bpe0 % 128u == 0u && (uintptr_t)p.w0 % 128u == 0u &&
+                    (!PAIR || (p.bpe1 % 128u == 0u && (uintptr_t)p.w1 % 128u == 0u));
     const size_t lds = Q8GemmLds<PAIR, COLS>::kBytes;
     const uint32_t per_xcd = (max_wi + 7u) / 8u;
     const uint64_t grid = (uint64_t)8u * per_xcd * p.n_row_tiles;
@@ -804,8 +859,7 @@ inline int q8_0_gemm_launch(hipStream_t st, const Q8GemmParams &p, uint32_t max_
 template <bool PAIR>
 inline int q8_0_gemm(hipStream_t st, const Q8GemmParams &p, uint32_t max_wi) {
     if (p.chunk <= (uint32_t)kQgColsNarrow) return q8_0_gemm_launch<PAIR, kQgColsNarrow>(st, p, max_wi);
-    if constexpr (!PAIR)
-        if (p.chunk <= (uint32_t)kQgColsMiddle) return q8_0_gemm_launch<PAIR, kQgColsMiddle>(st, p, max_wi);
+    if (p.chunk <= (uint32_t)kQgColsMiddle) return q8_0_gemm_launch<PAIR, kQgColsMiddle>(st, p, max_wi);
     return q8_0_gemm_launch<PAIR, kQgCols>(st, p, max_wi);
 }
 

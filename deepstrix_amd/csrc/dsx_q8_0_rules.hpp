@@ -9,7 +9,7 @@ namespace dsx {
 
 constexpr uint32_t kQ8StreamMembers = 16;   // members of a streaming work item (dsx_stream_kernels.hpp)
 // columns of the int8 GEMM's tiles (k_q8_0_gemm), rows of them all
-constexpr uint32_t kQgCols = 128, kQgColsMiddle = 64 /* down only */, kQgColsNarrow = 32, kQgRows = 64;
+constexpr uint32_t kQgCols = 128, kQgColsMiddle = 64, kQgColsNarrow = 32, kQgRows = 64;
 
 struct Q8Shape {
     uint32_t hidden, inter, n_expert, n_used;
@@ -69,6 +69,18 @@ inline uint32_t q8_gemm_columns(const Q8Shape &s, uint32_t T, uint32_t n_cu) {
     const uint32_t narrow = s.n_expert <= 16u && workgroups < 3u * n_cu ? 84u : 56u;
     if ((T <= 256u || s.elements() <= (2ull << 20)) && s.picks_below_halves(T, narrow)) return kQgColsNarrow;
     return s.picks_below_halves(T, workgroups >= 24u * n_cu ? 112u : 84u) ? kQgColsMiddle : kQgCols;
+}
+
+// The same for gate/up of an all-Q8_0 layer whose down product has `down` columns by the above; down takes no more than
+// gate/up.  64 between the narrow tile's end and 60 picks per expert, where experts begin to make two items (us per layer, gate/up
+// and down in 128 and 64 or 128 columns, the better of the two / both in 64: 2048 x 1408, 64 experts, top-6: 300 tokens
+// [28 picks] 187 / 179, 512 [48] 222 / 212, 600 [56] 243 / 240, 700 [66] 267 / 284; 4096 x 1536, 128, top-8: 400 [25] 617 /
+// 605, 768 [48] 804 / 758, 900 [56] 884 / 846, 1200 [75] 1021 / 1198; 3072 x 2048, 64, top-4: 450 [28] 345 / 339, 900 [56] 525 /
+// 468, 1100 [69] 604 / 591; 2048 x 768, 128, top-8: 512 [32] 205 / 200, 900 [56] 272 / 259, 1200 [75] 319 / 350; 1024 x 2048,
+// 32, top-4: 300 [38] 102 / 92, 600 [75] 144 / 147; 4096 x 14336, 8, top-2: 192 [48] 835 / 664; 7168 x 2048, 256, top-8: 1000 [31]
+// 3124 / 2835, 2000 [63] 4352 / 4284).
+inline uint32_t q8_gate_up_columns(const Q8Shape &s, uint32_t T, uint32_t down) {
+    return down == kQgColsNarrow ? down : s.picks_below_halves(T, 120u) ? kQgColsMiddle : kQgCols;
 }
 
 // Columns per work item of a dense Q8_0 expert of b tokens (dsx_dense_ffn; both products, one list): 32 where the wide

@@ -1,5 +1,5 @@
 // Prints what the size rules of csrc/dsx_q8_0_rules.hpp say, one answer per line of stdin (CPU; driven by
-// tests/test_q8_0_rules.py): "gemm hidden inter n_expert n_used tokens cus" and "dense hidden inter 0 0 tokens cus" ->
+// tests/test_q8_0_rules.py): "gemm hidden inter n_expert n_used tokens cus", "gate_up ..." and "dense hidden inter 0 0 tokens cus" ->
 // columns per work item.
 #include <cstdio>
 #include <cstring>
@@ -11,7 +11,10 @@ int main() {
     unsigned v[6];
     while (std::scanf("%15s %u %u %u %u %u %u", what, &v[0], &v[1], &v[2], &v[3], &v[4], &v[5]) == 7) {
         if (std::strcmp(what, "gemm") == 0) std::printf("%u\n", dsx::q8_gemm_columns({v[0], v[1], v[2], v[3]}, v[4], v[5]));
-        else if (std::strcmp(what, "dense") == 0) std::printf("%u\n", dsx::q8_dense_columns(v[0], v[1], v[4], v[5]));
+        else if (std::strcmp(what, "gate_up") == 0) {
+            const dsx::Q8Shape s{v[0], v[1], v[2], v[3]};
+            std::printf("%u\n", dsx::q8_gate_up_columns(s, v[4], dsx::q8_gemm_columns(s, v[4], v[5])));
+        } else if (std::strcmp(what, "dense") == 0) std::printf("%u\n", dsx::q8_dense_columns(v[0], v[1], v[4], v[5]));
         else return 1;
     }
     return 0;

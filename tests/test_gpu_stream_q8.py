@@ -189,6 +189,16 @@ def test_middle_tile_of_the_down_gemm_matches_the_oracle(monkeypatch, down_fmt, 
         assert torch.equal(out, old)
 
 
+@pytest.mark.parametrize("hidden,inter", [(128, 1152), (640, 128), (1152, 640), (2048, 1408)])
+@pytest.mark.parametrize("T", [168, 201, 239])
+def test_middle_tile_of_both_products_matches_the_oracle(monkeypatch, hidden, inter, T):
+    """42 to 60 picks per expert: gate/up by 64-column items as well, on rows of 1 to 16 chunks, whose scales come by segments of
+    eight with a last one of 1 to 8; the wide tile's bits."""
+    s = H.Shape(hidden, inter, 8, 2, FMT_Q8_0, FMT_Q8_0, shared=T != 201, seed=846, **ROUTER)
+    out, old, _ = _run(s, T, T, monkeypatch)
+    assert torch.equal(out, old)
+
+
 def test_middle_tile_on_many_workgroups(monkeypatch):
     """48 picks per expert and enough row tiles for many rounds: the middle tile again, the wide one's bits."""
     monkeypatch.setattr(MoeLayer, "v3_thresholds_below_experts", None)

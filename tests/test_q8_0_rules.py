@@ -35,6 +35,14 @@ def test_columns_of_the_int8_gemm(shape, columns):
 
 
 @pytest.mark.parametrize("shape,columns", [
+    ((7168, 2048, 256, 8), {256: 32, 512: 64, 1000: 64, 1900: 64, 2000: 128}),
+    ((2048, 1408, 64, 6), {200: 32, 300: 64, 512: 64, 600: 64, 700: 128}),
+    ((4096, 14336, 8, 2), {128: 32, 192: 64, 300: 128})])
+def test_gate_up_columns_of_the_int8_gemm(shape, columns):
+    assert dict(zip(columns, ask([("gate_up", *shape, T, CUS) for T in columns]))) == columns
+
+
+@pytest.mark.parametrize("shape,columns", [
     ((7168, 2048), {96: 32, 768: 32, 1000: 128, 1900: 128, 2000: 128}),
     ((7168, 3072), {512: 32, 640: 32, 1000: 128}),
     ((5120, 1536), {1500: 32, 1900: 128}),
