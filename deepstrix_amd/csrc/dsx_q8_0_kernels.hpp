@@ -577,8 +577,9 @@ struct Q8GemmLds {
     static_assert(kPerCu * ((kBytes + 1279u) / 1280u * 1280u) <= 160u * 1024u, "the workgroups of a CU fit into its LDS");
 };
 
+// 64 rows (tile rt) of the work item of `cnt` members of expert e, the first of them members[mbase].
 template <bool PAIR, int COLS>
-__global__ __launch_bounds__(kQgWaves * 64, (Q8GemmLds<PAIR, COLS>::kPerCu)) void k_q8_0_gemm(const Q8GemmParams p) {
+__device__ __forceinline__ void q8_0_gemm_tile(const Q8GemmParams &p, const uint32_t e, const uint32_t cnt, const uint32_t mbase, const uint32_t rt) {
     constexpr uint32_t M = PAIR ? 2u : 1u;
     using L = Q8GemmLds<PAIR, COLS>;
     constexpr int DEPTH = L::DEPTH;
@@ -589,29 +590,6 @@ __global__ __launch_bounds__(kQgWaves * 64, (Q8GemmLds<PAIR, COLS>::kPerCu)) voi
 
     const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63u;
     const uint32_t g4 = lane >> 4, n16 = lane & 15u;
-
-    if (COLS == kQgColsNarrow && p.choice.offered() && p.choice.streams()) return;   // uniform
-
-    // the row tiles of a work item run on one XCD (they share the activations in its L2); the
-    // items are dealt to the XCDs like cards, which spreads the wide groups of skewed routing
-    const uint32_t xcd = blockIdx.x & 7u, seq = blockIdx.x >> 3;
-    const uint32_t n_items = (uint32_t)*p.n_work_items;  // the grid is only an upper bound
-    const uint32_t local = seq / p.n_row_tiles;
-    // Many column tiles per expert (skewed routing, many tokens): the items are dealt to the XCDs
-    // like cards, which spreads the wide groups -- contiguous ranges of the list (it is by expert)
-    // left the busiest XCD with 17 % more column groups than the average at Zipf-skewed routing,
-    // against 8 % (layer at T=4096: -4.6 %).  About a tile per expert: contiguous ranges, so that
-    // an XCD streams one contiguous stretch of the weights (3-5 % faster then).
-    const bool deal = n_items > p.n_expert + (p.n_expert >> 1);
-    if (!deal && local >= (n_items + 7u) / 8u) return;  // uniform
-    const uint32_t item = deal ? local * 8u + xcd : xcd * ((n_items + 7u) / 8u) + local;
-    const uint32_t rt = seq % p.n_row_tiles;
-    if (item >= n_items) return;
-
-    const uint32_t wi = (uint32_t)p.work_items[item];
-    const uint32_t e = wi >> 16, start = wi & 0xFFFFu;
-    const uint32_t cnt = min(p.chunk, (uint32_t)p.group_count[e] - start);
-    const uint32_t mbase = (uint32_t)p.group_offset[e] + start;
     const bool extra = e >= p.n_expert;
     uint32_t my_dest = 0;
     float my_ew = 1.0f;
@@ -826,6 +804,49 @@ __global__ __launch_bounds__(kQgWaves * 64, (Q8GemmLds<PAIR, COLS>::kPerCu)) voi
     }
 }
 
+// The middle tile's launch computes items of up to 32 members as the narrow tile does, which has one chunk more under way (MXFP4
+// gate/up, 7168 x 2048, 256 experts, uniform picks, us, 64 columns / both: 512 tokens 1621 / 1600, 700: 1734 / 1706, 1000: 2134 / 2082).
+template <bool PAIR, int COLS>
+constexpr bool q8_gemm_both = !PAIR && COLS == kQgColsMiddle;
+template <bool PAIR, int COLS>
+constexpr uint32_t q8_gemm_lds_bytes() {
+    return q8_gemm_both<PAIR, COLS> ? std::max(Q8GemmLds<PAIR, COLS>::kBytes, Q8GemmLds<PAIR, kQgColsNarrow>::kBytes) : Q8GemmLds<PAIR, COLS>::kBytes;
+}
+
+template <bool PAIR, int COLS>
+__global__ __launch_bounds__(kQgWaves * 64, (Q8GemmLds<PAIR, COLS>::kPerCu)) void k_q8_0_gemm(const Q8GemmParams p) {
+    if (COLS == kQgColsNarrow && p.choice.offered() && p.choice.streams()) return;   // uniform
+
+    // the row tiles of a work item run on one XCD (they share the activations in its L2); the
+    // items are dealt to the XCDs like cards, which spreads the wide groups of skewed routing
+    const uint32_t xcd = blockIdx.x & 7u, seq = blockIdx.x >> 3;
+    const uint32_t n_items = (uint32_t)*p.n_work_items;  // the grid is only an upper bound
+    const uint32_t local = seq / p.n_row_tiles;
+    // Many column tiles per expert (skewed routing, many tokens): the items are dealt to the XCDs
+    // like cards, which spreads the wide groups -- contiguous ranges of the list (it is by expert)
+    // left the busiest XCD with 17 % more column groups than the average at Zipf-skewed routing,
+    // against 8 % (layer at T=4096: -4.6 %).  About a tile per expert: contiguous ranges, so that
+    // an XCD streams one contiguous stretch of the weights (3-5 % faster then).
+    const bool deal = n_items > p.n_expert + (p.n_expert >> 1);
+    if (!deal && local >= (n_items + 7u) / 8u) return;  // uniform
+    const uint32_t item = deal ? local * 8u + xcd : xcd * ((n_items + 7u) / 8u) + local;
+    const uint32_t rt = seq % p.n_row_tiles;
+    if (item >= n_items) return;
+
+    const uint32_t wi = (uint32_t)p.work_items[item];
+    const uint32_t e = wi >> 16, start = wi & 0xFFFFu;
+    const uint32_t cnt = min(p.chunk, (uint32_t)p.group_count[e] - start);
+    const uint32_t mbase = (uint32_t)p.group_offset[e] + start;
+    if constexpr (q8_gemm_both<PAIR, COLS>) {
+        static_assert(Q8GemmLds<PAIR, COLS>::kPerCu == Q8GemmLds<PAIR, kQgColsNarrow>::kPerCu, "as many workgroups of a CU for either tile");
+        if (cnt <= kQgColsNarrow) {   // uniform
+            q8_0_gemm_tile<PAIR, kQgColsNarrow>(p, e, cnt, mbase, rt);
+            return;
+        }
+    }
+    q8_0_gemm_tile<PAIR, COLS>(p, e, cnt, mbase, rt);
+}
+
 // Raised once per device by the library's set-up, with the device current.
 inline void q8_0_gemm_raise_lds_limits() {
     (void)hipFuncSetAttribute((const void *)k_q8_0_gemm<true, kQgCols>, hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
@@ -846,7 +867,7 @@ inline int q8_0_gemm_launch(hipStream_t st, Q8GemmParams p, uint32_t max_wi) {
         return q8_0_fail(DSX_ERR_INVALID_ARG, "q8_0 gemm", "a weight matrix or the activation rows exceed 4 GiB");
     p.whole_lines = p.n_blocks % 64u == 0u && p.bpe0 % 128u == 0u && (uintptr_t)p.w0 % 128u == 0u &&
                     (!PAIR || (p.bpe1 % 128u == 0u && (uintptr_t)p.w1 % 128u == 0u));
-    const size_t lds = Q8GemmLds<PAIR, COLS>::kBytes;
+    const size_t lds = q8_gemm_lds_bytes<PAIR, COLS>();
     const uint32_t per_xcd = (max_wi + 7u) / 8u;
     const uint64_t grid = (uint64_t)8u * per_xcd * p.n_row_tiles;
     if (grid > 0x7FFFFFFFull) return q8_0_fail(DSX_ERR_INVALID_ARG, "q8_0 gemm", "grid too large");
