@@ -197,6 +197,14 @@ __device__ __forceinline__ void lds_dma16(uint32_t lds_addr, const void *base, u
         asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2"
                      :: "s"(lds_addr), "v"(off), "s"(base) : "memory");
 }
+// The same with the kind of load told by a uniform value at run time (the branch is the instruction sequence's own: in code
+// that the compiler schedules, a branch of its own would be the end of a block).
+__device__ __forceinline__ void lds_dma16_if_nt(uint32_t lds_addr, const void *base, uint32_t off, uint32_t nt) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_cmp_lg_u32 %3, 0\n\ts_cbranch_scc1 .Ldma_nt_%=\n\t"
+                 "global_load_lds_dwordx4 %1, %2\n\ts_branch .Ldma_end_%=\n"
+                 ".Ldma_nt_%=:\n\tglobal_load_lds_dwordx4 %1, %2 nt\n.Ldma_end_%=:"
+                 :: "s"(lds_addr), "v"(off), "s"(base), "s"(nt) : "memory", "scc");
+}
 __device__ __forceinline__ void lds_dma4(uint32_t lds_addr, const void *base, uint32_t off) {
     asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, %2"
                  :: "s"(lds_addr), "v"(off), "s"(base) : "memory");

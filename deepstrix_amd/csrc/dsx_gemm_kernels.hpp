@@ -256,12 +256,20 @@ __global__ __launch_bounds__(kGemmWaves * 64, MT == kGemmMT ? 2 : 4) void k_mxfp
     // of scales, private to the wave (no barrier).  B: the 128 columns' 192 B of half a
     // super-block, shared, double buffered; wave w fetches columns 16 w .. 16 w + 15.
     constexpr int kALoads = 4 * kGemmRF + 2;  // per wave and super-block
+    // whether the group has no other tile (arithmetic on scalars and opaque: a truth value would end up in a vector register)
+    uint32_t one_tile = 0u;
+    if constexpr (PLANAR && MT == kGemmMT) {
+        one_tile = (uint32_t)__builtin_amdgcn_readfirstlane(p.group_count[e] - MT - 1) >> 31;
+        asm volatile("" : "+s"(one_tile));
+    }
     // load L of those: 0..7 the halves of the four fragments, 8 and 9 the scales of the row sets
     // (row runs: loads 0..4 the first row set, 5..9 the second)
-    // NT: non-temporal loads.  Planar weights in the narrow tile of a group that has no other: every line is then fetched
+    // NT: non-temporal loads.  Planar weights of a group that has no other tile: every line is then fetched
     // once and whole (7168 x 2048, 256 experts, layer us without / with: 16 tokens 473 / 429, 100: 1033 / 960, 200: 1105 /
     // 1077; 4096 x 1024, 128 experts, 37: 168 / 147).  Groups of several tiles find each other's lines in the L2 (400
     // tokens, with such loads throughout: 1240 / 1290), the engine's rows their neighbours' (4096 tokens 3095 / 4085).
+    // The wide tile tells the two apart at run time, load by load: 7168 x 2048, 500 tokens 1243 / 1228, 777: 1404 / 1349, Zipf-skewed
+    // 2900: 2202 / 2165; 4096 x 1024, 500: 300 / 283; 2048 x 1536, 64 experts, 700: 166 / 160.
     auto issue_a_one = [&](auto ntc, int L, uint32_t sb) __attribute__((always_inline)) {
         constexpr bool NT = decltype(ntc)::value;
         if constexpr (kRun) {
@@ -269,8 +277,10 @@ __global__ __launch_bounds__(kGemmWaves * 64, MT == kGemmMT ? 2 : 4) void k_mxfp
             lds_dma16(a_lds + (uint32_t)(m * 5120 + i * 1024), wbase[m] + (a_slab[0][m] + sb * kStepW), run_off[i]);
         } else if (L < 4 * kGemmRF) {
             const int f = L >> 1, i = L & 1, r = f >> 1, m = f & 1;
-            lds_dma16<NT>(a_lds + (uint32_t)(f * 2048 + i * 1024),
-                      wbase[m] + (a_slab[r][m] + (uint32_t)i * 8u * row_stride + sb * kStepW), a_fetch);
+            const uint32_t dst = a_lds + (uint32_t)(f * 2048 + i * 1024);
+            const uint8_t *src = wbase[m] + (a_slab[r][m] + (uint32_t)i * 8u * row_stride + sb * kStepW);
+            if constexpr (PLANAR && MT == kGemmMT) lds_dma16_if_nt(dst, src, a_fetch, one_tile);
+            else lds_dma16<NT>(dst, src, a_fetch);
         } else {
             const int m = L - 4 * kGemmRF;
             lds_dma4(a_lds + kScaleOff + (uint32_t)m * 256u, wbase[m] + (a_slab[0][m] + sb * kStepW), sc_fetch);
