@@ -518,11 +518,10 @@ inline int q8_0_down_by_expert(hipStream_t st, float *partials, const uint8_t *d
 // that the 8-byte operand reads spread over the banks.  The extra expert (index n_expert,
 // slot n_used) like in the MXFP4 GEMM.
 // Which tile a layer takes: q8_gemm_columns and q8_gate_up_columns (dsx_q8_0_rules.hpp).
-// The narrow tile is for few picks per expert, where the kernel only streams weights: its workgroups need less
-// LDS, so that three of a CU wait for their chunks side by side where the wide tile has two.  A value's terms and their order are those of the wide tile: the same bits.  Measured, us wide /
-// narrow: down 7168 x 2048, 256 experts, top-8: 100 tokens 871 / 681 (5.7 TB/s); 2048 x 1408, 64 experts, top-6, both
-// products, 64 tokens: 157 / 142, 200: 166 / 152.  There (19 picks per expert) the vector pipe is 31 % busy in gate/up and 25 % in
-// down, the matrix pipe 14 and 10 %.
+// The narrow tile is for few picks per expert, where the kernel only streams weights: its workgroups need less LDS, so
+// that three of a CU wait for their chunks side by side where the wide tile has two.  A value's terms and their order
+// are those of the wide tile: the same bits.  Measured, us, wide / narrow: down 7168 x 2048, 256 experts, top-8: 100 tokens
+// 871 / 681; both products, 2048 x 1408, 64 experts, top-6: layer of 64 tokens 160 / 142, 200: 178 / 160.
 // Non-temporal weight loads where a row's quants are whole lines and its group is one item, which then reads every line
 // once: MXFP4 gate/up, 7168 x 2048, 512 tokens 1751 / 1662; 2048 x 1408, 100 tokens 163 / 157.
 // The middle tile is for the picks between, while most experts still make one item of 64: down has three workgroups per

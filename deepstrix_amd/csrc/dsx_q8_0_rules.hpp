@@ -2,6 +2,8 @@
 //
 // Figures: us, on one MI355X; old: the by-expert kernels below 1.5 picks per expert and the 128-column int8 GEMM from there
 // on, before these rules (that GEMM 3 to 12 % slower than it is now).  "same picks": every token names the same experts.
+// Taken with the int8 GEMM of that time, 2 to 10 % slower in all tiles than since its scales come in segments (k_q8_0_gemm), but
+// for q8_gate_up_columns.
 #pragma once
 #include <stdint.h>
 

@@ -313,7 +313,8 @@ void dsx_moe_layer_destroy(dsx_moe_layer *layer);
 /* No counterpart in the reference: rewrites every MXFP4 tensor the layer was created with -- the
  * caller's weight buffers -- in place into the planar form (DSX_FMT_MXFP4_PLANAR above), or back
  * into the engine's rows, and switches the layer over (its default thresholds included: a planar
- * layer leaves the decode path at 12 tokens and starts with the 16-column GEMM tile).  A layer
+ * layer leaves the decode path at 0.24 picks per expert [8 tokens at 256 experts, top-8], 0.375 where a matrix has at most
+ * 12 M elements, and starts with the 16-column GEMM tile).  A layer
  * without MXFP4 tensors, or one already in the form asked for, is left as it is.  Shapes are
  * checked before the first byte moves; MXFP4 tensors whose byte ranges overlap are refused.
  * The rewrite is enqueued on `stream` like a kernel launch, while the layer switches over on the
@@ -342,6 +343,7 @@ int dsx_moe_layer_set_profile_events(dsx_moe_layer *layer, void *gate_up_begin, 
  * does, below gemm_min_tokens, and the int8 GEMMs behind the streaming ranges have 32 columns per work item up to 28 picks
  * per expert and 256 tokens (any number where a matrix has up to 2 M elements), and (down) 64 up to 42, or up to 56 where
  * n_expert * hidden / 64 is at least 24 times the CUs; on up to 16 experts, where it is below 3 times the CUs, 32 up to 42.
+ * Gate/up of an all-Q8_0 layer, and down with it, has 64 behind the 32 up to 60 picks per expert.
  * by_expert_chunk (1..16): token columns per work item of the small-batch by-expert path.
  * gemm_min_tokens (default for an all-MXFP4 layer: 3.5 picks per expert [112 tokens], 7 where
  * n_expert * inter / 256 < 512; MXFP4 gate/up with a Q8_0 down matrix 2 [64], 4 for
