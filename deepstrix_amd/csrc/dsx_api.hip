@@ -695,7 +695,7 @@ static int reduce_impl(hipStream_t st, float *out, const float *partials, const 
         (add && !aligned(add, 16)) || (residual && !aligned(residual, 16)))
         return fail(DSX_ERR_SHAPE, "moe_reduce_partials: n_rows=%u must be a multiple of 4, buffers 16-byte aligned", n_rows);
     const uint64_t n4 = (uint64_t)b * (n_rows / 4);
-    hipLaunchKernelGGL(k_reduce_partials, dim3((uint32_t)((n4 + 255) / 256)), dim3(256), 0, st, out,
+    hipLaunchKernelGGL(n_used > 2u ? k_reduce_partials<true> : k_reduce_partials<false>, dim3((uint32_t)((n4 + 255) / 256)), dim3(256), 0, st, out,
                        partials, selected, add, residual, n_used, n_rows, b, hc);
     return launched("moe_reduce_partials");
 }

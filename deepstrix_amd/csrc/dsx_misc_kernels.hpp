@@ -836,8 +836,12 @@ __global__ __launch_bounds__(kGbThreads) void k_group_tables(
 // `residual` (nullable, may be `out`).
 // ---------------------------------------------------------------------------------------
 // `hc` (n_hc != 0): the sum is not stored but goes through the hyper-connection combine.
-// Bound by the partial rows, which are read here for the last time: non-temporal loads (7168 x 2048, top-8, 4096 tokens,
-// layer: 3132 / 3110 us).
+// Bound by the partial rows, whose loads go out together, those of the slots that are there and no others.  us, every load waited
+// for / a clamped row for every slot of the eight that is not there / this: 7168 columns, 512 tokens, top-4: 15.6 / 17.2 /
+// 13.9, top-8: 27.2 / 24.1 / 24.1, half of the slots empty: 18.8 / 24.1 / 14.9; 4096 tokens, top-2: 63 / 84 / 54, top-6: 151 /
+// 135 / 129.  NT: the rows are read here for the last time, but one or two of a token are still in the caches (512 tokens,
+// one row, ordinary / non-temporal: 6.7 / 8.2; two: 8.8 / 9.9).
+template <bool NT>
 __global__ __launch_bounds__(256) void k_reduce_partials(float *out, const float *__restrict__ partials,
                                                          const int32_t *__restrict__ selected,
                                                          const float *__restrict__ add, const float *residual,
@@ -847,26 +851,32 @@ __global__ __launch_bounds__(256) void k_reduce_partials(float *out, const float
     const uint64_t per_row = n_rows / 4u;
     if (i >= (uint64_t)b * per_row) return;
     const uint64_t t = i / per_row, c = i - t * per_row;
-    // eight slots at a time, all of their loads ahead of the sums (an empty slot's row is read and not added)
+    // eight slots at a time: their picks, then the rows of those that are there, then the sums
     constexpr uint32_t kAhead = 8;
     float4 acc = {0.f, 0.f, 0.f, 0.f};
     const float *rows = partials + t * n_used * n_rows + c * 4u;
     for (uint32_t s0 = 0; s0 < n_used; s0 += kAhead) {
         v4f v[kAhead];
-        bool live[kAhead];
+        int32_t pick[kAhead];
 #pragma unroll
         for (uint32_t q = 0; q < kAhead; q++) {
-            const uint32_t s = min(s0 + q, n_used - 1u);
-            live[q] = s0 + q < n_used && (selected == nullptr || selected[t * n_used + s] >= 0);
-            v[q] = __builtin_nontemporal_load((const v4f *)(rows + (uint64_t)s * n_rows));
+            pick[q] = -1;
+            if (s0 + q < n_used) pick[q] = selected != nullptr ? selected[t * n_used + s0 + q] : 0;   // uniform
         }
 #pragma unroll
-        for (uint32_t q = 0; q < kAhead; q++) {
-            acc.x = live[q] ? acc.x + v[q].x : acc.x;
-            acc.y = live[q] ? acc.y + v[q].y : acc.y;
-            acc.z = live[q] ? acc.z + v[q].z : acc.z;
-            acc.w = live[q] ? acc.w + v[q].w : acc.w;
-        }
+        for (uint32_t q = 0; q < kAhead; q++)
+            if (pick[q] >= 0) {
+                const v4f *row = (const v4f *)(rows + (uint64_t)(s0 + q) * n_rows);
+                v[q] = NT ? __builtin_nontemporal_load(row) : *row;
+            }
+#pragma unroll
+        for (uint32_t q = 0; q < kAhead; q++)
+            if (pick[q] >= 0) {
+                acc.x += v[q].x;
+                acc.y += v[q].y;
+                acc.z += v[q].z;
+                acc.w += v[q].w;
+            }
     }
     for (const float *a : {add, residual}) {
         if (a == nullptr) continue;

@@ -357,3 +357,24 @@ def test_argument_errors_are_reported_before_launch():
     # empty problems succeed without touching anything
     dispatch.q8k_quantize(z, f, 0)
     dispatch.router_topk(i, f, f, None, 256, 8, 1.0, 1e-20, 0, 1)
+
+
+@pytest.mark.parametrize("n_used", [1, 2, 3, 7, 8, 9, 16])
+@pytest.mark.parametrize("n_rows,T", [(64, 5), (260, 33)])
+def test_slot_order_sum_leaves_empty_slots_out(n_used, n_rows, T):
+    """Slots in order, eight at a time; a token with every slot empty, one with none, the rest mixed (rows of empty slots hold
+    NaN).  f32 sums in the same order: the same bits."""
+    rng = np.random.default_rng(n_used)
+    sel = np.where(rng.random((T, n_used)) < 0.4, -1, 1).astype(np.int32)
+    sel[0], sel[-1] = -1, 0
+    part = rng.standard_normal((T, n_used, n_rows)).astype(np.float32)
+    want, plain = np.zeros((T, n_rows), np.float32), np.zeros((T, n_rows), np.float32)
+    for s in range(n_used):
+        want = np.where(sel[:, s:s + 1] >= 0, want + part[:, s], want)
+        plain = plain + part[:, s]
+    out = torch.full((T, n_rows), np.nan, dtype=torch.float32, device="cuda")
+    dispatch.moe_reduce_partials(out, dev(part.reshape(-1)), None, n_used, n_rows, T)
+    assert np.array_equal(out.cpu().numpy(), plain)
+    part[sel < 0] = np.nan
+    dispatch.moe_reduce_partials(out, dev(part.reshape(-1)), dev(sel), n_used, n_rows, T)
+    assert np.array_equal(out.cpu().numpy(), want)
