@@ -22,10 +22,12 @@
 // x 2048, 256 experts, down, 16 tokens: 413 / 298.  32 and 64 columns per item lost to the int8 GEMM's narrow tile (512
 // tokens, down 7168 x 2048, 32 columns: 915 / 870): a stage's products, sums and two barriers then outlast its loads.
 //
-// MXFP4: bound by the weight stream.  Every line of it is asked for once, whole and by one instruction (but the ends of
-// a unit), so the loads are non-temporal: whole layers, us with ordinary loads / with these: 7168 x 2048, 256 experts,
-// top-8: 16 tokens 453 / 389, 64: 966 / 865, 300: 1249 / 1226; 4096 x 1024, 128 experts, 37 tokens 188 / 171; all-Q8_0
-// 2048 x 1408: 4 tokens 66 / 61, 40: 140 / 124.  The
+// MXFP4: bound by the weight stream.  Every line of a group's weights is asked for once per item, whole and by one instruction
+// (but the ends of a unit), so the loads of a group that is one item are non-temporal: whole layers, us with ordinary loads /
+// with these: 7168 x 2048, 256 experts, top-8: 16 tokens 478 / 421, 100: 1096 / 963; 4096 x 1024, 128 experts, 37 tokens 182 /
+// 158; all-Q8_0 2048 x 1408: 4 tokens 65.6 / 59.2, 40: 149 / 131.  The items of one group find each other's lines in the L2
+// (non-temporal throughout / there not: 7168 x 2048, every token on the same picks: 100 tokens 272 / 254, 40: 142 / 139;
+// Zipf-skewed 200: 1132 / 1120; gate/up beside a Q8_0 down matrix, same picks, 60: 214 / 204; two items, 24: 104.7 / 105.7).  The
 // workgroups of one launch end within 5 % of each other at 64 tokens and 10 % at 16.  Measured and not
 // taken: the last tenth of the work claimed in chunks through a counter (64 tokens 4 % faster, 200 tokens 2
 // to 5 % slower: every chunk loads an item's columns again); a stage read into registers and its place
@@ -88,6 +90,16 @@ inline bool stream_layout(StreamParams &p, bool pair, uint32_t rt, uint32_t ncg,
 }
 inline size_t stream_lds_bytes(const StreamParams &p, bool pair, uint32_t rt, uint32_t ncg, uint32_t waves) {
     return stream_head_bytes(ncg) + (size_t)stream_fragments(pair, rt, ncg) * stream_part_bytes(waves) + (size_t)p.depth * p.stage_bytes;
+}
+
+// 1 where a group has no item but `wi`, which `after` follows in the list (`last`: nothing does); uniform.  (Written out, as the
+// compiler would keep the truth value in a vector register.)
+__device__ __forceinline__ uint32_t only_item(uint32_t wi, uint32_t after, uint32_t last) {
+    uint32_t once, start;
+    asm volatile("s_xor_b32 %0, %2, %3\n\ts_lshr_b32 %0, %0, 16\n\ts_cselect_b32 %0, 1, %4\n\t"   // (SCC: another expert's)
+                 "s_and_b32 %1, %2, 0xffff\n\ts_cselect_b32 %0, 0, %0"
+                 : "=&s"(once), "=&s"(start) : "s"(wi), "s"(after), "s"(last) : "scc");
+    return once;
 }
 
 // ---- what a wave keeps of an item's columns, and how it multiplies a tile with them ------------------
@@ -285,8 +297,12 @@ __device__ __forceinline__ void stream_body(const StreamParams &p) {
     const uint32_t last_piece = unit_bytes / 16u - 1u;
     uint32_t q_item = item0, q_ut = ut0, q_m = 0, q_slot = 0, q_left = n_stages;   // the next stage to request
     const uint8_t *q_base[2];
+    uint32_t q_once;   // whether nobody else reads the item's weights
     auto q_bases = [&]() {
-        const uint32_t e = __builtin_amdgcn_readfirstlane((uint32_t)p.work_items[q_item]) >> 16;
+        const uint32_t wi = __builtin_amdgcn_readfirstlane((uint32_t)p.work_items[q_item]), e = wi >> 16;
+        // (a group's items follow each other in the list)
+        const uint32_t after = __builtin_amdgcn_readfirstlane((uint32_t)p.work_items[min(q_item + 1u, n_items - 1u)]);
+        q_once = only_item(wi, after, (n_items - q_item - 2u) >> 31);
         const bool extra = e >= p.n_expert;
         q_base[0] = extra ? p.sh_w0 : p.w0 + (uint64_t)e * p.bpe0;
         q_base[1] = !PAIR ? nullptr : extra ? p.sh_w1 : p.w1 + (uint64_t)e * p.bpe1;
@@ -304,7 +320,7 @@ __device__ __forceinline__ void stream_body(const StreamParams &p) {
             uint32_t piece = s - run * p.pitch;
             piece = min(piece, p.run - 1u);   // a row's padding repeats its last piece
             // (slots past the last row fetch the unit's last piece: the load stays in the unit)
-            lds_dma16<true>(dst + L * 1024u, second ? src1 : src0, min(run * p.run + piece, last_piece) * 16u);
+            lds_dma16_if_nt(dst + L * 1024u, second ? src1 : src0, min(run * p.run + piece, last_piece) * 16u, q_once);
         }
         q_left--;
         q_slot = q_slot + 1u == p.depth ? 0u : q_slot + 1u;
