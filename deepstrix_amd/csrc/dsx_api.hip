@@ -76,17 +76,23 @@ int need_init(const char *who) {
     return DSX_OK;
 }
 
-// f(kernel, row tiles per stage) for the instance of k_mxfp4_stream that serves rows of n_sb super-blocks.
+// f(kernel, row tiles per stage, waves) for the instance of k_mxfp4_stream that serves rows of n_sb super-blocks; NCG 0: of
+// k_mxfp4_stream_widths.
+template <bool PAIR, int NCG, int NI, int RT>
+constexpr auto stream_kernel() {
+    if constexpr (NCG == 0) return k_mxfp4_stream_widths<PAIR, NI, RT>;
+    else return k_mxfp4_stream<PAIR, NI, NCG, RT>;
+}
 template <bool PAIR, int NCG, typename F>
 int with_stream_kernel(uint32_t n_sb, F &&f) {
     if constexpr (PAIR) {
-        if (n_sb <= 8u) return f(k_mxfp4_stream<PAIR, 2, NCG, 2>, 2u, 8u);
+        if (n_sb <= 8u) return f(stream_kernel<PAIR, NCG, 2, 2>(), 2u, 8u);
     } else {
-        if (n_sb <= 4u) return f(k_mxfp4_stream<PAIR, 1, NCG, 4>, 4u, 8u);
-        if (n_sb <= 8u) return f(k_mxfp4_stream<PAIR, 2, NCG, 2>, 2u, 8u);
+        if (n_sb <= 4u) return f(stream_kernel<PAIR, NCG, 1, 4>(), 4u, 8u);
+        if (n_sb <= 8u) return f(stream_kernel<PAIR, NCG, 2, 2>(), 2u, 8u);
     }
-    if (n_sb <= 16u) return f(k_mxfp4_stream<PAIR, 4, NCG, 1>, 1u, 8u);
-    return f(k_mxfp4_stream<PAIR, 7, NCG, 1>, 1u, 8u);
+    if (n_sb <= 16u) return f(stream_kernel<PAIR, NCG, 4, 1>(), 1u, 8u);
+    return f(stream_kernel<PAIR, NCG, 7, 1>(), 1u, 8u);
 }
 
 // The same for k_q8_0_stream (16 columns) and rows of n_sb groups of four blocks: f(kernel, row tiles per stage,
@@ -114,6 +120,7 @@ void stream_raise_lds_limits() {
         return 0;
     };
     for (uint32_t n_sb : {4u, 8u, 16u, kStMaxSb}) {
+        with_stream_kernel<PAIR, 0>(n_sb, raise);
         with_stream_kernel<PAIR, 1>(n_sb, raise);
         with_stream_kernel<PAIR, 2>(n_sb, raise);
     }
@@ -218,12 +225,12 @@ static int fit_nt(uint32_t chunk, uint32_t n_blocks, int cap) {
 int group_build_big(hipStream_t st, int32_t *group_count, int32_t *group_offset, int32_t *members,
                     int32_t *work_items, int32_t *n_work_items, const int32_t *selected, uint32_t b,
                     uint32_t n_used, uint32_t n_expert, uint32_t chunk, bool extra, ItemList list2 = {}, ItemList list3 = {},
-                    GroupSplit split = {}) {
-    // list2, list3 (with list2): further lists of work items; split: which groups the first two of them have
-    const uint32_t lists = 1u + (list2.items ? 1u : 0u) + (list3.items ? 1u : 0u);
+                    ItemList list4 = {}, GroupSplit split = {}) {
+    // list2, list3 (with list2), list4 (with both): further lists of work items; split: which groups the first two of them have
+    const uint32_t lists = 1u + (list2.items ? 1u : 0u) + (list3.items ? 1u : 0u) + (list4.items ? 1u : 0u);
     hipLaunchKernelGGL(k_group_tables, dim3(n_expert + (extra ? 1u : 0u) + lists), dim3(kGbThreads), 0, st,
                        group_count, group_offset, members, work_items, n_work_items, selected, b, n_used,
-                       n_expert, chunk, extra ? 1u : 0u, list2, list3, split);
+                       n_expert, chunk, extra ? 1u : 0u, list2, list3, list4, split);
     return launched("group_tables");
 }
 
@@ -253,19 +260,27 @@ int launch_gemm(hipStream_t st, const GemmParams &p, uint32_t max_wi, bool plana
 
 // Streaming launch for groups of few members (items of up to 16 ncg members): as many workgroups as are resident, one
 // of eight waves or two of four per CU.
-// q8: Q8_0 weights and activation rows.
+// q8: Q8_0 weights and activation rows.  narrow: p is on items of 32 members (ncg 2), *narrow the same product on items of
+// 16, and the device chooses between the two.
 template <bool PAIR>
-int launch_stream(hipStream_t st, StreamParams p, uint32_t ncg, bool q8 = false) {
+int launch_stream(hipStream_t st, StreamParams p, uint32_t ncg, bool q8 = false, const StreamParams *narrow = nullptr) {
     auto go = [&](auto kernel, uint32_t rt, uint32_t waves) -> int {
+        constexpr bool kWidths = std::is_invocable_v<decltype(kernel), StreamParams, StreamParams>;
+        StreamParams n = kWidths ? *narrow : StreamParams{};
         const uint64_t act_rows = (uint64_t)p.n_tokens * (p.n_used + 1u);
-        if (p.n_rows % (16u * rt) || p.n_sb > (q8 ? kStQ8MaxSb : kStMaxSb) || !stream_layout(p, PAIR, rt, ncg, waves))
+        if (p.n_rows % (16u * rt) || p.n_sb > (q8 ? kStQ8MaxSb : kStMaxSb) || !stream_layout(p, PAIR, rt, ncg, waves) ||
+            (kWidths && !stream_layout(n, PAIR, rt, 1u, waves)))
             return fail(DSX_ERR_SHAPE, "stream: %u rows of %u super-blocks", p.n_rows, p.n_sb);
         if (act_rows * p.act_row_bytes > 0xFFFFFFFFull)
             return fail(DSX_ERR_INVALID_ARG, "stream: the activation rows exceed 4 GiB");
-        hipLaunchKernelGGL(kernel, dim3((uint32_t)g_num_cu * 8u / waves), dim3(waves * 64u), stream_lds_bytes(p, PAIR, rt, ncg, waves), st, p);
+        const dim3 grid((uint32_t)g_num_cu * 8u / waves), block(waves * 64u);
+        const size_t lds = std::max(stream_lds_bytes(p, PAIR, rt, ncg, waves), kWidths ? stream_lds_bytes(n, PAIR, rt, 1u, waves) : 0u);
+        if constexpr (kWidths) hipLaunchKernelGGL(kernel, grid, block, lds, st, n, p);
+        else hipLaunchKernelGGL(kernel, grid, block, lds, st, p);
         return launched(PAIR ? "gate_up stream" : "down stream");
     };
     if (q8) return with_q8_stream_kernel<PAIR>(p.n_sb, go);   // ncg == 1
+    if (narrow) return with_stream_kernel<PAIR, 0>(p.n_sb, go);
     return ncg == 1u ? with_stream_kernel<PAIR, 1>(p.n_sb, go) : with_stream_kernel<PAIR, 2>(p.n_sb, go);
 }
 

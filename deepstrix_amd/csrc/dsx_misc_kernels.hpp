@@ -741,7 +741,7 @@ __global__ __launch_bounds__(kGbThreads) void k_group_tables(
     int32_t *__restrict__ members, int32_t *__restrict__ work_items,
     int32_t *__restrict__ n_work_items, const int32_t *__restrict__ selected, uint32_t b,
     uint32_t n_used, uint32_t n_expert, uint32_t chunk, uint32_t extra, const ItemList list2,
-    const ItemList list3, const GroupSplit split) {
+    const ItemList list3, const ItemList list4, const GroupSplit split) {
     constexpr uint32_t kWaves = kGbThreads / 64;
     __shared__ uint32_t s_mine[kWaves], s_below[kWaves];
     const uint32_t n_groups = n_expert + (extra ? 1u : 0u);
@@ -749,7 +749,7 @@ __global__ __launch_bounds__(kGbThreads) void k_group_tables(
         // other cuts of the same groups (other items) have a workgroup each, which writes the counts and
         // offsets too, with the same values
         const uint32_t which = blockIdx.x - n_groups;
-        const ItemList l = which == 0u ? ItemList{work_items, n_work_items, chunk} : which == 1u ? list2 : list3;
+        const ItemList l = which == 0u ? ItemList{work_items, n_work_items, chunk} : which == 1u ? list2 : which == 2u ? list3 : list4;
         group_count_body(group_count, group_offset, l, selected, b, n_used, n_expert, extra, split);
         return;
     }

@@ -458,6 +458,18 @@ __global__ __launch_bounds__(512, 2) void k_mxfp4_stream(const StreamParams p) {
     stream_body<StreamMxfp4<NI, NCG>, PAIR, NCG, RT>(p);
 }
 
+// Items of 16 and of 32 columns are both there: the narrower ones unless they are over a fifth more, as each of them reads its
+// weights anew (items of 16 per item of 32, time with these per time with those: 4096 x 1024, 128 experts, 110 tokens: spread
+// picks 1.02, 0.85, Zipf-skewed 1.05, 0.87, on 48 experts 1.69, 1.15; 180: spread 1.11, 0.94, Zipf 1.18, 0.95; 5120 x 1536, 160, 220:
+// Zipf 1.11, 0.98, on 100 experts 1.23, 1.04, on 60 1.96, 1.37; 2048 x 1536, 64, 100: on 40 1.34, 1.09).
+template <bool PAIR, int NI, int RT>
+__global__ __launch_bounds__(512, 2) void k_mxfp4_stream_widths(const StreamParams narrow, const StreamParams wide) {
+    if (5u * (uint32_t)*narrow.n_work_items <= 6u * (uint32_t)*wide.n_work_items)   // uniform
+        stream_body<StreamMxfp4<NI, 1>, PAIR, 1, RT>(narrow);
+    else
+        stream_body<StreamMxfp4<NI, 2>, PAIR, 2, RT>(wide);
+}
+
 template <bool PAIR, int W, int NI, int RT>
 __global__ __launch_bounds__(W * 64, 2) void k_q8_0_stream(const StreamParams p) {
     stream_body<StreamQ8<W, NI>, PAIR, 1, RT>(p);

@@ -54,6 +54,54 @@ def test_stream_matches_the_oracle(monkeypatch, hidden, inter, which):
     H.assert_close(out, ref.moe_forward(H.host_weights(s), x, sel, w), 2e-3, f"{hidden} x {inter} T={T}")
 
 
+def _items(sel, E, members, shared):
+    n = np.bincount(sel[sel >= 0], minlength=E)
+    return int((-(-n // members)).sum()) + (-(-len(sel) // members) if shared else 0)
+
+
+@pytest.mark.parametrize("hidden,inter", SHAPES)
+@pytest.mark.parametrize("kind", ["spread", "few"])
+@pytest.mark.parametrize("T", [26, 34])
+def test_either_width_of_item_gives_the_same_bits(monkeypatch, hidden, inter, kind, T):
+    """6 to 9 picks per expert: spread picks make hardly more items of 16 members than of 32, picks on three experts twice as many;
+    the first 20 tokens alone (under 6 picks per expert) take items of 16."""
+    monkeypatch.setattr(MoeLayer, "v3_thresholds_below_experts", None)
+    s = H.Shape(hidden, inter, 8, 2, shared=T == 34, seed=520, **ROUTER)
+    layer = MoeLayer(H.device_weights(s), T)
+    x, _, _ = H.host_inputs(s, T)
+    rng = np.random.default_rng(T)
+    sel = np.stack([(2 * t + np.arange(2)) % 8 if kind == "spread" else rng.permutation(3)[:2] for t in range(T)]).astype(np.int32)
+    sel[T // 2, 1] = -1
+    assert (5 * _items(sel, 8, 16, s.shared) <= 6 * _items(sel, 8, 32, s.shared)) == (kind == "spread")
+    w = rng.uniform(0.05, 0.6, sel.shape).astype(np.float32)
+    dx, ds, dwt = torch.from_numpy(x).cuda(), torch.from_numpy(sel).cuda(), torch.from_numpy(w).cuda()
+    out = layer.run(dx, None, selected_in=ds, weights_in=dwt).clone()
+    first = layer.run(dx[:20].contiguous(), None, selected_in=ds[:20].contiguous(), weights_in=dwt[:20].contiguous())
+    torch.cuda.synchronize()
+    assert torch.equal(out[:20], first)
+    H.assert_close(out.cpu().numpy(), ref.moe_forward(H.host_weights(s), x, sel, w), 2e-3, f"{hidden} x {inter} T={T} {kind}")
+
+
+@pytest.mark.parametrize("kind", ["spread", "few", "same"])
+def test_either_width_or_the_gemm(kind):
+    """8 picks per expert where the GEMM is offered as well (three lists of items): same picks take it."""
+    s = H.Shape(5120, 1536, 160, 6, seed=530, **ROUTER)
+    dw = H.device_weights(s)
+    layer, gemm = MoeLayer(dw, 220), MoeLayer(dw, 220)
+    gemm.set_tuning(gemm_min_tokens=1)
+    x = torch.from_numpy(H.host_inputs(s, 220)[0]).cuda()
+    sel, w = _picks(s, 220, kind, 530)
+    if kind == "few":
+        sel = (np.argsort(np.random.default_rng(531).random((220, 60)), axis=1)[:, :6]).astype(np.int32)
+    assert (5 * _items(sel, 160, 16, True) <= 6 * _items(sel, 160, 32, True)) == (kind == "spread")
+    ds, dwt = torch.from_numpy(sel).cuda(), torch.from_numpy(w).cuda()
+    out = layer.run(x, None, selected_in=ds, weights_in=dwt).clone()
+    want = gemm.run(x, None, selected_in=ds, weights_in=dwt).clone()
+    first = layer.run(x[:90].contiguous(), None, selected_in=ds[:90].contiguous(), weights_in=dwt[:90].contiguous())   # (below gemm_min_tokens)
+    torch.cuda.synchronize()
+    assert torch.equal(out, want) == (kind == "same") and torch.equal(out[:90], first) == (kind != "same")
+
+
 @pytest.mark.parametrize("hidden,inter", [(512, 256), (1280, 768), (2048, 1280), (4352, 1024), (7168, 512)])
 @pytest.mark.parametrize("T", [2, 10, 15, 16, 47, 64])
 @pytest.mark.parametrize("shared", ["none", "same", "q8_0"])
