@@ -197,6 +197,16 @@ def test_default_thresholds_follow_the_picks_per_expert():
     assert 49 <= mixed["gemm_q8"] <= 64
 
 
+@pytest.mark.parametrize("shape,decode_max", [
+    # (hidden, inter, experts, top), last token count at which the decode launch was measured no slower than the narrow tile
+    ((7168, 2048, 256, 8), 7), ((7168, 2048, 256, 4), 15), ((7168, 2048, 192, 8), 6), ((7168, 2048, 160, 8), 6), ((7168, 2048, 160, 6), 8),
+    ((7168, 2048, 128, 8), 5), ((7168, 2048, 64, 8), 2), ((7168, 2048, 64, 4), 5), ((7168, 2048, 32, 4), 2), ((6144, 4096, 16, 2), 2),
+    ((6144, 4096, 32, 2), 5), ((4096, 14336, 8, 2), 1), ((5120, 1536, 160, 6), 9), ((4096, 1024, 128, 8), 5), ((2048, 1536, 64, 6), 3)])
+def test_planar_layers_leave_the_decode_launch_where_it_is_slower(shape, decode_max):
+    t = _thresholds(*shape, capi.FMT_MXFP4_PLANAR, capi.FMT_MXFP4_PLANAR)
+    assert t["decode_max"] == decode_max and t["gemm"] * 11 // 16 <= decode_max + 1 and t["narrow"] == 14
+
+
 def _workspace_bytes(T, hidden, inter, n_expert, n_used, gate_fmt, down_fmt):
     l = capi.lib()
     d = _desc(hidden=hidden, inter=inter, n_expert=n_expert, n_used=n_used, gate_fmt=gate_fmt, up_fmt=gate_fmt,
