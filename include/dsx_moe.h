@@ -369,15 +369,14 @@ int dsx_moe_layer_set_tuning(dsx_moe_layer *layer, uint32_t by_expert_chunk, uin
 int dsx_moe_layer_get_tuning(const dsx_moe_layer *layer, uint32_t out[6]);
 /* The token counts that take the streaming kernels: out[0] the first, out[1] the last, both 0 where there are
  * none (planar weights, Q8_0 gate/up with an MXFP4 down matrix, weights that are not 8-byte aligned, rows of more
- * than 7168 values -- Q8_0: 4096 -- values set by the caller as above).  By default, all-MXFP4: from 9 tokens at the
- * earliest to below 18 picks per expert, 28 where a matrix has up to 4 M elements [9 .. 575]; beside a Q8_0 down
- * matrix the range of gate/up, from 2 tokens to below 28 picks per expert [2 .. 895]; few picks in all and matrices
- * under 4 M elements start later; all-Q8_0: from 2 tokens to below 4 picks per expert, 1.5 where a matrix has up to
+ * than 7168 values -- Q8_0: 4096 -- values set by the caller as above).  By default, all-MXFP4: from 28 picks in all on
+ * [4 tokens], 48 where a matrix has under 8 M elements, 112 under 3 M (beside a shared expert of another format from 7 tokens at
+ * the earliest), from 9 tokens or where the decode path ends in any case -- matrices under 4 M elements: from 2.25 or 3.5 picks per
+ * expert -- to below 18 picks per expert, 28 where a matrix has up to 4 M elements [4 .. 575]; beside a Q8_0 down
+ * matrix the range of gate/up, from 2 tokens (matrices under 4 M elements: 1.25 picks per expert) to below 28 picks per expert
+ * [2 .. 895]; all-Q8_0: from 2 tokens to below 4 picks per expert, 1.5 where a matrix has up to
  * 2 M elements.  Where the same token count would take a grouped GEMM otherwise, the device chooses between the two by
- * the picks (all-Q8_0: for more than 16 tokens where n_expert * hidden * inter is at least 256 M).
- * Below out[0] the decode path of an all-MXFP4 layer on the engine's rows uses the same kernels from 28 picks on (48 where a
- * matrix has under 8 M elements, 112 under 3 M; beside a shared expert of another format from 7 tokens at the earliest)
- * [4 .. 8 tokens], until the caller sets decode_max_tokens or a decode form other than 1. */
+ * the picks (all-Q8_0: for more than 16 tokens where n_expert * hidden * inter is at least 256 M). */
 int dsx_moe_layer_get_streaming(const dsx_moe_layer *layer, uint32_t out[2]);
 /* Decode path of an all-MXFP4 layer (up to decode_max_tokens tokens, or to where streaming begins); no
  * counterpart in the reference.  fused: 1 = gate/up, mid quantization, down and the slot-order sum in ONE launch
@@ -388,14 +387,15 @@ int dsx_moe_layer_get_streaming(const dsx_moe_layer *layer, uint32_t out[2]);
  * with and without pairing.  3 = the same launch, never pairing; 4 = the same launch, pairing
  * from 2 tokens on (for steps whose tokens mostly name the same experts, such as the
  * verification of consecutive draft tokens); 2 = one launch per stage; 0 keeps the current
- * value.  2, 3 and 4 hold up to decode_max_tokens tokens, where by default (1) streaming may begin earlier.  spin_limit (0 keeps): bound, in polling rounds of about half a microsecond, of every
+ * value.  2, 3 and 4 hold up to decode_max_tokens tokens, where by default (1) streaming begins earlier [4 tokens].  spin_limit (0 keeps): bound, in polling rounds of about half a microsecond, of every
  * wait one workgroup does for another; values above 2^20 are taken as 2^20, so that every wait
  * stays bounded. */
 int dsx_moe_layer_set_decode(dsx_moe_layer *layer, uint32_t fused, uint32_t spin_limit);
 /* Measurement aid with no counterpart in the reference: a device buffer of n_items x 4 uint64
  * that the one-launch decode path fills with clock readings (constant 100 MHz counter) per
  * work item -- start, operands staged / weights requested, wait over, end; items in grid order:
- * gate/up tiles, the relay, down blocks.  Ignored while n_items is smaller than the grid;
+ * gate/up tiles, the relay, down blocks.  Ignored while n_items is smaller than the grid, and by the token counts that
+ * stream (dsx_moe_layer_get_streaming; decode_max_tokens, set by the caller, brings the launch back);
  * NULL turns it off. */
 int dsx_moe_layer_set_trace(dsx_moe_layer *layer, uint64_t *trace, size_t n_items);
 /* Status word of the last dsx_moe_layer_forward / dsx_moe_block_forward that used `workspace`

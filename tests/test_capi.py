@@ -245,27 +245,34 @@ def _streaming(tuning=(0, 0, 0, 0), decode=0, **kw):
     return tuple(int(x) for x in v)
 
 
+def _sh(inter):
+    """A shared expert of the routed shape."""
+    return dict(sh_inter=inter, sh_gate_fmt=capi.FMT_MXFP4, sh_up_fmt=capi.FMT_MXFP4, sh_down_fmt=capi.FMT_MXFP4,
+                sh_gate=0x1000, sh_up=0x1000, sh_down=0x1000)
+
+
 _V3 = dict(hidden=7168, inter=2048, n_expert=256, n_used=8)
 
 
 @pytest.mark.parametrize("shape,slower,faster", [
-    # (hidden, inter, experts, top), token counts at which the older path was measured faster, and streaming
-    ((7168, 2048, 256, 8), [8], [9, 10, 64]),
-    ((7168, 2048, 256, 4), [9, 10, 12, 14], [17, 20]),
-    ((4096, 1024, 256, 4), [9, 12, 14, 16], [17, 20]),
-    ((4096, 1024, 128, 8), [8], [9, 10, 37]),
-    ((5120, 1536, 160, 6), [8, 9], [11, 12]),
-    ((4096, 1536, 128, 4), [9, 10], [11, 12]),
-    ((2048, 1536, 64, 6), [14, 16, 20, 22], [24, 28]),
-    ((2048, 768, 128, 8), [18, 20, 28, 32], [36, 40]),
-    ((1536, 1536, 64, 6), [14, 20, 28, 36], [38, 64])])
+    # (hidden, inter, experts, top), token counts at which the older path was measured faster, and streaming (a shared expert
+    # of the routed shape among the slots)
+    ((7168, 2048, 256, 8), [2, 3], [4, 6, 9, 64]),
+    ((7168, 2048, 256, 4), [4], [8, 9, 17]),
+    ((4096, 1024, 256, 4), [8], [12, 14, 20]),
+    ((4096, 1024, 128, 8), [4], [6, 8, 37]),
+    ((5120, 1536, 160, 6), [6], [8, 9, 12]),
+    ((4096, 1536, 128, 4), [6], [12, 14]),
+    ((2048, 1536, 64, 6), [4], [10, 16, 28]),
+    ((2048, 768, 128, 8), [8], [14, 20, 40]),
+    ((1536, 1536, 64, 6), [8], [19, 28, 64])])
 def test_streaming_begins_where_it_is_faster(shape, slower, faster):
-    first, last = _streaming(**dict(zip(("hidden", "inter", "n_expert", "n_used"), shape)))
+    first, last = _streaming(**dict(zip(("hidden", "inter", "n_expert", "n_used"), shape)), **_sh(shape[1]))
     assert max(slower) < first <= min(faster) and max(faster) <= last, (first, last)
 
 
 def test_values_that_the_caller_sets_are_not_passed_over_by_streaming():
-    assert _streaming(**_V3) == (9, 575)
+    assert _streaming(**_V3) == (4, 575)   # (where the decode launch is left: the range reported is the range taken)
     mixed = dict(_V3, down_fmt=capi.FMT_Q8_0)
     assert _streaming(**mixed) == (2, 895)
     for tuning in [(4, 0, 0, 0), (0, 112, 0, 0), (0, 0, 0, 1)]:   # (the values that are the defaults)
@@ -275,7 +282,7 @@ def test_values_that_the_caller_sets_are_not_passed_over_by_streaming():
     for form in (2, 3, 4):
         assert _streaming(decode=form, **_V3) == (15, 575)
         assert _streaming(decode=form, **mixed) == (2, 895)   # (no decode path beside a Q8_0 down matrix)
-    assert _streaming(decode=1, **_V3) == (9, 575)
+    assert _streaming(decode=1, **_V3) == (4, 575)
 
 
 def test_streaming_range_of_an_all_q8_0_layer_is_reported():
@@ -307,9 +314,8 @@ def test_all_q8_0_streaming_ends_where_it_is_slower(shape, last):
                                  dict(gate_fmt=capi.FMT_Q8_0, up_fmt=capi.FMT_Q8_0, sh_inter=0)])
 def test_operands_that_the_streaming_kernels_do_not_take(odd):
     """Weights that are not 8-byte aligned, rows of more than 28 super-blocks, other formats."""
-    sh = dict(sh_inter=2048, sh_gate_fmt=capi.FMT_MXFP4, sh_up_fmt=capi.FMT_MXFP4, sh_down_fmt=capi.FMT_MXFP4,
-              sh_gate=0x1000, sh_up=0x1000, sh_down=0x1000)
-    assert _streaming(**dict(_V3, **sh)) == (9, 575)
+    sh = _sh(2048)
+    assert _streaming(**dict(_V3, **sh)) == (4, 575)
     assert _streaming(**{**_V3, **sh, **odd}) == (0, 0)
 
 

@@ -111,6 +111,19 @@ def test_config2_v3_shape_decode(T, cfg2_layer):
     assert H.max_rel(out, want) < OUT_TOL
 
 
+@pytest.mark.parametrize("T", [4, 7])
+def test_config2_v3_shape_one_launch_with_pairing(T, cfg2_layer):
+    """Token counts that stream by default: the one-launch form, whose tokens that name one expert are paired, up to the limit
+    that the caller sets."""
+    dw = cfg2_layer[1]
+    layer = MoeLayer(dw, T)
+    assert layer.streaming()[0] <= T and layer.tuning()["share_min_tokens"] <= T
+    layer.set_tuning(decode_max_tokens=8)
+    assert layer.streaming()[0] > T
+    out, want, sel, rsel = run_case(H.CFG2, T, layer, dw)
+    assert H.max_rel(out, want) < OUT_TOL and layer.status() == 0
+
+
 @pytest.fixture(scope="module")
 def cfg2_layer():
     dw = H.device_weights(H.CFG2)

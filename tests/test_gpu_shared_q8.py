@@ -82,7 +82,7 @@ def v3_layers():
     dw = H.device_weights(V3)
     layer, older = MoeLayer(dw, 512), MoeLayer(dw, 512)
     older.set_tuning(by_expert_chunk=4)
-    assert layer.streaming() == (9, 575) and older.streaming() == (0, 0)
+    assert layer.streaming() == (7, 575) and older.streaming() == (0, 0)
     return layer, older, H.host_weights_from_device(V3, dw)
 
 

@@ -257,17 +257,20 @@ def test_a_stack_of_streaming_blocks(monkeypatch, fmt, T):
 
 
 @pytest.mark.parametrize("hidden,inter,E,k,T", [(4096, 2048, 16, 8, 4), (4096, 2048, 16, 8, 8), (7168, 2048, 64, 8, 4), (2048, 1536, 16, 6, 8),
-                                                (1536, 1536, 64, 6, 19), (2048, 1536, 16, 6, 7), (4096, 2048, 16, 8, 3)])
+                                                (1536, 1536, 64, 6, 19), (2048, 1536, 16, 6, 7), (4096, 2048, 16, 8, 3), (4096, 2048, 64, 8, 3)])
 @pytest.mark.parametrize("shared", ["none", "same", "q8_0"])
 def test_few_tokens_stream_in_the_decode_launch_s_place(monkeypatch, hidden, inter, E, k, T, shared):
-    """From 28, 48 or 112 picks on by size of a matrix (the last two: one token short of it); a decode limit set by the
-    caller brings the one-launch form back, the same sums in another order."""
+    """From 28, 48 or 112 picks on by size of a matrix (the last two: one token short of it; a Q8_0 shared expert: from 7
+    tokens); a decode limit set by the caller brings the one-launch form back, the same sums in another order, whose bits the
+    token counts short of both ranges have (three tokens on 64 experts)."""
     monkeypatch.setattr(MoeLayer, "v3_thresholds_below_experts", None)
     fmts = dict(sh_gate_fmt=FMT_Q8_0, sh_down_fmt=FMT_Q8_0) if shared == "q8_0" else {}
     s = H.Shape(hidden, inter, E, k, shared=shared != "none", seed=950 + T, **fmts, **ROUTER)
     dw = H.device_weights(s)
     layer, launch = MoeLayer(dw, T), MoeLayer(dw, T)
     launch.set_tuning(decode_max_tokens=16)
+    streams = T * k >= (28 if hidden * inter >= 8 << 20 else 48 if hidden * inter >= 3 << 20 else 112) and (shared != "q8_0" or T >= 7)
+    assert (T >= layer.streaming()[0]) == streams
     x, _, _ = H.host_inputs(s, T)
     rng = np.random.default_rng(T)
     sel = np.stack([rng.permutation(E)[:k] for _ in range(T)]).astype(np.int32)
@@ -279,10 +282,11 @@ def test_few_tokens_stream_in_the_decode_launch_s_place(monkeypatch, hidden, int
     if T <= 16:
         other = launch.run(dx, None, selected_in=ds, weights_in=dwt)
         assert layer.status() == 0 and launch.status() == 0
+        assert torch.equal(out, other) == (not streams and T <= layer.tuning()["decode_max_tokens"])
         assert H.max_rel(out.cpu().numpy(), other.cpu().numpy()) < 1e-3
     torch.cuda.synchronize()
     assert torch.equal(out, again)
-    H.assert_close(out.cpu().numpy(), ref.moe_forward(H.host_weights(s), x, sel, w), 2e-3, f"{hidden} x {inter} T={T} {shared}")
+    H.assert_close(out.cpu().numpy(), ref.moe_forward(H.host_weights(s, experts=np.unique(sel[sel >= 0])), x, sel, w), 2e-3, f"{hidden} x {inter} T={T} {shared}")
 
 
 def test_a_stack_of_few_token_streaming_blocks(monkeypatch):
