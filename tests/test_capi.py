@@ -271,8 +271,32 @@ def test_streaming_begins_where_it_is_faster(shape, slower, faster):
     assert max(slower) < first <= min(faster) and max(faster) <= last, (first, last)
 
 
+# (hidden, inter, experts, top): first token count with a shared expert alike, without one, with a Q8_0 one
+FIRST_STREAMING = {
+    (7168, 2048, 256, 8): (4, 6, 7), (7168, 2048, 256, 6): (6, 8, 10), (7168, 2048, 256, 4): (8, 12, 14), (7168, 2048, 256, 16): (3, 3, 7),
+    (4096, 2048, 128, 8): (4, 4, 7), (4096, 2048, 64, 4): (7, 7, 7), (4096, 1024, 128, 8): (6, 7, 9), (5120, 1536, 160, 6): (8, 9, 9),
+    (3072, 1024, 128, 8): (8, 8, 9), (2048, 1536, 64, 6): (10, 10, 10), (2048, 768, 128, 8): (14, 14, 14), (1024, 512, 128, 8): (36, 36, 36),
+    (1024, 1024, 64, 6): (24, 24, 24)}
+
+
+def first_streaming(shape, **sh):
+    return _streaming(**dict(zip(("hidden", "inter", "n_expert", "n_used"), shape)), **sh)[0]
+
+
+@pytest.mark.parametrize("shape", FIRST_STREAMING)
+def test_few_tokens_stream_where_that_was_measured_faster(shape):
+    assert (first_streaming(shape, **_sh(shape[1])), first_streaming(shape)) == FIRST_STREAMING[shape][:2]
+
+
+@pytest.mark.gpu   # (a shared expert of another format has a stream of its own)
+@pytest.mark.parametrize("shape", FIRST_STREAMING)
+def test_few_tokens_stream_beside_a_q8_0_shared_expert_where_that_was_measured_faster(shape):
+    Q = capi.FMT_Q8_0
+    assert first_streaming(shape, **dict(_sh(shape[1]), sh_gate_fmt=Q, sh_up_fmt=Q, sh_down_fmt=Q)) == FIRST_STREAMING[shape][2]
+
+
 def test_values_that_the_caller_sets_are_not_passed_over_by_streaming():
-    assert _streaming(**_V3) == (4, 575)   # (where the decode launch is left: the range reported is the range taken)
+    assert _streaming(**_V3) == (6, 575)   # (where the decode launch is left: the range reported is the range taken)
     mixed = dict(_V3, down_fmt=capi.FMT_Q8_0)
     assert _streaming(**mixed) == (2, 895)
     for tuning in [(4, 0, 0, 0), (0, 112, 0, 0), (0, 0, 0, 1)]:   # (the values that are the defaults)
@@ -282,7 +306,7 @@ def test_values_that_the_caller_sets_are_not_passed_over_by_streaming():
     for form in (2, 3, 4):
         assert _streaming(decode=form, **_V3) == (15, 575)
         assert _streaming(decode=form, **mixed) == (2, 895)   # (no decode path beside a Q8_0 down matrix)
-    assert _streaming(decode=1, **_V3) == (4, 575)
+    assert _streaming(decode=1, **_V3) == (6, 575)
 
 
 def test_streaming_range_of_an_all_q8_0_layer_is_reported():
