@@ -530,7 +530,7 @@ def main():
             lps[i % L].run(x_all[i:i + 1], lg_all[i:i + 1], out=out)
         torch.cuda.synchronize()
         extra["us_per_token_T1_planar_weights"] = (time.perf_counter() - t1) * 1e6 / K
-        # ... and the other token counts of config 2 (the grouped GEMMs from 12 tokens on)
+        # ... and the other token counts of config 2 (the grouped GEMMs from 8 tokens on)
         for T in small_t:
             lpt = [MoeLayer(lp.w, T) for lp in lps]
             leg = decode_leg(lpt, H, torch, np, base, T)

@@ -840,7 +840,7 @@ __global__ __launch_bounds__(kGbThreads) void k_group_tables(
 // for / a clamped row for every slot of the eight that is not there / this: 7168 columns, 512 tokens, top-4: 15.6 / 17.2 /
 // 13.9, top-8: 27.2 / 24.1 / 24.1, half of the slots empty: 18.8 / 24.1 / 14.9; 4096 tokens, top-2: 63 / 84 / 54, top-6: 151 /
 // 135 / 129.  NT: the rows are read here for the last time, but one or two of a token are still in the caches (512 tokens,
-// one row, ordinary / non-temporal: 6.7 / 8.2; two: 8.8 / 9.9).
+// one row, ordinary / non-temporal: 7.2 / 8.2; two: 8.6 / 9.9).
 template <bool NT>
 __global__ __launch_bounds__(256) void k_reduce_partials(float *out, const float *__restrict__ partials,
                                                          const int32_t *__restrict__ selected,

@@ -32,8 +32,8 @@
 // taken: the last tenth of the work claimed in chunks through a counter (64 tokens 4 % faster, 200 tokens 2
 // to 5 % slower: every chunk loads an item's columns again); a stage read into registers and its place
 // requested before the products (16 columns: no change; 32: the registers spill).  Scalar registers run out in
-// the instances for long rows (45 to 53 of them live in lanes of a vector register in gate/up, 32 to 36 in down;
-// no memory); what that costs was not measured.
+// the instances for long rows (16 / 32 columns: 43 / 65 of them live in lanes of a vector register in gate/up, 27 / 51 in
+// down; no memory); what that costs was not measured.
 //
 // A shared expert of another format runs beside these on the layer's side stream although they take nearly all
 // of every CU's LDS: the layer of 256 experts 7168 x 2048 with a Q8_0 shared expert, us before / with the streaming
@@ -256,7 +256,8 @@ __device__ __forceinline__ void stream_body(const StreamParams &p) {
     constexpr int kW = COLS::kWaves;
     // Between two stages a wave requests the next one or adds up and stores the last one's sums.  MXFP4: the first half of
     // the waves does the one, the second half the other, at the same time and without a load that waits behind a store
-    // (vmcnt counts them in order); Q8_0: every wave does its part of both (half each: 2048 x 1408, 40 tokens 124 / 126 us).
+    // (vmcnt counts them in order; 7168 x 2048, 256 experts, every wave both / so: 100 tokens 977 / 961 us, Zipf-skewed 200: 1146 / 1117, but
+    // with every token on the same picks, whose lines come from the L2 faster than half of the waves ask for them, 100: 240 / 254); Q8_0: every wave does its part of both (half each: 2048 x 1408, 40 tokens 124 / 126 us).
     constexpr uint32_t kLoaders = COLS::kRoles ? (uint32_t)kW / 2u : (uint32_t)kW;
     constexpr uint32_t kSummer0 = COLS::kRoles ? kLoaders : 0u;               // the first wave that sums
     constexpr uint32_t kSummers = ((uint32_t)kW - kSummer0) * 64u;            // threads that do

@@ -72,7 +72,8 @@ class LayerWeights:
 class MoeLayer:
     # Set by a test-suite whose small shapes stand in for the paths of a large one: layers with
     # fewer experts than this get fixed token thresholds (decode path up to 16 tokens, grouped
-    # GEMM from 100; planar: 11 / 17 / narrow tile below 14 picks), so that a token count names the
+    # GEMM from 100; planar: 11 / 17 / narrow tile below 14 picks; not those that 256 experts of 7168 x 2048 have
+    # by default), so that a token count names the
     # same path on every small shape.  None (the default): the library's own, shape-derived
     # thresholds.
     v3_thresholds_below_experts: Optional[int] = None

@@ -313,8 +313,8 @@ void dsx_moe_layer_destroy(dsx_moe_layer *layer);
 /* No counterpart in the reference: rewrites every MXFP4 tensor the layer was created with -- the
  * caller's weight buffers -- in place into the planar form (DSX_FMT_MXFP4_PLANAR above), or back
  * into the engine's rows, and switches the layer over (its default thresholds included: a planar
- * layer leaves the decode path at 0.24 picks per expert [8 tokens at 256 experts, top-8], 0.375 where a matrix has at most
- * 12 M elements, and starts with the 16-column GEMM tile).  A layer
+ * layer leaves the decode path at 0.375 picks per expert, 0.24 where a matrix has over 12 M elements and there are 54 picks
+ * [8 tokens at 256 experts, top-8], and starts with the 16-column GEMM tile).  A layer
  * without MXFP4 tensors, or one already in the form asked for, is left as it is.  Shapes are
  * checked before the first byte moves; MXFP4 tensors whose byte ranges overlap are refused.
  * The rewrite is enqueued on `stream` like a kernel launch, while the layer switches over on the
@@ -348,19 +348,20 @@ int dsx_moe_layer_set_profile_events(dsx_moe_layer *layer, void *gate_up_begin, 
  * gemm_min_tokens (default for an all-MXFP4 layer: 3.5 picks per expert [112 tokens], 7 where
  * n_expert * inter / 256 < 512; MXFP4 gate/up with a Q8_0 down matrix 2 [64], 4 for
  * matrices under 4 M elements; all-Q8_0 layers 1.5, and there behind the streaming range; on planar weights
- * right behind the decode path [17]): from this many tokens
+ * right behind the decode path, 16/11 of where that ends [11]): from this many tokens
  * on, a layer with MXFP4 gate/up runs the grouped-GEMM path (128 token columns per work item,
  * shared expert as an extra group; a Q8_0 down matrix takes the int8 grouped GEMM) and an all-Q8_0
  * layer the int8 grouped GEMMs; an all-MXFP4 layer whose GEMMs use the narrow tile (below)
  * switches at 11/16 of it.
  * decode_max_tokens (default: 0.45 picks per expert -- 0.85 where inter <= 1024 -- and at most 16 [14];
- * 0.375 on planar weights [11]):
+ * on planar weights up to 0.375, 0.24 where a matrix has over 12 M elements and there are 54 picks [7]):
  * up to this many tokens, an all-MXFP4 layer runs the decode path (dsx_moe_layer_set_decode: every
  * token on its own picks, no grouping by expert; the one-launch form serves at most 16 tokens,
  * beyond that the decode kernels run once per stage).
  * gemm_narrow_members (default 1 = never; 14 on planar weights): while the picks per expert average
  * less than this, the all-MXFP4 grouped GEMMs use 16 token columns per work item and two
- * workgroups per CU. */
+ * workgroups per CU.  Until the caller sets it, planar layers whose experts have 3 G elements per kind of matrix use both widths
+ * from 12 to 32 picks per expert, groups of up to 16 members the narrow one [384 .. 1023 tokens]. */
 int dsx_moe_layer_set_tuning(dsx_moe_layer *layer, uint32_t by_expert_chunk, uint32_t gemm_min_tokens,
                              uint32_t decode_max_tokens, uint32_t gemm_narrow_members);
 /* The current values: out[0] by_expert_chunk, [1] gemm_min_tokens, [2] the same for layers whose

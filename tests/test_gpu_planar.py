@@ -96,7 +96,7 @@ def test_layer_is_bitwise_the_same_on_planar_weights(name):
     dwp = H.device_weights(s, planar=True)
     assert dwp.gate_fmt == FMT_MXFP4_PLANAR
     planar = MoeLayer(dwp, max(TOKENS))
-    # a planar layer has its own thresholds (decode up to 11 tokens, then the grouped GEMMs, narrow
+    # a planar layer has its own thresholds (these shapes: decode up to 11 tokens, then the grouped GEMMs, narrow
     # tile first): the row layout follows them here, so that both run the same kernels at every
     # token count
     if s.down_fmt == FMT_MXFP4:   # (a layer with a Q8_0 matrix keeps the row layout's thresholds)
@@ -122,7 +122,7 @@ def test_decode_modes_on_planar_weights(fused):
     planar = MoeLayer(H.device_weights(s, planar=True), 16)
     rows.set_decode(fused)
     planar.set_decode(fused)
-    planar.set_tuning(decode_max_tokens=16)   # (a planar layer leaves the decode path at 12 tokens)
+    planar.set_tuning(decode_max_tokens=16)   # (these planar layers leave the decode path at 12 tokens)
     for T in (1, 2, 5, 12, 16):
         a, _, _, _ = _run(rows, s, T)
         b, _, _, _ = _run(planar, s, T)
