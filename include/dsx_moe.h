@@ -313,8 +313,8 @@ void dsx_moe_layer_destroy(dsx_moe_layer *layer);
 /* No counterpart in the reference: rewrites every MXFP4 tensor the layer was created with -- the
  * caller's weight buffers -- in place into the planar form (DSX_FMT_MXFP4_PLANAR above), or back
  * into the engine's rows, and switches the layer over (its default thresholds included: a planar
- * layer leaves the decode path at 0.375 picks per expert, 0.24 where a matrix has over 12 M elements and there are 54 picks
- * [8 tokens at 256 experts, top-8], and starts with the 16-column GEMM tile).  A layer
+ * layer leaves the decode path at 0.375 picks per expert, 0.24 where a matrix has over 12 M elements and the picks
+ * make 432 workgroups (n_used * inter / 256 each token) [8 tokens at 256 experts, top-8], and starts with the 16-column GEMM tile).  A layer
  * without MXFP4 tensors, or one already in the form asked for, is left as it is.  Shapes are
  * checked before the first byte moves; MXFP4 tensors whose byte ranges overlap are refused.
  * The rewrite is enqueued on `stream` like a kernel launch, while the layer switches over on the
@@ -354,7 +354,7 @@ int dsx_moe_layer_set_profile_events(dsx_moe_layer *layer, void *gate_up_begin, 
  * layer the int8 grouped GEMMs; an all-MXFP4 layer whose GEMMs use the narrow tile (below)
  * switches at 11/16 of it.
  * decode_max_tokens (default: 0.45 picks per expert -- 0.85 where inter <= 1024 -- and at most 16 [14];
- * on planar weights up to 0.375, 0.24 where a matrix has over 12 M elements and there are 54 picks [7]):
+ * on planar weights up to 0.375, 0.24 where a matrix has over 12 M elements (above) [7]):
  * up to this many tokens, an all-MXFP4 layer runs the decode path (dsx_moe_layer_set_decode: every
  * token on its own picks, no grouping by expert; the one-launch form serves at most 16 tokens,
  * beyond that the decode kernels run once per stage).

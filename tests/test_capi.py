@@ -201,7 +201,7 @@ def test_default_thresholds_follow_the_picks_per_expert():
     # (hidden, inter, experts, top), last token count at which the decode launch was measured no slower than the narrow tile
     ((7168, 2048, 256, 8), 7), ((7168, 2048, 256, 4), 15), ((7168, 2048, 192, 8), 6), ((7168, 2048, 160, 8), 6), ((7168, 2048, 160, 6), 8),
     ((7168, 2048, 128, 8), 5), ((7168, 2048, 64, 8), 2), ((7168, 2048, 64, 4), 5), ((7168, 2048, 32, 4), 2), ((6144, 4096, 16, 2), 2),
-    ((6144, 4096, 32, 2), 5), ((4096, 14336, 8, 2), 1), ((5120, 1536, 160, 6), 9), ((4096, 1024, 128, 8), 5), ((2048, 1536, 64, 6), 3)])
+    ((6144, 4096, 32, 2), 5), ((6144, 2560, 160, 6), 7), ((4096, 14336, 8, 2), 1), ((5120, 1536, 160, 6), 9), ((4096, 1024, 128, 8), 5), ((2048, 1536, 64, 6), 3)])
 def test_planar_layers_leave_the_decode_launch_where_it_is_slower(shape, decode_max):
     t = _thresholds(*shape, capi.FMT_MXFP4_PLANAR, capi.FMT_MXFP4_PLANAR)
     assert t["decode_max"] == decode_max and t["gemm"] * 11 // 16 <= decode_max + 1 and t["narrow"] == 14
@@ -273,10 +273,11 @@ def test_streaming_begins_where_it_is_faster(shape, slower, faster):
 
 # (hidden, inter, experts, top): first token count with a shared expert alike, without one, with a Q8_0 one
 FIRST_STREAMING = {
-    (7168, 2048, 256, 8): (4, 6, 7), (7168, 2048, 256, 6): (6, 8, 10), (7168, 2048, 256, 4): (8, 12, 14), (7168, 2048, 256, 16): (3, 3, 7),
+    (7168, 2048, 256, 8): (4, 6, 7), (7168, 2048, 256, 6): (6, 8, 10), (7168, 2048, 256, 4): (7, 12, 14), (7168, 2048, 256, 16): (3, 3, 7),
     (4096, 2048, 128, 8): (4, 4, 7), (4096, 2048, 64, 4): (7, 7, 7), (4096, 1024, 128, 8): (6, 7, 9), (5120, 1536, 160, 6): (8, 9, 9),
-    (3072, 1024, 128, 8): (8, 8, 9), (2048, 1536, 64, 6): (10, 10, 10), (2048, 768, 128, 8): (14, 14, 14), (1024, 512, 128, 8): (36, 36, 36),
-    (1024, 1024, 64, 6): (24, 24, 24)}
+    (3072, 1024, 128, 8): (8, 8, 9), (2048, 1536, 64, 6): (8, 8, 9), (2048, 768, 128, 8): (14, 14, 14), (1024, 512, 128, 8): (36, 36, 36),
+    (1024, 1024, 64, 6): (24, 24, 24), (7168, 2048, 64, 8): (4, 4, 7), (7168, 2048, 32, 4): (7, 7, 9), (6144, 4096, 16, 4): (7, 7, 9),
+    (2048, 1792, 64, 6): (8, 8, 9), (3072, 1024, 32, 4): (12, 12, 12), (3072, 1024, 64, 6): (8, 8, 9)}
 
 
 def first_streaming(shape, **sh):

@@ -256,12 +256,12 @@ def test_a_stack_of_streaming_blocks(monkeypatch, fmt, T):
     assert np.array_equal(final, eager.cpu().numpy())
 
 
-@pytest.mark.parametrize("hidden,inter,E,k,T", [(4096, 2048, 16, 8, 4), (4096, 2048, 16, 8, 8), (7168, 2048, 64, 8, 4), (2048, 1536, 32, 6, 10),
-                                                (1536, 1536, 64, 6, 19), (2048, 1536, 32, 6, 9), (4096, 2048, 16, 8, 3), (4096, 2048, 64, 8, 3)])
+@pytest.mark.parametrize("hidden,inter,E,k,T", [(4096, 2048, 16, 8, 4), (4096, 2048, 16, 8, 8), (7168, 2048, 64, 8, 4), (2048, 1536, 32, 6, 9),
+                                                (1536, 1536, 64, 6, 19), (2048, 1536, 32, 6, 7), (4096, 2048, 16, 8, 3), (4096, 2048, 64, 8, 3)])
 @pytest.mark.parametrize("shared", ["none", "same", "q8_0"])
 def test_few_tokens_stream_in_the_decode_launch_s_place(monkeypatch, hidden, inter, E, k, T, shared):
-    """From 28, 60 or 112 picks on by size of a matrix (the last two shapes: one token short of it; the largest without a shared expert:
-    48; a Q8_0 shared expert: from 7 tokens); a decode limit set by the caller brings the one-launch form back, the same sums in another order, whose bits the
+    """Half a pick per expert and more: from 28, 48 or 112 picks on by size of a matrix (the last three shapes are short of it; a Q8_0
+    shared expert: from 7 tokens); a decode limit set by the caller brings the one-launch form back, the same sums in another order, whose bits the
     token counts short of both ranges have (three tokens on 64 experts)."""
     monkeypatch.setattr(MoeLayer, "v3_thresholds_below_experts", None)
     fmts = dict(sh_gate_fmt=FMT_Q8_0, sh_down_fmt=FMT_Q8_0) if shared == "q8_0" else {}
@@ -269,8 +269,7 @@ def test_few_tokens_stream_in_the_decode_launch_s_place(monkeypatch, hidden, int
     dw = H.device_weights(s)
     layer, launch = MoeLayer(dw, T), MoeLayer(dw, T)
     launch.set_tuning(decode_max_tokens=16)
-    streams = T * k >= (48 if (hidden, shared) == (7168, "none") else 28 if hidden * inter >= 8 << 20 else 60 if hidden * inter >= 3 << 20 else 112) and (
-        shared != "q8_0" or T >= 7)
+    streams = T * k >= (28 if hidden * inter >= 8 << 20 else 48 if hidden * inter >= 3 << 20 else 112) and (shared != "q8_0" or T >= 7)
     assert (T >= layer.streaming()[0]) == streams
     x, _, _ = H.host_inputs(s, T)
     rng = np.random.default_rng(T)
