@@ -26,13 +26,14 @@
 // (but the ends of a unit), so the loads of a group that is one item are non-temporal: whole layers, us with ordinary loads /
 // with these: 7168 x 2048, 256 experts, top-8: 16 tokens 478 / 421, 100: 1096 / 963; 4096 x 1024, 128 experts, 37 tokens 182 /
 // 158; all-Q8_0 2048 x 1408: 4 tokens 65.6 / 59.2, 40: 149 / 131.  The items of one group find each other's lines in the L2
-// (non-temporal throughout / there not: 7168 x 2048, every token on the same picks: 100 tokens 272 / 254, 40: 142 / 139;
-// Zipf-skewed 200: 1132 / 1120; gate/up beside a Q8_0 down matrix, same picks, 60: 214 / 204; two items, 24: 104.7 / 105.7).  The
+// (non-temporal throughout / there not: 7168 x 2048, every token on the same picks: 100 tokens 272 / 234, 40: 143 / 132; gate/up beside
+// a Q8_0 down matrix, same picks, 60: 215 / 200).  The kind of load is chosen once per stage: a branch beside every load delays
+// the stage's requests (same picks, 100: 254, 40: 138; 2560 x 2048, 96 experts, 95 tokens 216 / 205; 2048 x 1536, 64, 24: 84.0 / 79.5).  The
 // workgroups of one launch end within 5 % of each other at 64 tokens and 10 % at 16.  Measured and not
 // taken: the last tenth of the work claimed in chunks through a counter (64 tokens 4 % faster, 200 tokens 2
 // to 5 % slower: every chunk loads an item's columns again); a stage read into registers and its place
 // requested before the products (16 columns: no change; 32: the registers spill).  Scalar registers run out in
-// the instances for long rows (16 / 32 columns: 43 / 65 of them live in lanes of a vector register in gate/up, 27 / 51 in
+// the instances for long rows (16 / 32 columns: 44 / 68 of them live in lanes of a vector register in gate/up, 29 / 54 in
 // down; no memory); what that costs was not measured.
 //
 // A shared expert of another format runs beside these on the layer's side stream although they take nearly all
@@ -256,8 +257,7 @@ __device__ __forceinline__ void stream_body(const StreamParams &p) {
     constexpr int kW = COLS::kWaves;
     // Between two stages a wave requests the next one or adds up and stores the last one's sums.  MXFP4: the first half of
     // the waves does the one, the second half the other, at the same time and without a load that waits behind a store
-    // (vmcnt counts them in order; 7168 x 2048, 256 experts, every wave both / so: 100 tokens 977 / 961 us, Zipf-skewed 200: 1146 / 1117, but
-    // with every token on the same picks, whose lines come from the L2 faster than half of the waves ask for them, 100: 240 / 254); Q8_0: every wave does its part of both (half each: 2048 x 1408, 40 tokens 124 / 126 us).
+    // (vmcnt counts them in order; 7168 x 2048, 256 experts, every wave both / so: 100 tokens 977 / 961 us, Zipf-skewed 200: 1146 / 1117); Q8_0: every wave does its part of both (half each: 2048 x 1408, 40 tokens 124 / 126 us).
     constexpr uint32_t kLoaders = COLS::kRoles ? (uint32_t)kW / 2u : (uint32_t)kW;
     constexpr uint32_t kSummer0 = COLS::kRoles ? kLoaders : 0u;               // the first wave that sums
     constexpr uint32_t kSummers = ((uint32_t)kW - kSummer0) * 64u;            // threads that do
@@ -314,15 +314,19 @@ __device__ __forceinline__ void stream_body(const StreamParams &p) {
         const uint8_t *src1 = PAIR && !kTurns ? q_base[1] + (uint64_t)q_ut * unit_bytes : nullptr;
         const uint32_t dst = lds0 + q_slot * p.stage_bytes;
         // (the offsets are the same for every stage, but there are no registers to keep them in)
-        for (uint32_t L = wave; L < n_loads; L += kLoaders) {
-            const bool second = PAIR && !kTurns && L >= p.loads;
-            const uint32_t s = (second ? L - p.loads : L) * 64u + lane;
-            const uint32_t run = __umulhi(s, p.pitch_magic);   // s / pitch
-            uint32_t piece = s - run * p.pitch;
-            piece = min(piece, p.run - 1u);   // a row's padding repeats its last piece
-            // (slots past the last row fetch the unit's last piece: the load stays in the unit)
-            lds_dma16_if_nt(dst + L * 1024u, second ? src1 : src0, min(run * p.run + piece, last_piece) * 16u, q_once);
-        }
+        auto loads = [&](auto nt) __attribute__((always_inline)) {
+            for (uint32_t L = wave; L < n_loads; L += kLoaders) {
+                const bool second = PAIR && !kTurns && L >= p.loads;
+                const uint32_t s = (second ? L - p.loads : L) * 64u + lane;
+                const uint32_t run = __umulhi(s, p.pitch_magic);   // s / pitch
+                uint32_t piece = s - run * p.pitch;
+                piece = min(piece, p.run - 1u);   // a row's padding repeats its last piece
+                // (slots past the last row fetch the unit's last piece: the load stays in the unit)
+                lds_dma16<decltype(nt)::value>(dst + L * 1024u, second ? src1 : src0, min(run * p.run + piece, last_piece) * 16u);
+            }
+        };
+        if (q_once) loads(std::true_type{});   // uniform
+        else loads(std::false_type{});
         q_left--;
         q_slot = q_slot + 1u == p.depth ? 0u : q_slot + 1u;
         if (kTurns) {
