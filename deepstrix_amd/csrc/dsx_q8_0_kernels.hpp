@@ -577,7 +577,10 @@ struct Q8GemmLds {
 };
 
 // 64 rows (tile rt) of the work item of `cnt` members of expert e, the first of them members[mbase].
-template <bool PAIR, int COLS>
+// NT: the weight loads are non-temporal.  (Told once per item: a branch beside every load delays a chunk's requests; us per layer,
+// branch / so: 2048 x 1408, 64 experts, top-6, 100 tokens 145 / 138; every token on the same picks: 4096 x 1024, 16, top-4, 78: 66 / 62, 3072
+// x 512, 96, top-4, 617: 118 / 114, 6144 x 4096, 16, top-6, 154: 421 / 414.)
+template <bool PAIR, int COLS, bool NT>
 __device__ __forceinline__ void q8_0_gemm_tile(const Q8GemmParams &p, const uint32_t e, const uint32_t cnt, const uint32_t mbase, const uint32_t rt) {
     constexpr uint32_t M = PAIR ? 2u : 1u;
     using L = Q8GemmLds<PAIR, COLS>;
@@ -646,7 +649,6 @@ __device__ __forceinline__ void q8_0_gemm_tile(const Q8GemmParams &p, const uint
     __syncthreads();  // s_col has been read
     const bool b_live = wave_u * (uint32_t)kBLoads * 8u < cnt;
     const uint32_t xs_all = (cnt + kXsCols - 1u) / kXsCols, xs_live = xs_all > wave_u ? (xs_all - wave_u + kQgWaves - 1u) / kQgWaves : 0u;
-    const bool nt = p.whole_lines && !extra && (uint32_t)p.group_count[e] <= p.chunk;   // uniform
     auto issue = [&](uint32_t c, uint32_t buf) {
 #pragma unroll
         for (uint32_t mm = 0; mm < M; mm++)
@@ -654,8 +656,7 @@ __device__ __forceinline__ void q8_0_gemm_tile(const Q8GemmParams &p, const uint
             for (int i = 0; i < 2; i++) {
                 const uint32_t dst = a_lds + (mm * DEPTH + buf) * 2048u + (uint32_t)i * 1024u;
                 const uint32_t src = a_fetch + (uint32_t)i * 8u * row_bytes + c * 128u;
-                if (nt) lds_dma16<true>(dst, wbase[mm], src);
-                else lds_dma16(dst, wbase[mm], src);
+                lds_dma16<NT>(dst, wbase[mm], src);
             }
         if (b_live) {
 #pragma unroll
@@ -836,14 +837,17 @@ __global__ __launch_bounds__(kQgWaves * 64, (Q8GemmLds<PAIR, COLS>::kPerCu)) voi
     const uint32_t e = wi >> 16, start = wi & 0xFFFFu;
     const uint32_t cnt = min(p.chunk, (uint32_t)p.group_count[e] - start);
     const uint32_t mbase = (uint32_t)p.group_offset[e] + start;
+    const bool nt = p.whole_lines && e < p.n_expert && (uint32_t)p.group_count[e] <= p.chunk;   // uniform
     if constexpr (q8_gemm_both<PAIR, COLS>) {
         static_assert(Q8GemmLds<PAIR, COLS>::kPerCu == Q8GemmLds<PAIR, kQgColsNarrow>::kPerCu, "as many workgroups of a CU for either tile");
         if (cnt <= kQgColsNarrow) {   // uniform
-            q8_0_gemm_tile<PAIR, kQgColsNarrow>(p, e, cnt, mbase, rt);
+            if (nt) q8_0_gemm_tile<PAIR, kQgColsNarrow, true>(p, e, cnt, mbase, rt);
+            else q8_0_gemm_tile<PAIR, kQgColsNarrow, false>(p, e, cnt, mbase, rt);
             return;
         }
     }
-    q8_0_gemm_tile<PAIR, COLS>(p, e, cnt, mbase, rt);
+    if (nt) q8_0_gemm_tile<PAIR, COLS, true>(p, e, cnt, mbase, rt);
+    else q8_0_gemm_tile<PAIR, COLS, false>(p, e, cnt, mbase, rt);
 }
 
 // Raised once per device by the library's set-up, with the device current.
