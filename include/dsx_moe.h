@@ -371,7 +371,7 @@ int dsx_moe_layer_get_tuning(const dsx_moe_layer *layer, uint32_t out[6]);
 /* The token counts that take the streaming kernels: out[0] the first, out[1] the last, both 0 where there are
  * none (planar weights, Q8_0 gate/up with an MXFP4 down matrix, weights that are not 8-byte aligned, rows of more
  * than 7168 values -- Q8_0: 4096 -- values set by the caller as above).  By default, all-MXFP4: from 28 to 112 picks in all on, by the
- * size of a matrix and the shared expert [4 tokens; 6 without a shared expert, 7 beside one of another format] -- matrices under
+ * size of a matrix, the shared expert and half a pick per expert [4 tokens; 6 without a shared expert, 7 beside one of another format] -- matrices under
  * 1.5 M elements not --, from 9 tokens or where the decode path ends in any case -- matrices under 4 M elements: from 2.25 or 3.5 picks per
  * expert -- to below 18 picks per expert, 28 where a matrix has up to 4 M elements [4 .. 575]; beside a Q8_0 down
  * matrix the range of gate/up, from 2 tokens (matrices under 4 M elements: 1.25 picks per expert) to below 28 picks per expert
