@@ -543,6 +543,10 @@ struct Q8GemmParams {
     uint32_t chunk;                // members of a work item, up to the tile's columns
     uint32_t whole_lines;          // every 128-byte piece of a routed row's quants is one cache line
     StreamChoice choice;           // a streaming launch offers the same product
+    // gate/up's middle tile (q8_takes_wide_items): a list of items of kQgCols members beside the one of kQgColsMiddle, or null; how many
+    // workgroups are resident at a time
+    const int32_t *wide_items, *n_wide_items;
+    uint32_t slots;
     float clamp, sh_clamp;
 };
 
@@ -808,9 +812,14 @@ __device__ __forceinline__ void q8_0_gemm_tile(const Q8GemmParams &p, const uint
 // gate/up, 7168 x 2048, 256 experts, uniform picks, us, 64 columns / both: 512 tokens 1621 / 1600, 700: 1734 / 1706, 1000: 2134 / 2082).
 template <bool PAIR, int COLS>
 constexpr bool q8_gemm_both = !PAIR && COLS == kQgColsMiddle;
+// Gate/up's takes the wide tile, on a list of its own, where the picks make that the faster one (q8_takes_wide_items).
+template <bool PAIR, int COLS>
+constexpr bool q8_gemm_widths = PAIR && COLS == kQgColsMiddle;
 template <bool PAIR, int COLS>
 constexpr uint32_t q8_gemm_lds_bytes() {
-    return q8_gemm_both<PAIR, COLS> ? std::max(Q8GemmLds<PAIR, COLS>::kBytes, Q8GemmLds<PAIR, kQgColsNarrow>::kBytes) : Q8GemmLds<PAIR, COLS>::kBytes;
+    return q8_gemm_both<PAIR, COLS>     ? std::max(Q8GemmLds<PAIR, COLS>::kBytes, Q8GemmLds<PAIR, kQgColsNarrow>::kBytes)
+           : q8_gemm_widths<PAIR, COLS> ? std::max(Q8GemmLds<PAIR, COLS>::kBytes, Q8GemmLds<PAIR, kQgCols>::kBytes)
+                                        : Q8GemmLds<PAIR, COLS>::kBytes;
 }
 
 template <bool PAIR, int COLS>
@@ -820,7 +829,20 @@ __global__ __launch_bounds__(kQgWaves * 64, (Q8GemmLds<PAIR, COLS>::kPerCu)) voi
     // the row tiles of a work item run on one XCD (they share the activations in its L2); the
     // items are dealt to the XCDs like cards, which spreads the wide groups of skewed routing
     const uint32_t xcd = blockIdx.x & 7u, seq = blockIdx.x >> 3;
-    const uint32_t n_items = (uint32_t)*p.n_work_items;  // the grid is only an upper bound
+    const int32_t *items = p.work_items;
+    uint32_t n_items = (uint32_t)*p.n_work_items, chunk = p.chunk;  // the grid is only an upper bound
+    bool wide = false;
+    if constexpr (q8_gemm_widths<PAIR, COLS>) {
+        if (p.wide_items) {   // uniform
+            const uint32_t n_wide = (uint32_t)*p.n_wide_items;
+            wide = q8_takes_wide_items(n_items, n_wide, p.n_row_tiles, p.slots);
+            if (wide) {
+                items = p.wide_items;
+                n_items = n_wide;
+                chunk = kQgCols;
+            }
+        }
+    }
     const uint32_t local = seq / p.n_row_tiles;
     // Many column tiles per expert (skewed routing, many tokens): the items are dealt to the XCDs
     // like cards, which spreads the wide groups -- contiguous ranges of the list (it is by expert)
@@ -833,11 +855,18 @@ __global__ __launch_bounds__(kQgWaves * 64, (Q8GemmLds<PAIR, COLS>::kPerCu)) voi
     const uint32_t rt = seq % p.n_row_tiles;
     if (item >= n_items) return;
 
-    const uint32_t wi = (uint32_t)p.work_items[item];
+    const uint32_t wi = (uint32_t)items[item];
     const uint32_t e = wi >> 16, start = wi & 0xFFFFu;
-    const uint32_t cnt = min(p.chunk, (uint32_t)p.group_count[e] - start);
+    const uint32_t cnt = min(chunk, (uint32_t)p.group_count[e] - start);
     const uint32_t mbase = (uint32_t)p.group_offset[e] + start;
-    const bool nt = p.whole_lines && e < p.n_expert && (uint32_t)p.group_count[e] <= p.chunk;   // uniform
+    const bool nt = p.whole_lines && e < p.n_expert && (uint32_t)p.group_count[e] <= chunk;   // uniform
+    if constexpr (q8_gemm_widths<PAIR, COLS>) {
+        static_assert(Q8GemmLds<PAIR, COLS>::kPerCu == Q8GemmLds<PAIR, kQgCols>::kPerCu, "as many workgroups of a CU for either tile");
+        if (wide) {
+            q8_0_gemm_tile<PAIR, kQgCols, false>(p, e, cnt, mbase, rt);
+            return;
+        }
+    }
     if constexpr (q8_gemm_both<PAIR, COLS>) {
         static_assert(Q8GemmLds<PAIR, COLS>::kPerCu == Q8GemmLds<PAIR, kQgColsNarrow>::kPerCu, "as many workgroups of a CU for either tile");
         if (cnt <= kQgColsNarrow) {   // uniform

@@ -85,6 +85,19 @@ inline uint32_t q8_gate_up_columns(const Q8Shape &s, uint32_t T, uint32_t down) 
     return down == kQgColsNarrow ? down : s.picks_below_halves(T, 120u) ? kQgColsMiddle : kQgCols;
 }
 
+// Whether gate/up's launch in 64 columns takes the list of 128-column items after all (on the device, by the items that the picks make):
+// where few experts are hot, 64 columns cut their groups into up to twice as many items.  A round of resident workgroups takes about three
+// fifths as long with 64 columns (three rounds beat two of 128, seven lose to four).  us per layer, 128 / 64 columns (items,
+// rounds): 4096 x 1536, 128 experts, top-8, 900 tokens on 32 experts (72, 4 / 143, 7) 650 / 688; 3072 x 2048, 64, top-4, 900 tokens on the
+// same picks (40, 3 / 75, 5) 364 / 377; 7168 x 2048, 256, top-8, 1000 on 64 experts 1766 / 1828; but 4096 x 1536, 300, same (27, 2 /
+// 45, 3) 293 / 256; 2048 x 1408, 64, top-6, 512, same (28, 2 / 56, 3) 163, with older scale loads, / 151.  The number of items is asked
+// as well because a few items more can make a round, which is not a full one.  Spread picks keep their 64 columns, Zipf-skewed ones were as
+// fast (4096 x 1536, 900 tokens 866 / 870; 2048 x 1408, 512: 220 / 220).  The choice costs passes that keep 64 columns up to 1 % (253 / 255).
+constexpr bool q8_takes_wide_items(uint32_t middle, uint32_t wide, uint32_t row_tiles, uint32_t slots) {
+    const uint32_t rounds_middle = (middle * row_tiles + slots - 1u) / slots, rounds_wide = (wide * row_tiles + slots - 1u) / slots;
+    return 5u * middle >= 7u * wide && 5u * rounds_wide <= 3u * rounds_middle;
+}
+
 // Columns per work item of a dense Q8_0 expert of b tokens (dsx_dense_ffn; both products, one list): 32 where the wide
 // tile would leave workgroup slots empty in gate/up (two per CU) -- over 128 tokens unless the items, each of which
 // reads gate and up whole, come to about a gigabyte of reads, in brackets (us, wide / narrow: 7168 x 2048: 96 tokens

@@ -212,6 +212,34 @@ def test_middle_tile_on_many_workgroups(monkeypatch):
     assert torch.equal(out, older.run(dx, dl)) and torch.isfinite(out).all()
 
 
+@pytest.mark.parametrize("named,wide", [(8, True), (16, True), (64, False)])
+@pytest.mark.parametrize("hidden", [640, 1152])
+def test_gate_up_items_of_128_on_few_hot_experts(monkeypatch, hidden, named, wide):
+    """31 picks per expert: the middle tile's launch, which takes the list of 128-column items where 250 tokens name eight or sixteen of
+    64 experts (16 row tiles: two rounds of 64-column items, one of 128-column ones); groups of every remainder; the wide tile's bits."""
+    monkeypatch.setattr(MoeLayer, "v3_thresholds_below_experts", None)
+    T, s = 250, H.Shape(hidden, 1024, 64, 8, FMT_Q8_0, FMT_Q8_0, seed=848, **ROUTER)
+    rng = np.random.default_rng(named)
+    sel = np.stack([rng.permutation(named)[:8] for _ in range(T)]).astype(np.int32)
+    sel[T // 2, 1] = -1
+    n = np.append(np.bincount(sel[sel >= 0], minlength=64), T)
+    middle, big = (int((-(-n // c)).sum()) for c in (64, 128))
+    slots = 2 * torch.cuda.get_device_properties(0).multi_processor_count
+    assert (5 * middle >= 7 * big and 5 * -(-big * 16 // slots) <= 3 * -(-middle * 16 // slots)) == wide
+    w = rng.uniform(0.05, 0.6, sel.shape).astype(np.float32)
+    x, dw = H.host_inputs(s, T)[0], H.device_weights(s)
+    layer, older = MoeLayer(dw, T), MoeLayer(dw, T)
+    older.set_tuning(by_expert_chunk=4)             # the wide tile alone
+    args = dict(selected_in=torch.from_numpy(sel).cuda(), weights_in=torch.from_numpy(w).cuda())
+    dx = torch.from_numpy(x).cuda()
+    out = layer.run(dx, None, **args).clone()
+    old = older.run(dx, None, **args)
+    torch.cuda.synchronize()
+    assert layer.status() == 0 and torch.equal(out, old)
+    hw = H.host_weights(s)
+    H.assert_parity_up_to_rounding_steps(out.cpu().numpy(), ref.moe_forward(hw, x, sel, w), hw, sel, f"{hidden} {named}")
+
+
 def test_rows_longer_than_the_registers_take_the_older_paths(monkeypatch):
     """Gate/up rows of 33 groups: the older paths' bits."""
     s = H.Shape(4224, 256, 8, 2, FMT_Q8_0, FMT_Q8_0, shared=False, seed=850, **ROUTER)

@@ -42,6 +42,15 @@ def test_gate_up_columns_of_the_int8_gemm(shape, columns):
     assert dict(zip(columns, ask([("gate_up", *shape, T, CUS) for T in columns]))) == columns
 
 
+@pytest.mark.parametrize("middle,wide,row_tiles,takes", [
+    (143, 72, 24, 1), (75, 40, 32, 1), (72, 36, 12, 1),   # 900 tokens on 32 of 128 experts; all on the same picks
+    (56, 28, 22, 0), (45, 27, 24, 0),                     # the wide items make as many or two thirds of the rounds
+    (144, 130, 24, 0), (90, 66, 22, 0),                   # spread, skewed picks
+    (7, 5, 128, 0), (14, 10, 256, 0)])
+def test_wide_items_of_gate_up(middle, wide, row_tiles, takes):
+    assert ask([("wide", middle, wide, row_tiles, 2 * CUS, 0, 0)]) == [takes]
+
+
 @pytest.mark.parametrize("shape,columns", [
     ((7168, 2048), {96: 32, 768: 32, 1000: 128, 1900: 128, 2000: 128}),
     ((7168, 3072), {512: 32, 640: 32, 1000: 128}),
